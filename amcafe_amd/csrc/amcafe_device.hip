@@ -43,64 +43,6 @@
 #include "ddmath.h"
 #include "gl25.h"
 
-// Phase timers of the capture loop (core-clock cycles summed over events), compiled in
-// only with -DAMCD_PHASE_PROFILE; read with amcd_phase_profile().
-#ifdef AMCD_PHASE_PROFILE
-__device__ unsigned long long g_phase[32];
-#define PHASE_INIT(v) unsigned long long v = clock64()
-#define PHASE(v, slot, pred)                                \
-  do {                                                      \
-    unsigned long long t_ = clock64();                      \
-    if (pred) atomicAdd(&g_phase[slot], t_ - v);            \
-    v = t_;                                                 \
-  } while (0)
-// barrier arrival of wave w (lane 0) with a flag word of what the wave did this event
-#define PHASE_ARRIVE(sh, par, w, flag)         \
-  do {                                         \
-    int wf_ = 0;                               \
-    for (int b_ = 0; b_ < 6; ++b_)             \
-      if (__ballot(((flag) >> b_) & 1)) wf_ |= 1 << b_; \
-    if ((threadIdx.x & 63) == 0) {             \
-      (sh).arr[par][w] = clock64();            \
-      (sh).aflag[par][w] = wf_;                \
-    }                                          \
-  } while (0)
-// after the barrier: which wave arrived last, by how much, and what it had done
-#define PHASE_LAST(sh, par, NW)                                              \
-  do {                                                                       \
-    if (threadIdx.x == 0) {                                                  \
-      int wl = 0;                                                            \
-      unsigned long long mx = 0, mn = ~0ull, m2 = 0;                         \
-      for (int q = 0; q < (NW); ++q) {                                       \
-        const unsigned long long a = (sh).arr[par][q];                       \
-        if (a > mx) { m2 = mx; mx = a; wl = q; } else if (a > m2) m2 = a;    \
-        if (a < mn) mn = a;                                                  \
-      }                                                                      \
-      atomicAdd(&g_phase[16 + wl], 1ull);                                    \
-      atomicAdd(&g_phase[24], mx - mn);                                      \
-      atomicAdd(&g_phase[25], mx - m2);                                      \
-      const int fl = (sh).aflag[par][wl];                                    \
-      for (int b = 0; b < 6; ++b)                                            \
-        if ((fl >> b) & 1) atomicAdd(&g_phase[26 + b], 1ull);                \
-    }                                                                        \
-  } while (0)
-#else
-#define PHASE_INIT(v)
-#define PHASE(v, slot, pred)
-#define PHASE_ARRIVE(sh, par, w, flag)
-#define PHASE_LAST(sh, par, NW)
-#endif
-// a per-lane word of what a wave did in the event, for the arrival record (profile builds only)
-#ifdef AMCD_PHASE_PROFILE
-#define PHASE_FLAGS(v) int v = 0
-#define PHASE_FLAG(v, bits) (v) |= (bits)
-#define PHASE_FLAGS_CLEAR(v) (v) = 0
-#else
-#define PHASE_FLAGS(v)
-#define PHASE_FLAG(v, bits)
-#define PHASE_FLAGS_CLEAR(v)
-#endif
-
 // A pointer known to address global memory.  The capture loop reads its array pointers
 // from a descriptor copied to LDS, so the compiler cannot tell their address space and
 // would emit flat accesses, which also count against the LDS wait counter: every LDS
@@ -151,6 +93,7 @@ struct LoopState {
   int pending;       // 1: a nucleation was decided but the pool was empty
   int pend_tgt;      // active index of the voxel to nucleate
   int Na, nmushy0;
+  int npre;          // entries of the lists built ahead
   int zhot0, zhot1;  // z planes the last temperature evaluation could have melted
   // T holds the analytic field of a laser plane at lz_prev (tvalid = 1): every voxel is xi
   // where its hot flag (vs bit 7) is set, else T0 above lz_prev and tS below it
@@ -158,6 +101,40 @@ struct LoopState {
   double lz_prev;
 };
 
+// One entry of a growing cell's candidate list: everything the capture loop reads of it in one
+// 32-byte record (four to a cache line; as an array per field, an entry cost five lines).
+struct alignas(16) CandRec {
+  double D, r;  // capture distance, ruqs
+  int tgt;      // target (active index)
+  int nb;       // neighbour rank
+  float tn;     // lower bound on the time from a capture through this entry to the first capture
+                // by the cell it creates (-inf: unknown)
+  int n;        // entries from this one to the list's end
+};
+// What the capture loop reads of an active cell whose voxel is captured, in one cache line.
+struct alignas(128) CellRow {
+  int nbr[AMCD_NB];  // active indices of the Moore neighbours (-1: outside or not active)
+  int vox, cold;     // voxel; all active neighbours below tL (S/VoxelsCA.C:396-397)
+  double T;
+  int pad[2];
+};
+// What a capture through an entry of a list the set-up built does: the re-centred octahedron, the
+// grain, the new cell's velocity and its list built ahead (-1: none).
+struct alignas(16) CapRec {
+  double x, y, z, E;
+  int pre, G;
+  double V;
+};
+// A growing cell's constants; n: entries of its list (-1: the cell carries no valid grain).
+struct alignas(16) SlotRec {
+  double c[3];
+  int vox, G, act, scan, base, n;
+};
+// A performed event, for the active arrays at the loop's end.
+struct alignas(16) EventRec {
+  int i1, G;
+  double E, x, y, z, pad;
+};
 struct Inst {
   amcd_params p;
   int N, nxy, nblkZ, nblkG, nblkS, nblkT;
@@ -179,24 +156,20 @@ struct Inst {
   uint8_t* aVS;
   int* aG;
   double *aT, *aExt, *aCx, *aCy, *aCz, *ruq;
-  int* aNbr;
-  double* aRN;     // ruqs .5*(ruq[a] + ruq[aNbr[a][q]]) of every active cell a and neighbour q
-  uint8_t* aCold;
+  CellRow* aRow;
+  EventRec* events;
   int* aScan;
   // growing list + candidates (26 slots per growing cell)
-  int *gAct, *gScan;
+  SlotRec* slots;
   double *gExt, *gVhat;
-  double *gR, *gC;  // per slot: the cell's grain rotation (9) and centroid (3)
-  int *gV, *gG;     // per slot: the cell's voxel and grain
   float2* gLH;      // per slot: capture-clock bounds (lo, hi) of the memory-resident tier
   int2* gHd;        // per slot: list head (entry, target) of the memory-resident tier
-  uint8_t *gN, *gDead, *gGrow;
-  unsigned* gdead;  // liveness bitmap of the capture loop in memory (one bit per active cell),
-                    // for interfaces larger than the LDS bitmap holds
-  double *cD, *cF, *cR;
-  double4* cRC;     // per entry of a set-up list: the capture's re-centred centroid and extent
-  int *cTgt, *cV;   // per entry: target (active index) and its voxel
-  uint8_t* cK;
+  // Lists: slot s's at 26 s when the set-up or the loop built it; from 26 acap on, the lists that
+  // the set-up built ahead for the cells that captures would create.
+  CandRec* cand;
+  double* cF;       // per entry: shape factor
+  CapRec* cap;      // per entry (of the lists that the set-up built)
+  int precap;       // entries that the lists built ahead may take
   // grains
   int gcap;
   double* rot;
@@ -251,7 +224,8 @@ __device__ static inline int find_inst(const int* start, int n, int b) {
   }
   return lo;
 }
-__device__ static inline void decode(const Inst& d, int v, int& i, int& j, int& k) {
+template <class DI>
+__device__ static inline void decode(DI& d, int v, int& i, int& j, int& k) {
   k = v / d.nxy;
   int r = v - k * d.nxy;
   j = r / d.p.nx;
@@ -890,6 +864,7 @@ __global__ __launch_bounds__(1024) void k_scan(Inst* I, const amcd_step* S, amcd
     ls->nmushy0 = Nm;
     ls->nslots = 0;
     ls->nslots_pre = -1;
+    ls->npre = 0;
     ls->vSind2 = Nm;
     ls->tinc = 0.0;
     ls->events = ls->captures = ls->nucs = 0;
@@ -998,7 +973,8 @@ __global__ __launch_bounds__(256) void k_compact(Inst* I, const int* bstart, int
 }
 
 // Voxel centre, S/VoxelsCA.C:409-414.
-__device__ static inline void centre(const Inst& d, int v, double* c) {
+template <class DI>
+__device__ static inline void centre(DI& d, int v, double* c) {
   int i, j, k;
   decode(d, v, i, j, k);
   c[0] = ((double)i + .5) * d.p.dx;
@@ -1032,7 +1008,8 @@ __device__ static inline void candidate(const Inst& d, const double* c, const do
 
 // vhat = Avel * pow(tL - T, nvel) (S/VoxelsCA.C:405), pow rounded to nearest; the two
 // temperatures of the analytic model are precomputed, any other (EASM) is evaluated here.
-__device__ static inline double growth_velocity(const amcd_params& p, double T) {
+template <class P>
+__device__ static inline double growth_velocity(P& p, double T) {
   if (T >= p.tL) return 0.0;
   if (T == p.tS) return p.vhat_tS;
   if (T == p.T0) return p.vhat_T0;
@@ -1056,25 +1033,31 @@ __global__ __launch_bounds__(GB) void k_active_setup(Inst* I, const int* bstart,
     int v = d.aVox[a];
     int i, j, k;
     decode(d, v, i, j, k);
-    int* nb = d.aNbr + (size_t)a * AMCD_NB;
+    CellRow row;
     int q = 0;
     bool cold = true, liq = false;
+#pragma unroll
     for (int dz = -1; dz <= 1; ++dz)
+#pragma unroll
       for (int dy = -1; dy <= 1; ++dy)
+#pragma unroll
         for (int dx = -1; dx <= 1; ++dx) {
           if (dx == 0 && dy == 0 && dz == 0) continue;
           int x = i + dx, y = j + dy, z = k + dz;
           int n = -1;
           if (x >= 0 && x < d.p.nx && y >= 0 && y < d.p.ny && z >= 0 && z < d.p.nz)
             n = d.amap[v + dz * d.nxy + dy * d.p.nx + dx];
-          d.aRN[(size_t)a * AMCD_NB + q] = n >= 0 ? .5 * (d.ruq[a] + d.ruq[n]) : 0.0;
-          nb[q++] = n;
+          row.nbr[q++] = n;
           if (n >= 0) {
             if (!(d.aT[n] < d.p.tL)) cold = false;
             if (d.aVS[n] == 1) liq = true;
           }
         }
-    d.aCold[a] = cold;
+    row.vox = v;
+    row.cold = cold;
+    row.T = d.aT[a];
+    row.pad[0] = row.pad[1] = 0;
+    d.aRow[a] = row;
     grow = cold && liq && d.aVS[a] == 2;
   }
   unsigned long long bal = __ballot(grow);
@@ -1087,28 +1070,12 @@ __global__ __launch_bounds__(GB) void k_active_setup(Inst* I, const int* bstart,
   if (!grow) return;
   unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int slot = base + __popcll(bal & lt);
-  d.gAct[slot] = a;
-  d.gScan[slot] = d.aScan[a];
   d.gExt[slot] = d.aExt[a];
   d.gVhat[slot] = growth_velocity(d.p, d.aT[a]);
-  d.gDead[slot] = 0;
-  double c[3] = {d.aCx[a], d.aCy[a], d.aCz[a]};
   const int G = d.aG[a];
-  if (G < 1 || G > d.gcap) {  // a growing cell must carry a valid grain
-    atomicOr(&O[ii].err_state, 1);
-    d.gN[slot] = 0;
-    d.gDead[slot] = 1;
-    return;
-  }
-  const double* R = d.rot + 9 * (size_t)(G - 1);
-  double Rl[9];
-  for (int q = 0; q < 9; ++q) {
-    Rl[q] = R[q];
-    d.gR[9 * (size_t)slot + q] = R[q];
-  }
-  for (int q = 0; q < 3; ++q) d.gC[3 * (size_t)slot + q] = c[q];
-  d.gV[slot] = d.aVox[a];
-  d.gG[slot] = G;
+  const bool bad = G < 1 || G > d.gcap;  // a growing cell must carry a valid grain
+  if (bad) atomicOr(&O[ii].err_state, 1);
+  d.slots[slot] = {{d.aCx[a], d.aCy[a], d.aCz[a]}, d.aVox[a], G, a, d.aScan[a], slot * AMCD_NB, bad ? -1 : 0};
 }
 
 // Re-centring of the decentred octahedron after a capture, S/VoxelsCA.C:528-605 and
@@ -1131,9 +1098,10 @@ __device__ static inline void project_point_line(const double* A, const double* 
 __device__ static inline double dist3(const double* p, const double* q) {
   return sqrt((p[0] - q[0]) * (p[0] - q[0]) + (p[1] - q[1]) * (p[1] - q[1]) + (p[2] - q[2]) * (p[2] - q[2]));
 }
-__device__ static inline void recentre(const Inst& d, int vcap, int vnew, const double* cen, const double* R, double f,
+template <class DI>
+__device__ static inline void recentre(DI& d, int vcap, int vnew, const double* cen, const double* R, double f,
                                 double* ncen, double* next) {
-  const amcd_params& p = d.p;
+  auto& p = d.p;
   int jx0, jx1, jx2, jy0, jy1, jy2;
   decode(d, vnew, jx0, jx1, jx2);
   decode(d, vcap, jy0, jy1, jy2);
@@ -1202,49 +1170,197 @@ __device__ static inline void recentre(const Inst& d, int vcap, int vnew, const 
 }
 
 // Candidate lists of the growing cells (S/VoxelsCA.C:396-440): one wave per slot, lane q
-// evaluates neighbour q when it is liquid, and the entries are placed by rank in
-// (D, ruqs, scan key) order -- the order the capture loop reads the list in.
+// evaluates neighbour q when it is liquid, and the entries are placed by rank in (D, ruqs,
+// neighbour) order -- the order the capture loop reads the list in.
+//
+// What a capture through an entry does depends, but for the voxels captured before it, on the
+// entry alone: the re-centred octahedron, the new cell's velocity and its candidates.  They are
+// evaluated here for every entry, over the whole chip, instead of on the capture loop's one compute
+// unit: the re-centring by the entry's lane, the new cell's sorted list two entries at a time (a
+// half wave each), with the re-centring of its own entries and a single-precision bound on the time
+// to the captures after them.  About one list in forty of those built ahead is used.  Bound by the
+// latency of a wave's own chain, not by the chip (a few thousand waves): 64 us for 3.3 thousand
+// growing cells and 37 us for 300 (18 and 15 us with the cells' own lists alone); with the lists
+// ahead the loop's windows end later: 3291 -> 2863 cycles per event in the former deck.
+__device__ static inline int list_rank(double D, double r, bool on, int half) {
+  // position in (D, ruqs, neighbour) order among the entries of this lane's half wave (all of it
+  // for half < 0), NaN distances last
+  const int lane = threadIdx.x & 63, q = half < 0 ? lane : lane & 31;
+  const unsigned long long bal = __ballot(on);
+  const unsigned mine = half < 0 ? (unsigned)bal : (half ? (unsigned)(bal >> 32) : (unsigned)bal);
+  const unsigned any = half < 0 ? (unsigned)bal : (unsigned)bal | (unsigned)(bal >> 32);
+  int rank = 0;
+  for (unsigned b = any; b != 0; b &= b - 1) {
+    const int j = __builtin_ctz(b);
+    double Dj = lane_f64(D, j), rj = lane_f64(r, j);
+    if (half >= 0) {
+      const double Dh = lane_f64(D, j + 32), rh = lane_f64(r, j + 32);
+      Dj = half ? Dh : Dj;
+      rj = half ? rh : rj;
+    }
+    rank += ((mine >> j) & 1u) != 0 && j != q && cand_less(Dj, rj, j, D, r, q) ? 1 : 0;
+  }
+  return rank;
+}
+// Capture distance D for an offset (x, y, z), in single precision: the shape factor's cosine and
+// sine are ratios of the offsets; within 1e-5 of the exact one.
+__device__ static inline float distance_f32(float x, float y, float z, const float* R) {
+  const float rho = sqrtf(x * x + y * y), rr = sqrtf(rho * rho + z * z);
+  const float cs = rho > 0.0f ? fmaxf(fabsf(x), fabsf(y)) / rho : 1.0f;
+  const float sn = rr > 0.0f ? fmaxf(rho, fabsf(z)) / rr : 1.0f;
+  return sqrtf(cs * sn) * (fabsf(R[0] * x + R[3] * y + R[6] * z) + fabsf(R[1] * x + R[4] * y + R[7] * z) +
+                           fabsf(R[2] * x + R[5] * y + R[8] * z));
+}
+// Lower bound, in single precision, on the time to grow by `lead` at velocity V (-inf: none).
+__device__ static inline float time_bound(double lead, double V) {
+  if (!(lead > 0.0) || !(V >= 0.0)) return -__builtin_inff();
+  const double x = lead / V * (1.0 - 1e-6);  // (+inf for V = 0: it never captures)
+  const float f = (float)x;
+  return (double)f > x ? nextafterf(f, 0.0f) : f;
+}
+// Lower bound on the time from the capture of active cell t (voxel v; new centroid c, rotation R,
+// half-diagonal E0) to the first capture by the cell it becomes, over the neighbours that are
+// liquid before the loop.  -inf: no useful bound; +inf: the cell does not grow.
+__device__ static inline float first_capture_after(const Inst& d, int t, int v, const double* c, double E0,
+                                                   const float* Rf) {
+  if (!d.aRow[t].cold) return __builtin_inff();
+  const amcd_params& p = d.p;
+  const double T = d.aRow[t].T;
+  const double V = T == p.tS ? p.vhat_tS : (T == p.T0 ? p.vhat_T0 : p.Avel * pow(p.tL - T, p.nvel) * (1 + 1e-9));
+  if (!(V > 0.0) || !(E0 == E0)) return -__builtin_inff();
+  int i, j, k;
+  decode(d, v, i, j, k);
+  float Dm = __builtin_inff();
+  bool bad = false;
+  for (int dz = -1; dz <= 1; ++dz) {
+    const int z = k + dz;
+    if (z < 0 || z >= p.nz) continue;
+    for (int dy = -1; dy <= 1; ++dy) {
+      const int y = j + dy;
+      if (y < 0 || y >= p.ny) continue;
+      const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * p.nx;
+      const float fy = (float)(((double)y + .5) * p.dy - c[1]), fz = (float)(((double)z + .5) * p.dz - c[2]);
+#pragma unroll
+      for (int dx = -1; dx <= 1; ++dx) {
+        const int x = i + dx;
+        if (x < 0 || x >= p.nx || (dx == 0 && dy == 0 && dz == 0)) continue;
+        if ((row[x] & 3) != 1) continue;
+        const float D = distance_f32((float)(((double)x + .5) * p.dx - c[0]), fy, fz, Rf);
+        bad |= !(D == D);
+        Dm = fminf(Dm, D);
+      }
+    }
+  }
+  return bad ? -__builtin_inff() : time_bound((double)Dm * (1.0 - 1e-5) - E0, V);
+}
+
 __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
-  const int a = d.gAct[slot];
-  const int t = lane < AMCD_NB ? d.aNbr[(size_t)a * AMCD_NB + lane] : -1;
+  const amcd_params& p = d.p;
+  const SlotRec sr = d.slots[slot];
+  if (sr.n < 0) return;
+  const int a = sr.act;
+  const int t = lane < AMCD_NB ? d.aRow[a].nbr[lane] : -1;
   const bool liq = t >= 0 && d.aVS[t] == 1;
   double D = __builtin_inf(), f = 0.0, r = __builtin_inf();
-  int key = 0x7fffffff, tv = -1;
+  int tv = -1, cold = 0;
+  float tnew = __builtin_inff();
   double4 rc = make_double4(0.0, 0.0, 0.0, 0.0);
+  double V = 0.0, R[9];
+  float Rf[9];
+  for (int q = 0; q < 9; ++q) {
+    R[q] = d.rot[9 * (size_t)(sr.G - 1) + q];
+    Rf[q] = (float)R[q];
+  }
   if (liq) {
-    double c[3], R[9];
-    for (int q = 0; q < 3; ++q) c[q] = d.gC[3 * (size_t)slot + q];
-    for (int q = 0; q < 9; ++q) R[q] = d.gR[9 * (size_t)slot + q];
-    tv = d.aVox[t];
+    const double c[3] = {sr.c[0], sr.c[1], sr.c[2]};
+    tv = d.aRow[t].vox;
+    cold = d.aRow[t].cold;
+    const double T = d.aRow[t].T;
+    V = !(T < p.tL) ? 0.0 : T == p.tS ? p.vhat_tS : T == p.T0 ? p.vhat_T0 : growth_velocity(p, T);
     candidate(d, c, R, tv, &D, &f);
-    r = d.aRN[(size_t)a * AMCD_NB + lane];
-    key = d.gScan[slot] * 32 + lane;
-    // the re-centring a capture through this entry performs depends on the entry and its
-    // cell alone (voxels, centroid, rotation, shape factor): evaluated here, in parallel,
-    // instead of on the capture loop's serial path
+    r = .5 * (d.ruq[a] + d.ruq[t]);
     double nc[3], ne;
-    recentre(d, d.gV[slot], tv, c, R, f, nc, &ne);
+    recentre(d, sr.vox, tv, c, R, f, nc, &ne);
     rc = make_double4(nc[0], nc[1], nc[2], ne);
   }
   const unsigned long long bal = __ballot(liq);
-  int rank = 0;  // (lane j's entry read with readlane: j is a constant of the unrolled loop)
-#pragma unroll
-  for (int j = 0; j < AMCD_NB; ++j) {
-    const double Dj = lane_f64(D, j), rj = lane_f64(r, j);
-    const int kj = __builtin_amdgcn_readlane(key, j);
-    if (((bal >> j) & 1) && j != lane && cand_less(Dj, rj, kj, D, r, key)) rank++;
-  }
+  const int n = (int)__popcll(bal);
   const size_t cb = (size_t)slot * AMCD_NB;
-  if (liq) {
-    d.cD[cb + rank] = D;
-    d.cF[cb + rank] = f;
-    d.cR[cb + rank] = r;
-    d.cTgt[cb + rank] = t;
-    d.cV[cb + rank] = tv;
-    d.cK[cb + rank] = (uint8_t)lane;
-    d.cRC[cb + rank] = rc;
+  const int rank = list_rank(D, r, liq, -1);
+  int pre = -1;
+  // the lists ahead, for the entries whose target would grow
+  const int half = lane >> 5, q = lane & 31;
+  const int qq = q < 13 ? q : q + 1, ddx = qq % 3 - 1, ddy = (qq / 3) % 3 - 1, ddz = qq / 9 - 1;
+  for (unsigned todo = (unsigned)__ballot(liq && cold); todo != 0;) {
+    const int j0 = __builtin_ctz(todo);
+    todo &= todo - 1;
+    const bool two = todo != 0;
+    const int j1 = two ? __builtin_ctz(todo) : j0;
+    todo &= todo - 1;
+    const int tj = half ? __builtin_amdgcn_readlane(t, j1) : __builtin_amdgcn_readlane(t, j0);
+    const int vj = half ? __builtin_amdgcn_readlane(tv, j1) : __builtin_amdgcn_readlane(tv, j0);
+    double c[3], E0;
+    c[0] = half ? lane_f64(rc.x, j1) : lane_f64(rc.x, j0);
+    c[1] = half ? lane_f64(rc.y, j1) : lane_f64(rc.y, j0);
+    c[2] = half ? lane_f64(rc.z, j1) : lane_f64(rc.z, j0);
+    E0 = half ? lane_f64(rc.w, j1) : lane_f64(rc.w, j0);
+    const double Vj = half ? lane_f64(V, j1) : lane_f64(V, j0);
+    const int t2 = q < AMCD_NB && (two || !half) ? d.aRow[tj].nbr[q] : -1;
+    const bool on = t2 >= 0 && d.aVS[t2] == 1;
+    double D2 = __builtin_inf(), f2 = 0.0, r2 = __builtin_inf();
+    float tn2 = -__builtin_inff();
+    CapRec cr = {0.0, 0.0, 0.0, 0.0, -1, sr.G, 0.0};
+    if (on) {
+      r2 = .5 * (d.ruq[tj] + d.ruq[t2]);
+      int vi, vy, vk;
+      decode(d, vj, vi, vy, vk);
+      const double ct[3] = {((double)(vi + ddx) + .5) * p.dx, ((double)(vy + ddy) + .5) * p.dy,
+                            ((double)(vk + ddz) + .5) * p.dz};
+      candidate_at(ct, c, R, &D2, &f2);
+      // and the bound for the cell that a capture through this entry would create
+      const int v2 = vj + ddz * d.nxy + ddy * p.nx + ddx;
+      double nc[3], ne;
+      recentre(d, vj, v2, c, R, f2, nc, &ne);
+      tn2 = first_capture_after(d, t2, v2, nc, ne, Rf);
+      cr.x = nc[0];
+      cr.y = nc[1];
+      cr.z = nc[2];
+      cr.E = ne;
+    }
+    const unsigned long long b2 = __ballot(on);
+    const int na = __popc((unsigned)b2), nb = __popc((unsigned)(b2 >> 32));
+    const int rank2 = list_rank(D2, r2, on, half);
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&d.ls->npre, na + nb);
+    base = __builtin_amdgcn_readfirstlane(base);
+    const bool fits = base >= 0 && base <= d.precap - na - nb;
+    const size_t at = (size_t)d.acap * AMCD_NB + (half ? base + na : base);
+    if (on && fits) {
+      d.cand[at + rank2] = {D2, r2, t2, q, tn2, (half ? nb : na) - rank2};
+      d.cF[at + rank2] = f2;
+      d.cap[at + rank2] = cr;
+    }
+    // the time to the new cell's first capture
+    const float tn = time_bound(D2 - E0, Vj);
+    const unsigned long long first = __ballot(on && rank2 == 0);
+    const unsigned fa = (unsigned)first, fb = (unsigned)(first >> 32);
+    if (fa != 0) {
+      const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tn), __builtin_ctz(fa)));
+      tnew = lane == j0 ? x : tnew;
+      pre = lane == j0 && fits ? d.acap * AMCD_NB + base : pre;
+    }
+    if (fb != 0) {
+      const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tn), 32 + __builtin_ctz(fb)));
+      tnew = lane == j1 ? x : tnew;
+      pre = lane == j1 && fits ? d.acap * AMCD_NB + base + na : pre;
+    }
   }
-  if (lane == 0) d.gN[slot] = (uint8_t)__popcll(bal);
+  if (liq) {
+    d.cand[cb + rank] = {D, r, t, lane, tnew, n - rank};
+    d.cF[cb + rank] = f;
+    d.cap[cb + rank] = {rc.x, rc.y, rc.z, rc.w, pre, sr.G, V};
+  }
+  if (lane == 0) d.slots[slot].n = n;
 }
 // every wave of an instance's blocks takes slots wave, wave + (its waves), ...
 __global__ __launch_bounds__(GB) void k_grow_lists(Inst* I, const int* bstart, int ninst) {
@@ -1255,32 +1371,60 @@ __global__ __launch_bounds__(GB) void k_grow_lists(Inst* I, const int* bstart, i
   const int nw = (bstart[ii + 1] - bstart[ii]) * (GB / 64);
   const int ns = d.ls->nslots;
   for (int slot = ((blockIdx.x - bstart[ii]) * GB + (int)threadIdx.x) >> 6; slot < ns; slot += nw)
-    if (!d.gDead[slot]) grow_list(d, slot, lane);
+    grow_list(d, slot, lane);
 }
 
-// The capture / nucleation loop of one instance (S/VoxelsCA.C:381-610): one workgroup
-// of NT threads per instance, in two roles.
-//   wave 0      the engine: performs each event (nucleation, or capture with octahedron
-//               re-centring, S/VoxelsCA.C:482-605) and builds the sorted candidate list
-//               of the newly mushy voxel;
-//   waves 1..   the owners: thread 64+j owns growing cells j, j+(NT-64), ... (K of them)
-//               and keeps each cell's half-diagonal E, velocity V, the head of its
-//               sorted candidate list and float bounds on its capture time in registers.
-// An event is EVAL | barrier | DECIDE | APPLY:
-//   EVAL    each owner wave finds its exact best candidate (t, ruqs, scan order) among
-//           the few cells whose time bounds reach the wave's smallest upper bound; the
-//           engine has already placed the best candidate of the cell it created last;
-//   DECIDE  every wave reads the per-wave bests and the pre-drawn uniform and reaches
-//           the same decision independently, so no second barrier is needed;
-//   APPLY   the owners grow their cells by V*Dt, take over the cell created in the
-//           previous event and re-read lists whose first live target was just captured,
-//           while the engine performs the event and evaluates the new cell.
-// The exchange areas are double-buffered by event parity: one barrier per event keeps
-// every wave within one event of the others.
+// (before the pass is run again in one step: the lists built ahead are allocated anew)
+__global__ void k_clear_npre(Inst* I) {
+  if (threadIdx.x == 0) I[blockIdx.x].ls->npre = 0;
+}
+
+// The capture / nucleation loop of one instance (S/VoxelsCA.C:381-610): one workgroup of NT
+// threads per instance.  The reference looks at every growing cell for every event; here an
+// event's only serial work is one wave's, and everything else happens once per window of
+// events.
+//
+// A candidate is a pair (growing cell, liquid neighbour) with the capture time
+// t = (D - E)/V of the cell's present half-diagonal E.  Between events E grows by V*Dt as the
+// clock T grows by Dt, so tau = T + t stays fixed up to rounding: float bounds [lo, hi] are kept
+// on the tau of each cell's first live candidate, and a thread holds E and V of its cells, j,
+// j + NT, ... in registers.  A window is a clock value W and every candidate with lo <= W (its
+// entries, at most 64):
+//   SELECT   a histogram of the lower bounds gives the W that takes about `want` heads (at least
+//            the smallest upper bound); the threads write the entries of their cells to LDS, and,
+//            where a cell that a capture creates may itself capture before W, the entries of the
+//            list built ahead for it, relative to the capture's own bounds;
+//   ENGINE   wave 0, one entry per lane, performs events while the smallest upper bound of its
+//            live entries stays below W: exact times (S/VoxelsCA.C:420-440), the first by (t, ruqs,
+//            scan order), the event's uniform draw, T += Dt, E += V*Dt of its lanes, and the
+//            captured voxel's entries drop out.  No candidate outside the window can come first:
+//            their lower bounds exceed W, and the earliest capture by a cell that an event creates
+//            is bounded from below by the set-up (CandRec::tn), which ends the window where the
+//            bound falls below W and the cell's candidates are not entries themselves;
+//   BUILD    meanwhile the other waves create the cells of the events as they are published:
+//            grain, centre, half-diagonal, list (S/VoxelsCA.C:396-440, 486-506, 528-605);
+//   APPLY    heads that died move to the next live candidate (the cells are listed in LDS first, so
+//            that their list reads run side by side), new cells are taken over, and the window's
+//            growth E += V*Dt is replayed event by event, in the reference's order of additions,
+//            so every half-diagonal has the reference's bits.
+// A window that does not fit takes less of the clock; one too full even at W = the smallest upper
+// bound (many candidates within rounding of each other) takes the exact best of every wave as its
+// entries and performs one event.
+//
+// What bounds it: a chain of dependent instructions.  An event is about 100 instructions of one
+// wave (11 to 13 cycles each), and every window pays five barriers and two rounds of list reads;
+// hence as many events per window as its 64 entries give (25 where the interface is wide, 8 where
+// a cell captures within a step of its own capture), records that are one cache line, and lists
+// and capture constants made by the set-up's parallel pass.  One wave per event with the window
+// built around each event took 6.9K cycles an event in these decks and 13.7K with the state in
+// memory; now (cycles per event, 2.4 GHz): 5.6K with few growing cells (at most 300), 3.0K with
+// 3 thousand, 2.9K with 3 thousand of a raster over a wide plate, 10.1K with 15 thousand (state in
+// memory).
+typedef const __attribute__((address_space(4))) Inst CInst;
 struct Best {
   double t, r;
   int key;   // scan position * 32 + neighbour rank: the reference's scan order
-  int cand;  // candidate entry (slot * AMCD_NB + position)
+  int cand;  // candidate entry (slot * AMCD_NB + position), or the lane that holds it
   int tgt;   // active index of the captured voxel
 };
 __device__ static inline Best best_none() {
@@ -1392,136 +1536,76 @@ __device__ static inline bool cand_less(double Da, double Ra, int ka, double Db,
   return (c1 & nb) | (!c1 & c2 & (Da < Db)) | (!c1 & !c2 & tail);
 }
 
-// Liveness of candidate targets during the loop: an LDS bitmap over active cells with
-// bit set = "not liquid" (filled from the state at launch, then set by the engine for
-// every voxel it captures or nucleates).  Every list entry was liquid when the lists
-// were built, so a clear bit means live.
+// Liveness of candidate targets: an LDS bitmap over the active cells, bit set = "not liquid"
+// (filled from the states at launch, set for every voxel captured or nucleated), or, for
+// interfaces of more than AMCD_DEAD_BITS cells, the state bytes themselves.  Every list entry was
+// liquid when its list was built, so "not dead" means live, and a dead entry stays dead.
 #define AMCD_DEAD_BITS (1 << 19)
-__device__ static inline bool dead_bit(const unsigned* dead, int t) { return (dead[t >> 5] >> (t & 31)) & 1u; }
-__device__ static inline bool live_target(const unsigned* dead, int t, int skip) {
-  return t >= 0 && t != skip && !dead_bit(dead, t);
-}
+template <bool GD>
+struct Liveness {
+  unsigned* bits;
+  uint8_t* vs;
+  __device__ __forceinline__ bool dead(int t) const {
+    if constexpr (GD)
+      return gmem(vs)[t] != 1;
+    else
+      return (bits[t >> 5] >> (t & 31)) & 1u;
+  }
+  __device__ __forceinline__ void kill(int t) const {  // (lanes of one wave, each its own voxel)
+    if constexpr (!GD) atomicOr(&bits[t >> 5], 1u << (t & 31));
+  }
+};
 
-// First live entry at or after position `from` of slot s's sorted list, read four
-// entries at a time (one round of loads in the common case).  Entries before the
-// first live one stay dead: a captured voxel never becomes liquid again within the
-// step.  `skip` is a voxel that counts as dead although its bit may not be set yet.
+// A list record as two 16-byte loads.
+__device__ static inline CandRec load_rec(const CandRec* p) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  const auto q = gmem((const v2d*)p);
+  const v2d x = q[0], y = q[1];
+  const unsigned long long a = (unsigned long long)__double_as_longlong(y.x);
+  const unsigned long long b = (unsigned long long)__double_as_longlong(y.y);
+  return {x.x, x.y, (int)a, (int)(a >> 32), __int_as_float((int)b), (int)(b >> 32)};
+}
+// First live entry of a sorted list from entry `from` on, four records at a time with no branches
+// between the loads.  Positions past the list's end read what follows it, at the array's end the
+// 256 bytes every device array is allocated beyond its length; they are never used.
 struct SlotHead {
-  double D1, Dn, r1;  // head distance, the next entry's distance (+inf: none), head ruqs
-  int c1, tgt1, k1;   // head entry, its target (-1: no live entry), its neighbour rank
+  double D1;
+  int c1, tgt1;  // head entry and its target (-1: no live entry)
 };
-// Positions p .. p+3 of a list and the distance at p+4 (p <= 26), read from one base
-// address per array with no branches.  Positions past a slot's 26 entries read the next
-// slot, or for the last slot the 256 bytes every device array is allocated beyond its
-// length; they lie beyond the list length and are never used.
-// The four neighbour ranks stay packed in one word until a head is picked: unpacked at
-// the load, they would make the loads of a block that is issued early wait there.
-struct SlotBlock {
-  double D[5], R[4];
-  int t[4], n;
-  unsigned kp;  // rank of position p + q in bits 8q .. 8q+7
-};
-typedef unsigned u32_any_align __attribute__((aligned(1)));
-__device__ static inline void block_entries(const Inst& d, size_t cb, int p, SlotBlock& b) {
-  const size_t e = cb + p;
-  b.kp = *gmem((u32_any_align*)(d.cK + e));  // four ranks, little-endian: one load
-#pragma unroll
-  for (int q = 0; q < 5; ++q) {
-    b.D[q] = gmem(d.cD)[e + q];
-    if (q < 4) {
-      b.t[q] = gmem(d.cTgt)[e + q];
-      b.R[q] = gmem(d.cR)[e + q];
-    }
-  }
-}
-// The first live entry among positions p .. p+3 of a loaded block into h: true when
-// found or when the list ends before p (h unchanged), false to go on at p + 4.  The four
-// liveness words are read unconditionally (an entry past the list end reads word 0), so
-// that they are requested together: read under each entry's own condition, every read
-// waited for the one before.
-__device__ static inline bool block_pick(const SlotBlock& b, const unsigned* dead, size_t cb, int p, int skip,
-                                         SlotHead& h) {
-  if (p >= b.n) return true;
-  int tq[4];
-  unsigned wq[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    tq[q] = (p + q < b.n && b.t[q] >= 0) ? b.t[q] : -1;
-    wq[q] = dead[(tq[q] >= 0 ? tq[q] : 0) >> 5];
-  }
-  int hit = -1;
-#pragma unroll
-  for (int q = 3; q >= 0; --q) {
-    const bool live = (tq[q] >= 0) & (tq[q] != skip) & (((wq[q] >> (tq[q] & 31)) & 1u) == 0);
-    hit = live ? q : hit;
-  }
-  if (hit < 0) return false;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    if (q == hit) {
-      h.c1 = (int)cb + p + q;
-      h.tgt1 = b.t[q];
-      h.D1 = b.D[q];
-      h.Dn = (p + q + 1 < b.n) ? b.D[q + 1] : __builtin_inf();
-      h.r1 = b.R[q];
-      h.k1 = (int)((b.kp >> (8 * q)) & 0xffu);
-    }
-  return true;
-}
-__device__ static inline SlotHead head_none(size_t cb, int n) {
+template <bool GD>
+__device__ static inline SlotHead slot_head(CInst& d, const Liveness<GD>& live, int from) {
   SlotHead h;
-  h.c1 = (int)cb + n;
   h.tgt1 = -1;
-  h.k1 = 0;
-  h.D1 = h.Dn = h.r1 = __builtin_inf();
-  return h;
-}
-// First live entry at or after position `from` of slot s.  The entries are read four at
-// a time together with the list length, so the common case is one round of loads
-// (positions past the length hold stale data and are masked afterwards).
-__device__ static inline SlotHead slot_head(const Inst& d, const unsigned* dead, int s, int from, int skip) {
-  const size_t cb = (size_t)s * AMCD_NB;
-  SlotBlock b;
-  b.n = gmem(d.gN)[s];
-  // the default head is set after the search, so that the length is not waited for
-  // before the entries are requested
-  SlotHead h = head_none(cb, 0);
-  for (int p = from; p < AMCD_NB; p += 4) {
-    block_entries(d, cb, p, b);
-    if (block_pick(b, dead, cb, p, skip, h)) break;
-  }
-  if (h.tgt1 < 0) h.c1 = (int)cb + b.n;
-  return h;
-}
-// slot_head's first block (positions p .. p+3, the distance at p+4 and the list length)
-// loaded ahead of its use, and the same search started from it.
-__device__ static inline SlotBlock slot_block(const Inst& d, int s, int p) {
-  SlotBlock b;
-  b.n = gmem(d.gN)[s];
-  block_entries(d, (size_t)s * AMCD_NB, p, b);
-  return b;
-}
-__device__ static inline SlotBlock slot_block_none() {
-  SlotBlock b;
+  h.D1 = __builtin_inf();
+  h.c1 = from;
+  for (int p = from;; p += 4) {
+    CandRec e[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    b.t[q] = -1;
-    b.D[q] = b.R[q] = 0.0;
+    for (int q = 0; q < 4; ++q) e[q] = load_rec(d.cand + p + q);
+    const int n = e[0].n;  // entries from position p on
+    bool dd[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // (an entry past the list end asks about cell 0)
+      const int t = q < n ? e[q].tgt : 0;
+      dd[q] = live.dead(t) | (q >= n);
+    }
+    int hit = -1;
+#pragma unroll
+    for (int q = 3; q >= 0; --q) hit = dd[q] ? hit : q;
+    if (hit < 0) {
+      if (n <= 4) break;
+      continue;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q == hit) {
+        h.c1 = p + q;
+        h.tgt1 = e[q].tgt;
+        h.D1 = e[q].D;
+      }
+    break;
   }
-  b.D[4] = 0.0;
-  b.n = 0;
-  b.kp = 0;
-  return b;
-}
-// slot_head(d, dead, s, from, skip) with its first block b = slot_block(d, s, from)
-// already loaded: the same result, the later blocks read only when the first holds no
-// live entry
-__device__ static inline SlotHead slot_head_pre(const Inst& d, const unsigned* dead, int s, int from, int skip,
-                                                const SlotBlock& b) {
-  const size_t cb = (size_t)s * AMCD_NB;
-  SlotHead h = head_none(cb, b.n);
-  if (from >= AMCD_NB || block_pick(b, dead, cb, from, skip, h)) return h;
-  return slot_head(d, dead, s, from + 4, skip);
+  return h;
 }
 
 // Float bounds [lo, hi] on tau = T + t, the event clock at which the cell's head would
@@ -1553,1077 +1637,1217 @@ __device__ static inline void tau_bounds(double D1, double e, double v, double T
   }
 }
 
-struct NewCell {  // a growing cell created by the engine, taken over by its owner
-  double E, V, D1, Dn1, r1;  // extent, velocity, head distance, next distance, head ruqs
-  int c1, tgt1, key1, slot, valid;
-};
-struct EngineShared {
-  Best sb[2][16];   // per-wave bests, by event parity
-  double ubuf[2][64];  // uniforms of draws 64b .. 64b+63 of this launch in ubuf[b & 1]
-  int susp[2];      // engine suspension request (-1 pool refill, -2 larger tier), by parity
-  NewCell mb[2];    // cell created in the event of this parity
-  int nslots;
-  int r_i1;         // resume: pending nucleation target
-  int fin;          // exit code of the loop
+// Phase timers of the loop (shader-clock cycles of wave 0), compiled in only with
+// -DAMCD_PHASE_PROFILE; read with amcd_phase_profile().
 #ifdef AMCD_PHASE_PROFILE
-  unsigned long long arr[2][16];
-  int aflag[2][16];
+__device__ unsigned long long g_phase[32];
+#define PHASE_INIT(v) unsigned long long v = clock64()
+#define PHASE(v, slot)                                        \
+  do {                                                        \
+    const unsigned long long t_ = clock64();                  \
+    if (threadIdx.x == 0) atomicAdd(&g_phase[slot], t_ - v);  \
+    v = t_;                                                   \
+  } while (0)
+#else
+#define PHASE_INIT(v)
+#define PHASE(v, slot)
 #endif
+
+// ---- windows
+constexpr int WCAP = 64;   // entries of a window: one per lane of the engine wave
+constexpr int TCAP = 256;  // touched cells (heads that died) listed per window
+struct Window {
+  // entries
+  double D[WCAP], E[WCAP], V[WCAP], r[WCAP];
+  int tgt[WCAP], key[WCAP], cand[WCAP], own[WCAP];  // own: the entry's cell (slot)
+  int lo[WCAP], hi[WCAP];  // bounds, as order keys
+  int lim[WCAP];  // after a capture through the entry: the largest bound that the new cell cannot precede
+  double y[WCAP];   // reciprocal of V
+  int parent[WCAP]; // the entry whose capture creates this one's cell (-1: the cell is there)
+  int rank[WCAP];   // position by hi
+  // events, in order: entry (-1: nucleation, -2: not performed yet) and voxel, published one by
+  // one; growth time; the slot of the cell it created (-1: none)
+  int2 ev[WCAP];
+  double dt[WCAP];
+  int slot[WCAP], base[WCAP];  // (base: its list's first entry)
+  double E0[WCAP], V0[WCAP];
+  int n;        // entries asked for (more than WCAP: the window is too full)
+  int m;        // events
+  int decided;  // events decided in this window (one more than m when the last waits for the pool)
+  int scan0;    // scan position of the first event's voxel
+  int G, pool;  // the nucleation's grain and pool entry (a window has at most one, its last event)
+  int done;     // the engine has published its last event
+  unsigned x2[WCAP];         // random engine states after the window's draws
+  unsigned long long draws;  // bit m: event m nucleates
 };
-// The decision every wave takes after the barrier (S/VoxelsCA.C:476-485).
-struct Decision {
-  int stop, nuc, i1, cand, wave;
-  double dt;
+struct LoopShared {
+  Window win;
+  // cells whose head died in the window, with their half-diagonal before it (for a cell that ran
+  // out of candidates: after it)
+  double tE[TCAP], tV[TCAP];
+  int tS[TCAP], tn;
+  float red[16];
+  int hist[32];  // heads by lower bound, in thirty-seconds of twice the window's span
+  int nslots;
+  int fin;  // 1: goes on, 0: finished, -1: pool refill, -2: larger tier, -4: no progress
+  double T;
+  int go, r_i1, all, neg, nexec;
+  unsigned cur;  // random engine state
+  unsigned long long units;
 };
-// Lane q < NW reads wave q's best (one entry per lane, so the eight waves that decide at
-// once after the barrier do not queue on the LDS for the whole table each), and the
-// tournament runs across lanes with row shifts: at level h lane q compares its entry
-// with lane q + h's.  `nd` is the number of draws this launch has consumed, which
-// selects the event's uniform.
-template <int H>
-__device__ static inline int row_from(int v) {  // lane i takes lane i + H of its row of 16
-  return __builtin_amdgcn_update_dpp(v, v, 0x100 + H, 0xf, 0xf, false);
+
+// The workgroup's exchange: the window, the liveness bitmap and, for the register tiers, every
+// cell's bounds and list head (one workgroup runs on a CU at a time).  File scope, for the routine
+// that is kept out of line.
+constexpr int LDS_CELLS = 4096;
+__shared__ LoopShared s_loop;
+__shared__ unsigned s_dead_bits[AMCD_DEAD_BITS / 32];
+__shared__ float2 s_lh[LDS_CELLS];
+__shared__ int2 s_hd[LDS_CELLS];
+
+// A cell's bounds and head: in LDS for the register tiers, else in memory.
+template <bool MEM>
+__device__ static inline float2 get_lh(CInst& d, int s) {
+  if constexpr (MEM) return gload8(d.gLH + s);
+  else return s_lh[s];
 }
-template <int H>
-__device__ static inline double row_from(double v) {
+template <bool MEM>
+__device__ static inline void set_lh(CInst& d, int s, float lo, float hi) {
+  if constexpr (MEM) gstore8(d.gLH + s, make_float2(lo, hi));
+  else s_lh[s] = make_float2(lo, hi);
+}
+template <bool MEM>
+__device__ static inline int2 get_hd(CInst& d, int s) {
+  if constexpr (MEM) return gload8(d.gHd + s);
+  else return s_hd[s];
+}
+template <bool MEM>
+__device__ static inline void set_hd(CInst& d, int s, int c1, int tgt) {
+  if constexpr (MEM) gstore8(d.gHd + s, make_int2(c1, tgt));
+  else s_hd[s] = make_int2(c1, tgt);
+}
+
+// A thread's half-diagonals and velocities: K cells in registers (or a batch of K streamed from
+// memory).  A cell without candidates has velocity 0.
+template <int K>
+struct Cells {
+  double E[K], V[K];
+};
+
+__device__ static inline double pack2(int lo, int hi) {
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// Float bounds as integers in the same order (no NaN among them): minima and comparisons are
+// then one instruction each, with the lane permutation as an operand modifier.
+__device__ static inline int order_key(float f) {
+  const int i = __float_as_int(f);
+  return i ^ ((i >> 31) & 0x7fffffff);
+}
+constexpr int kKeyInf = 0x7f800000, kKeyNone = 0x7fffffff;  // +inf; after every bound
+template <int CTRL, int ROWS = 0xf>
+__device__ static inline int dpp_min(int v) {
+  return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
+}
+__device__ static inline int wave_min(int v) {
+  v = dpp_min<kQuadX1>(v);
+  v = dpp_min<kQuadX2>(v);
+  v = dpp_min<kHalfMirror>(v);
+  v = dpp_min<kMirror>(v);
+  v = dpp_min<kBcast15, 0xa>(v);
+  v = dpp_min<kBcast31, 0xc>(v);
+  return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ static inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ static inline double uni(double v) {
   const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)row_from<H>((int)b), hi = (unsigned)row_from<H>((int)(b >> 32));
+  const unsigned lo = (unsigned)uni((int)b), hi = (unsigned)uni((int)(b >> 32));
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
-template <int NW, int H>
-__device__ static inline void tournament_level(Best& e, int& wi) {
-  if constexpr (H < NW) {
-    Best o;
-    o.t = row_from<H>(e.t);
-    o.r = row_from<H>(e.r);
-    o.key = row_from<H>(e.key);
-    o.cand = row_from<H>(e.cand);
-    o.tgt = row_from<H>(e.tgt);
-    const int ow = row_from<H>(wi);
-    const bool bt = better(o, e);
-    e.t = bt ? o.t : e.t;
-    e.r = bt ? o.r : e.r;
-    e.key = bt ? o.key : e.key;
-    e.cand = bt ? o.cand : e.cand;
-    e.tgt = bt ? o.tgt : e.tgt;
-    wi = bt ? ow : wi;
-    tournament_level<NW, 2 * H>(e, wi);
-  }
-}
-template <int NW>
-__device__ static inline Best lane_entry(const EngineShared& sh, int par) {  // wave `lane`'s best
-  static_assert(NW <= 16, "one row of lanes");
-  const int lane = threadIdx.x & 63;
-  Best e = best_none();
-  if (lane < NW) e = sh.sb[par][lane];
-  return e;
-}
-template <int NW>
-__device__ static inline Decision decide_from(const EngineShared& sh, Best e, int par, double T, double DelT,
-                                              double rX, int nd) {
-  const int lane = threadIdx.x & 63;
-  int wi = lane;
-  const double U = sh.ubuf[(nd >> 6) & 1][nd & 63];
-  const int susp = sh.susp[par];
-  // The smallest time first (three row shifts of one double): when a single entry holds it,
-  // that entry is the best whatever its ruqs and key.  Otherwise the pairwise tree, the
-  // left entry kept unless the right one is strictly better: the first best entry in wave
-  // order, as a sequential scan finds it (the order is a strict weak order: times and ruqs
-  // are never NaN here).
-  double tm = e.t;
-  tm = fmin(tm, row_from<1>(tm));
-  tm = fmin(tm, row_from<2>(tm));
-  tm = fmin(tm, row_from<4>(tm));
-  static_assert(NW <= 8, "three levels cover the entries");
-  const double t0 = lane_f64(tm, 0);
-  const unsigned long long at_min = __ballot((lane < NW) & (e.cand >= 0) & (e.t == t0));
-  int wq;
-  Best b;
-  if (__popcll(at_min) == 1) {
-    wq = __builtin_ctzll(at_min);
-    b = lane_best(e, wq);
-  } else {
-    tournament_level<NW, 1>(e, wi);
-    b.t = lane_f64(e.t, 0);
-    b.r = lane_f64(e.r, 0);
-    b.key = __builtin_amdgcn_readlane(e.key, 0);
-    b.cand = __builtin_amdgcn_readlane(e.cand, 0);
-    b.tgt = __builtin_amdgcn_readlane(e.tgt, 0);
-    wq = __builtin_amdgcn_readlane(wi, 0);
-  }
-  // branch-free, so that the reads of the uniform and the suspension flag are issued
-  // with the read of the bests and not one after another
-  Decision x;
-  const bool run = T < DelT;                      // loop condition (S/VoxelsCA.C:381)
-  const bool none = (b.cand < 0) | (b.t >= 1e6);  // S/VoxelsCA.C:480
-  const bool go = run & (susp == 0) & !none;
-  const bool nuc = U < rX;
-  x.stop = !run ? 1 : (susp != 0 ? susp : (none ? 1 : 0));
-  x.nuc = go & nuc;
-  x.i1 = b.tgt;
-  x.cand = b.cand;
-  x.wave = wq;
-  x.dt = (go & !nuc) ? b.t : 0.0;
-  return x;
-}
-template <int NW>
-__device__ static inline Decision decide(const EngineShared& sh, int par, double T, double DelT, double rX, int nd) {
-  return decide_from<NW>(sh, lane_entry<NW>(sh, par), par, T, DelT, rX, nd);
-}
-// What the engine needs to perform a capture, loaded for every wave's best while the
-// decision is being taken: lane q < NW holds the entry of wave q's best (target voxel,
-// capturing cell's grain and rotation, the target's cold flag and temperature, the
-// set-up's re-centring), and lane l holds positions l, l + 64, l + 128, l + 192 of the
-// candidates' neighbour rows laid end to end (26 per candidate).
-struct EnginePrefetch {
-  double R[9], T1, rpn[4];
-  double4 rc;
-  int v1, G, cold, nbr[4];
-};
-template <int NW>
-__device__ static inline EnginePrefetch engine_prefetch(const Inst& d, const EngineShared& sh, const Best& e, int par,
-                                                        int ns_pre) {
-  // branch-free, with every index clamped into its array (a lane without an entry reads
-  // entry 0), so that the loads are issued here and not moved past the decision
-  const int lane = threadIdx.x & 63;
-  EnginePrefetch f;
-  const int cand = e.cand >= 0 ? e.cand : 0, tgt = e.tgt >= 0 ? e.tgt : 0;
-  const size_t sw = (size_t)(cand / AMCD_NB);
-  f.v1 = gmem(d.cV)[cand];
-  f.G = gmem(d.gG)[sw];
-  f.cold = gmem(d.aCold)[tgt];
-  f.T1 = gmem(d.aT)[tgt];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) f.R[q] = gmem(d.gR)[9 * sw + q];
-  {  // meaningful for entries of set-up lists only
-    const auto q = gmem((double*)(d.cRC + cand));
-    f.rc = make_double4(q[0], q[1], q[2], q[3]);
-  }
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int fl = lane + 64 * m, q = min(fl / AMCD_NB, NW - 1), j = fl - (fl / AMCD_NB) * AMCD_NB;
-    int tq = sh.sb[par][q].tgt;
-    tq = tq >= 0 ? tq : 0;
-    f.nbr[m] = gmem(d.aNbr)[(size_t)tq * AMCD_NB + j];
-    f.rpn[m] = gmem(d.aRN)[(size_t)tq * AMCD_NB + j];
-  }
-  return f;
-}
-// keeps the prefetched registers live at this point: the loads must have been issued
-// before it, and their wait is placed here
-__device__ static inline void prefetch_landed(const EnginePrefetch& f) {
-  asm volatile("" ::"v"(f.v1), "v"(f.G), "v"(f.cold), "v"(f.T1), "v"(f.rc.x), "v"(f.rc.y), "v"(f.rc.z),
-               "v"(f.rc.w), "v"(f.nbr[0]), "v"(f.nbr[1]), "v"(f.nbr[2]), "v"(f.nbr[3]), "v"(f.rpn[0]),
-               "v"(f.rpn[1]), "v"(f.rpn[2]), "v"(f.rpn[3]));
-  asm volatile("" ::"v"(f.R[0]), "v"(f.R[1]), "v"(f.R[2]), "v"(f.R[3]), "v"(f.R[4]), "v"(f.R[5]), "v"(f.R[6]),
-               "v"(f.R[7]), "v"(f.R[8]));
-}
-// lane j < AMCD_NB takes position j of wave wq's neighbour row from the prefetch
-__device__ static inline void take_row(const EnginePrefetch& f, int wq, int lane, int& tn, double& rp) {
-  const int fl = wq * AMCD_NB + (lane < AMCD_NB ? lane : 0), src = (fl & 63) << 2, m = fl >> 6;
-  int t = -1, lo = 0, hi = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int a = __builtin_amdgcn_ds_bpermute(src, f.nbr[k]);
-    const long long b = __double_as_longlong(f.rpn[k]);
-    const int bl = __builtin_amdgcn_ds_bpermute(src, (int)b), bh = __builtin_amdgcn_ds_bpermute(src, (int)(b >> 32));
-    t = m == k ? a : t;
-    lo = m == k ? bl : lo;
-    hi = m == k ? bh : hi;
-  }
-  tn = lane < AMCD_NB ? t : -1;
-  rp = lane < AMCD_NB ? __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo))
-                      : 0.0;
-}
-// Uniforms 64b .. 64b+63 of a launch whose engine state was x0 at its start: lane j
-// jumps to x0 * 16807^(128b + 2j + 1) (aj = 16807^(2j+1), cb = 16807^(128b)).
-__device__ static inline double draw_batch(unsigned int x0, unsigned int cb, unsigned int aj) {
-  const unsigned int xb = mod_m((unsigned long long)x0 * cb);
-  const unsigned int x1 = mod_m((unsigned long long)xb * aj);
-  return canonical(x1, lcg_next(x1));
+
+template <int CTRL, int ROWS = 0xf>
+__device__ static inline int dpp_min_shift(int v) {  // with the lane's lower neighbour by the row shift
+  return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
 }
 
-// The register tiers keep each cell's head distance and next distance in LDS and its scan
-// key in a register, so that EVAL reads no global memory unless a tie has to be walked.  Up
-// to eight cells per owner thread the head's ruqs are in LDS too; the sixteen-cell tier
-// (7,168 cells) has room for two doubles per cell and reads the ruqs from the list, a load
-// issued with the LDS reads and needed only after the divisions.  The memory-resident tier
-// reads the head from the lists.
-template <int K>
-struct HeadCache {
-  static constexpr bool on = K > 0 && K <= 16;
-  static constexpr bool ruqs = K > 0 && K <= 8;
-  static constexpr int words = ruqs ? 3 : 2;  // doubles per cell
-};
-// Liveness bits in LDS: the 16-cells-per-thread tier gives half of them to its head cache, and
-// an interface beyond them runs in the memory-resident tier with the bitmap in memory.
-template <int K, bool GD>
-struct DeadBits {
-  static constexpr int n = GD ? 32 : (K == 16 ? (1 << 18) : AMCD_DEAD_BITS);
-};
-// Kept out of line: inlined into the kernel beside the engine's loop, the register tiers'
-// loops ran about 1% slower per event.
-template <int NT, int K>
-__device__ __attribute__((noinline)) static void owner_loop(const Inst& d_lds, EngineShared& sh,
-                                                            const unsigned* dead, double* hc, int go, double T,
-                                                            long long& visits_out, long long& evals_out) {
-  // The descriptor's fields in registers: read through the LDS copy, each would be read again
-  // after every store to LDS (head cache, bests, liveness), which might alias it.
-  const Inst d = d_lds;
-  constexpr bool HC = HeadCache<K>::on, HR = HeadCache<K>::ruqs;
-  // the refresh's block loaded ahead of its use (its registers spilled in the 16-cell tier)
-  constexpr bool PF = HC && K <= 8;
-  constexpr int HN = (NT - 64) * K;  // head-cache slots (one per cell of the tier)
-  // work counters are kept in registers and handed back once at the end (a reference
-  // incremented inside the loop would live in scratch memory)
-  long long visits = 0, evals = 0;
-  constexpr int NO = NT - 64;  // owner threads
-  constexpr int NW = NT / 64;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int me = tid - 64;
-  const float fInf = __builtin_inff();
-  const amcd_params& p = d.p;
-  // loop constants held in registers (a read through the descriptor in LDS would be
-  // repeated after every barrier)
-  const double DelT = p.DelT, rX = p.rX;
-  double E[K], V[K];
-  float lo[K], hi[K];
-  // c1: the head entry; with the head cache, its position in the slot's list (5 bits)
-  // packed with its scan key (scan position * 32 + neighbour rank, < 2^24) above them
-  int c1[K], tgt1[K];
-  const bool loaded = go != -2;
-  const int ns0 = sh.nslots;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int s = me + k * NO;
-    E[k] = V[k] = 0.0;
-    lo[k] = hi[k] = fInf;
-    c1[k] = 0;
-    tgt1[k] = -1;
-    if (loaded && s < ns0) {
-      E[k] = gmem(d.gExt)[s];
-      V[k] = gmem(d.gVhat)[s];
-      const SlotHead h = slot_head(d, dead, s, 0, -1);
-      c1[k] = h.c1;
-      tgt1[k] = h.tgt1;
-      if constexpr (HC) {
-        c1[k] = (h.c1 - s * AMCD_NB) | ((gmem(d.gScan)[s] * 32 + h.k1) << 5);
-        hc[s] = h.D1;
-        hc[HN + s] = h.Dn;
-        if constexpr (HR) hc[2 * HN + s] = h.r1;
-      }
-      if (h.tgt1 >= 0) tau_bounds(h.D1, E[k], V[k], T, lo[k], hi[k]);
-      // bring the rest of the list (positions 16..25 of the distances and ruqs, the
-      // targets' line) into the cache: later head refreshes read it within the event
-      const size_t cb = (size_t)s * AMCD_NB;
-      const double w0 = gmem(d.cD)[cb + 16], w1 = gmem(d.cR)[cb + 16];
-      const int w2 = gmem(d.cTgt)[cb + 25];
-      asm volatile("" ::"v"(w0), "v"(w1), "v"(w2));
-    }
-  }
-  int skip = -1;  // voxel the engine may be capturing right now
-  int par = 0;
-  int nd = 0;     // draws consumed by this launch
-  int nev = 0;    // events since the bounds were last recomputed
-  Decision x;
-  x.stop = 0;
-  x.nuc = 1;
-  x.i1 = sh.r_i1;
-  x.dt = 0.0;
-  bool apply_first = go == 2;
-  PHASE_FLAGS(aflag);
-  int ks = -1;  // the cell whose list block pb is loaded for its head refresh (-1: none)
-  SlotBlock pb = slot_block_none();
-  PHASE_INIT(ot);
-  while (go > 0) {
-    // The slot numbers are re-derived from an opaque copy of the thread index in every
-    // iteration: otherwise the compiler keeps per-cell addresses live across the loop,
-    // which costs more registers than the cell state itself.
-    int mo = me;
-    asm volatile("" : "+v"(mo));
-    if (!apply_first) {
-      // ---- EVAL
-      float u = fInf;
-#pragma unroll
-      for (int k = 0; k < K; ++k) u = fminf(u, hi[k]);
-      u = wave_min(u);
-      Best b = best_none();
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        if (lo[k] != fInf && lo[k] <= u) {
-          // exact capture time of the cell's head (S/VoxelsCA.C:420-440)
-          const int s = mo + k * NO;
-          const int c = HC ? s * AMCD_NB + (c1[k] & 31) : c1[k];
-          const int pos = c - s * AMCD_NB;
-          const double e = E[k], v = V[k];
-          double D1, Dn, rr;
-          int kb, ky;
-          if constexpr (HC) {
-            D1 = hc[s];
-            Dn = hc[HN + s];
-            rr = HR ? hc[2 * HN + s] : gmem(d.cR)[c];
-            ky = c1[k] >> 5;
-            kb = ky & ~31;
-          } else {
-            D1 = gmem(d.cD)[c];
-            Dn = (pos + 1 < AMCD_NB) ? gmem(d.cD)[c + 1] : __builtin_inf();
-            rr = gmem(d.cR)[c];
-            kb = gmem(d.gScan)[s] * 32;
-            ky = kb + gmem(d.cK)[c];
-          }
-          visits++;
-          evals++;
-          // the head's time and the next entry's, side by side (one round of head reads,
-          // two independent divisions)
-          const double t1 = (D1 - e) / v;
-          const double tn = (Dn - e) / v;
-          const bool ok = t1 <= 1e6;
-          {
-            Best y;
-            y.t = t1;
-            y.r = rr;
-            y.key = ky;
-            y.cand = c;
-            y.tgt = tgt1[k];
-            // times are non-decreasing along the list: a tie needs the next entry's
-            // time to equal t1; then walk the tied block
-            if (ok & (tn == t1)) {
-              PHASE_FLAG(aflag, 2);
-              const int n = gmem(d.gN)[s];
-              for (int q = pos + 1; q < n; ++q) {
-                const int tq = gmem(d.cTgt)[c - pos + q];
-                if (!live_target(dead, tq, skip)) continue;
-                evals++;
-                const double tt = (gmem(d.cD)[c - pos + q] - e) / v;
-                if (!(tt == t1)) break;
-                Best z;
-                z.t = tt;
-                z.r = gmem(d.cR)[c - pos + q];
-                z.key = kb + gmem(d.cK)[c - pos + q];
-                z.cand = c - pos + q;
-                z.tgt = tq;
-                if (better(z, y)) y = z;
-              }
-            }
-            if (ok && better(y, b)) b = y;
-          }
-        }
-      }
-      b = wave_best(b);
-      if (lane == 0) sh.sb[par][w] = b;
-      PHASE(ot, 7, tid == 64);
-      PHASE_ARRIVE(sh, par, w, aflag);
-      PHASE_FLAGS_CLEAR(aflag);
-      __syncthreads();
-      PHASE(ot, 8, tid == 64);
-      // ---- DECIDE
-      const Best eb = lane_entry<NW>(sh, par);
-      x = decide_from<NW>(sh, eb, par, T, DelT, rX, nd);
-      if (x.stop) break;
-      ++nd;
-      PHASE(ot, 5, tid == 64);
-    }
-    apply_first = false;
-    // the cell (first of each thread) whose head is the voxel captured now: the next
-    // block of its list is loaded before the growth and the takeover below, and waited
-    // for where the refresh of its head uses it
-    if constexpr (PF) {
-      ks = -1;
-      int pk = 0;
-#pragma unroll
-      for (int k = K - 1; k >= 0; --k) {
-        const bool take = (tgt1[k] == x.i1) & (tgt1[k] >= 0);
-        ks = take ? k : ks;
-        pk = take ? c1[k] : pk;
-      }
-      if (ks >= 0) pb = slot_block(d, mo + ks * NO, (pk & 31) + 1);
-    }
-    // ---- APPLY
-    const double Dt = x.dt;
-    if (!x.nuc) {  // growth of every cell growing at this scan (S/VoxelsCA.C:511-516)
-      // straight-line over the K cells, so that their updates interleave
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const bool grows = tgt1[k] >= 0;
-        const double e = E[k] + V[k] * Dt;
-        const bool clamp = grows & (e < 0.0);
-        E[k] = grows ? (clamp ? 0.0 : e) : E[k];
-        lo[k] = clamp ? -fInf : lo[k];  // clamped: recompute the bounds below
-      }
-    }
-    T = T + Dt;  // the engine's tinc: same additions in the same order
-    const int i1 = x.i1;
-    // the cell created by the previous event (its best was evaluated by the engine)
-    const NewCell& nc = sh.mb[par];
-    if (nc.valid && nc.slot % NO == mo) {
-      PHASE_FLAG(aflag, 4);
-      const int kk = nc.slot / NO;
-      double e = nc.E;
-      if (!x.nuc) {
-        const double g = e + nc.V * Dt;
-        e = (g < 0.0) ? 0.0 : g;
-      }
-#pragma unroll
-      for (int k = 0; k < K; ++k)
-        if (k == kk) {
-          E[k] = e;
-          V[k] = nc.V;
-          c1[k] = HC ? nc.key1 << 5 : nc.c1;  // the head is entry 0
-          tgt1[k] = nc.tgt1;
-          lo[k] = -fInf;  // bounds below (its head may also be the voxel captured now)
-        }
-      if constexpr (HC) {
-        hc[nc.slot] = nc.D1;
-        hc[HN + nc.slot] = nc.Dn1;
-        if constexpr (HR) hc[2 * HN + nc.slot] = nc.r1;
-      }
-      if (ks == kk) ks = -1;  // a block loaded for the slot's previous state
-    }
-    // heads captured now, clamped cells, the new cell, and every cell once per 2^20 events
-    ++nev;
-    const bool all = nev >= (1 << 20);
-    if (all) nev = 0;
-    bool any = false;
-#pragma unroll
-    for (int k = 0; k < K; ++k) any |= (tgt1[k] >= 0) & ((tgt1[k] == i1) | (lo[k] == -fInf) | all);
-    if (__ballot(any) != 0) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const bool hit = tgt1[k] >= 0 && (tgt1[k] == i1 || lo[k] == -fInf || all);
-        if (!hit) continue;
-        const int s = mo + k * NO;
-        if (tgt1[k] == i1) {
-          const int pos = HC ? (c1[k] & 31) : c1[k] - s * AMCD_NB;
-          PHASE_FLAG(aflag, (PF && k == ks) ? 8 : 1);
-          const SlotHead h = (PF && k == ks) ? slot_head_pre(d, dead, s, pos + 1, i1, pb)
-                                             : slot_head(d, dead, s, pos + 1, i1);
-          tgt1[k] = h.tgt1;
-          if constexpr (HC) {
-            c1[k] = (h.c1 - s * AMCD_NB) | ((((c1[k] >> 5) & ~31) + h.k1) << 5);
-            hc[s] = h.D1;
-            hc[HN + s] = h.Dn;
-            if constexpr (HR) hc[2 * HN + s] = h.r1;
-          } else {
-            c1[k] = h.c1;
-          }
-          lo[k] = hi[k] = fInf;
-          if (h.tgt1 >= 0) tau_bounds(h.D1, E[k], V[k], T, lo[k], hi[k]);
-        } else {
-          PHASE_FLAG(aflag, 16);
-          tau_bounds(HC ? hc[s] : gmem(d.cD)[c1[k]], E[k], V[k], T, lo[k], hi[k]);
-        }
-      }
-    }
-    skip = i1;
-    par ^= 1;
-    PHASE(ot, 6, tid == 64);
-  }
-  // half-diagonals back to the growing list (the cell still in the mailbox is current there)
-  if (loaded) {
-    const int ns = sh.nslots;
-    const NewCell& nc = sh.mb[par];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int s = me + k * NO;
-      if (s < ns && !(nc.valid && nc.slot == s)) gmem(d.gExt)[s] = E[k];
-    }
-  }
-  visits_out += visits;
-  evals_out += evals;
+// An event for BUILD to start on: one 8-byte store (a wave's LDS stores are performed in order, so
+// what was stored before it is there when it is seen).
+__device__ static inline void publish(Window& win, int m, int ent, int i1) {
+  asm volatile("" ::: "memory");
+  *(volatile unsigned long long*)&win.ev[m] = ((unsigned long long)(unsigned)i1 << 32) | (unsigned)ent;
 }
 
-// The owner protocol of owner_loop for growing lists larger than the register tiers hold:
-// each cell's state (E in gExt, V in gVhat, bounds in gLH, head in gHd) stays in global
-// memory and every event streams the lane's cells (slots me, me + NO, ...).  Same
-// decisions, same arithmetic, same order of additions as the register tiers.
-template <int NT>
-__device__ static __attribute__((always_inline)) void owner_loop_mem(const Inst& d_lds, EngineShared& sh,
-                                                                      const unsigned* dead, int go, double T,
-                                                                      long long& visits_out, long long& evals_out) {
-  const Inst d = d_lds;  // in registers, as in owner_loop
-  long long visits = 0, evals = 0;
-  constexpr int NO = NT - 64;
-  constexpr int NW = NT / 64;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int me = tid - 64;
-  const float fInf = __builtin_inff();
-  const amcd_params& p = d.p;
-  // loop constants held in registers (a read through the descriptor in LDS would be
-  // repeated after every barrier)
-  const double DelT = p.DelT, rX = p.rX;
-  int ns = go != -2 ? sh.nslots : 0;  // slots this lane knows of (new ones arrive by mailbox)
-  // The lane's smallest upper bound and its two smallest lower bounds (with their slots)
-  // and third smallest lower bound, gathered whenever every cell's bounds pass through the
-  // lane (set-up, and the growth pass of each event): the next evaluation needs no pass
-  // over the cells unless a third cell reaches the wave's smallest upper bound.
-  float hmin = fInf, l0 = fInf, l1 = fInf, l2 = fInf;
-  int f0 = -1, f1 = -1;
-  auto note = [&](int s, float2 lh) {
-    hmin = fminf(hmin, lh.y);
-    if (lh.x < l0) {
-      l2 = l1;
-      l1 = l0;
-      f1 = f0;
-      l0 = lh.x;
-      f0 = s;
-    } else if (lh.x < l1) {
-      l2 = l1;
-      l1 = lh.x;
-      f1 = s;
-    } else if (lh.x < l2) {
-      l2 = lh.x;
+// ENGINE: the events of window `win`, by one wave.  The entries are sorted by their upper
+// bounds once per window (the first to come in the highest lane), so an event takes the first
+// live lane without a search; only where a later entry's lower bound reaches it (they are equal
+// up to rounding) are the exact times compared.  Every value that steers the loop is made uniform
+// on entry (scalar branches, no loads).  The time is the quotient (D - E)/V rounded to nearest,
+// from V's reciprocal rounded to nearest and two residual corrections (Markstein's theorem: the
+// first makes the quotient faithful, the second correctly rounded); where a residual could leave
+// the normal range, by a division.
+struct EngineState {
+  double T;
+  int vSind2, nGrain, pool_used, events, captures, nucs;
+  int nd;  // draws consumed
+  int visits;
+};
+struct EngineRun {
+  double T, rdt;
+  int m, used, visits, fin, ri1, rent;
+  bool nuc;
+};
+template <bool PLAIN>
+__device__ static inline void engine_run(EngineRun& o, Window& win, double D, double E, double V, double y, double r,
+                                         int tgt, int key, int src, int parent, int lo, int hi, int lim_,
+                                         unsigned long long live, unsigned long long close, unsigned long long draws, int W, int mmax,
+                                         double DelT, int scan0) {
+  const int lane = threadIdx.x & 63;
+  double T = o.T, rdt = 0.0;
+  int m = 0, ri1 = -1, rent = -2, used = 0, visits = 0, fin = 1, lim = W;
+  bool nuc = false;
+  unsigned long long killed = 0;
+  double Vg = parent < 0 ? V : 0.0;  // a cell grows from the event that creates it on
+  while (live != 0) {
+    int wl = 63 - __builtin_clzll(live);
+    const int u = __builtin_amdgcn_readlane(hi, wl);
+    if (u > lim) break;
+    if (!(T < DelT)) {  // loop condition (S/VoxelsCA.C:381)
+      fin = 0;
+      break;
     }
+    const double a = D - E;
+    double t;
+    if constexpr (PLAIN) {
+      double q = a * y;
+      q = fma(fma(-V, q, a), y, q);
+      t = fma(fma(-V, q, a), y, q);
+    } else {
+      t = a / V;
+    }
+    ++visits;
+    if ((close >> wl) & 1ull) {
+      // several within rounding: the smallest time, then (ruqs, key) among the equal ones
+      const unsigned long long c = __ballot(lo <= u) & live;
+      visits += __popcll(c) - 1;
+      const bool ok = ((c >> lane) & 1ull) && t <= 1e6;
+      const double tmin = wave_min_f64(ok ? t : __builtin_inf());
+      unsigned long long at = __ballot(ok && t == tmin);
+      if (at == 0) {
+        if (m == 0) fin = 0;
+        break;
+      }
+      wl = __builtin_ctzll(at);
+      at &= at - 1;
+      if (at != 0) {
+        double rb = lane_f64(r, wl);
+        int kb = __builtin_amdgcn_readlane(key, wl);
+        for (; at != 0; at &= at - 1) {
+          const int l = __builtin_ctzll(at);
+          const double rl = lane_f64(r, l);
+          const int kl = __builtin_amdgcn_readlane(key, l);
+          const bool first = rl < rb || (!(rl > rb) && kl < kb);
+          wl = first ? l : wl;
+          rb = first ? rl : rb;
+          kb = first ? kl : kb;
+        }
+      }
+    }
+    const double tw = lane_f64(t, wl);
+    const int th = (int)(__double_as_longlong(tw) >> 32);
+    if (th >= 0x412e8480) {  // 1e6 or more, or not a number (S/VoxelsCA.C:480)
+      fin = 0;
+      break;
+    }
+    const int i1 = __builtin_amdgcn_readlane(tgt, wl), ent = __builtin_amdgcn_readlane(src, wl);
+    const bool me = lane == m;
+    ri1 = me ? i1 : ri1;
+    used = m + 1;
+    nuc = (draws >> m) & 1ull;
+    if (nuc) break;
+    // capture: growth of every cell (S/VoxelsCA.C:511-516); the lanes' cells all have a live
+    // candidate.  A step back in time (negative Dt) ends the window, since it may clamp a
+    // half-diagonal at zero and so move a capture time.
+    rent = me ? ent : rent;
+    *(volatile unsigned long long*)&win.ev[lane] = ((unsigned long long)(unsigned)ri1 << 32) | (unsigned)rent;
+    T = T + tw;
+    E = E + Vg * tw;
+    rdt = me ? tw : rdt;
+    killed |= __ballot(tgt == i1);
+    const unsigned long long kids = __ballot(parent == ent);
+    if (kids != 0) {  // candidates of the cell that this event creates
+      live |= kids;
+      const bool mine = parent == ent;
+      Vg = mine ? V : Vg;
+      key = mine ? (scan0 + m) * 32 + key : key;
+    }
+    live &= ~killed;
+    lim = min(lim, __builtin_amdgcn_readlane(lim_, wl));
+    lim = th < 0 ? (int)0x80000000 : lim;
+    ++m;
+    if (m >= mmax) break;
+  }
+  o.T = T;
+  o.rdt = rdt;
+  o.m = m;
+  o.used = used;
+  o.visits = visits;
+  o.fin = fin;
+  o.ri1 = ri1;
+  o.rent = rent;
+  o.nuc = nuc;
+}
+__device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& win, EngineState& es, float W, int mmax,
+                                            double DelT_, int n_pool, LoopState* ls) {
+  const int lane = threadIdx.x & 63;
+  const int n = uni(win.n);
+  // sorted by the upper bounds, the first to come in the highest lane
+  const int src = __builtin_amdgcn_ds_permute((63 - (lane < n ? win.rank[lane] : lane)) << 2, lane);
+  const bool in = lane >= 64 - n;
+  const double D = in ? win.D[src] : 0.0, V = in ? win.V[src] : 1.0, r = in ? win.r[src] : 0.0;
+  const double E = in ? win.E[src] : 0.0, y = in ? win.y[src] : 1.0;
+  const int tgt = in ? win.tgt[src] : -1, key = in ? win.key[src] : 0;
+  const int lo = in ? win.lo[src] : kKeyNone, hi = in ? win.hi[src] : kKeyNone, lim = in ? win.lim[src] : kKeyNone;
+  const int parent = in ? win.parent[src] : -1;
+  const bool plain = __all(!in || (V > 0x1p-300 && V < 0x1p300 && D > 0x1p-300 && D < 0x1p300 && fabs(E) < 0x1p300));
+  // entries that a later one's lower bound reaches: the smallest lower bound over the lower lanes
+  int sm = dpp_min_shift<0x111>(lo);  // row_shr:1, :2, :4, :8, then the rows below
+  sm = dpp_min_shift<0x112>(sm);
+  sm = dpp_min_shift<0x114>(sm);
+  sm = dpp_min_shift<0x118>(sm);
+  sm = dpp_min_shift<kBcast15, 0xa>(sm);
+  sm = dpp_min_shift<kBcast31, 0xc>(sm);
+  sm = __builtin_amdgcn_update_dpp(0x7fffffff, sm, 0x138, 0xf, 0xf, false);  // wave_shr:1
+  const unsigned long long close = __ballot(sm <= hi), live = __ballot(in && parent < 0);
+  const unsigned dlo = uni((int)win.draws), dhi = uni((int)(win.draws >> 32));
+  const unsigned long long draws = ((unsigned long long)dhi << 32) | dlo;
+  const double DelT = uni(DelT_);
+  EngineRun o;
+  o.T = uni(es.T);
+  const int Wk = uni(order_key(W));
+  mmax = uni(mmax);
+  if (plain)
+    engine_run<true>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
+                      uni(es.vSind2));
+  else
+    engine_run<false>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
+                      uni(es.vSind2));
+  int fin = n == 0 ? 0 : o.fin, m = o.m;  // n == 0: no candidate left
+  es.captures += m;
+  if (fin == 1 && o.nuc) {  // S/VoxelsCA.C:483-506
+    const int i1 = __builtin_amdgcn_readlane(o.ri1, m);
+    if (es.pool_used >= n_pool || es.pool_used >= d.poolcap || es.nGrain >= d.gcap) {
+      if (lane == 0) {
+        *gmem(&ls->pending) = 1;  // the host refills the pool and resumes
+        *gmem(&ls->pend_tgt) = i1;
+      }
+      fin = -1;
+    } else {
+      // (the nucleus's first capture is not bounded: the window ends)
+      es.nGrain++;
+      if (lane == 0) {
+        win.G = es.nGrain;
+        win.pool = es.pool_used;
+        publish(win, m, -1, i1);
+      }
+      es.pool_used++;
+      es.nucs++;
+      ++m;
+    }
+  }
+  if (lane == 0) *(volatile int*)&win.done = 1;
+  if (lane < m) {
+    win.dt[lane] = o.rdt;
+    gmem(d.aScan)[o.ri1] = es.vSind2 + lane;
+  }
+  es.events += o.used;
+  es.nd += o.used;
+  es.visits += o.visits;
+  es.T = o.T;
+  if (lane == 0) {
+    if (o.used > 0) sh.cur = win.x2[o.used - 1];
+    win.m = m;
+    win.decided = o.used;
+    sh.T = o.T;
+    sh.fin = fin;
+  }
+  es.vSind2 += m;
+}
+
+// The rare parts of BUILD out of line, so that their registers do not add to the cells' own: the
+// re-centring of a capture by a cell made in this launch, a velocity that is not tabulated (EASM
+// temperatures).
+struct Octahedron {
+  double x, y, z, E;
+};
+__device__ __attribute__((noinline)) static Octahedron recentre_out(const Inst* I, int sw, int cand, int v1) {
+  CInst& d = *(CInst*)I;
+  const auto q = gmem(d.slots) + sw;
+  const double c[3] = {q->c[0], q->c[1], q->c[2]};
+  const int G = q->G;
+  double R[9], o[3], e;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) R[q] = gmem(d.rot)[9 * (size_t)(G - 1) + q];
+  recentre(d, q->vox, v1, c, R, gmem(d.cF)[cand], o, &e);
+  return {o[0], o[1], o[2], e};
+}
+__device__ __attribute__((noinline)) static double velocity_out(const Inst* I, double T) {
+  CInst& d = *(CInst*)I;
+  return growth_velocity(d.p, T);
+}
+
+// The sorted list of a cell that no set-up list was built ahead for (a nucleus, or a capture by a
+// cell of this launch), out of line as the other rare parts.
+__device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb, int i1, int G, int v1, int tn, int liq,
+                                                          double c0, double c1, double c2) {
+  CInst& d = *(CInst*)I;
+  auto& p = d.p;
+  const int lane = threadIdx.x & 63;
+  double R[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) R[q] = gmem(d.rot)[9 * (size_t)(G - 1) + q];
+  double D = __builtin_inf(), f = 0, r = __builtin_inf();
+  // neighbour `lane` of v1, in the order of the active-neighbour table
+  int vi, vj, vk;
+  decode(d, v1, vi, vj, vk);
+  const int qq = lane < 13 ? lane : lane + 1;
+  const int ddx = qq % 3 - 1, ddy = (qq / 3) % 3 - 1, ddz = qq / 9 - 1;
+  if (liq) {
+    const double cen[3] = {c0, c1, c2};
+    const double ct[3] = {((double)(vi + ddx) + .5) * p.dx, ((double)(vj + ddy) + .5) * p.dy,
+                          ((double)(vk + ddz) + .5) * p.dz};
+    candidate_at(ct, cen, R, &D, &f);
+    r = .5 * (gmem(d.ruq)[i1] + gmem(d.ruq)[tn]);
+  }
+  const int rank = list_rank(D, r, liq != 0, -1), n = (int)__popcll(__ballot(liq != 0));
+  if (liq) {
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    const auto q = gmem((v2d*)(d.cand + cb + rank));
+    q[0] = v2d{D, r};
+    q[1] = v2d{pack2(tn, lane), pack2(__float_as_int(-__builtin_inff()), n - rank)};
+    gmem(d.cF)[cb + rank] = f;
+  }
+}
+
+// BUILD: the cell that event k of the window creates (one wave, while the engine goes on).  The
+// liveness is that of the window's start; the voxels of the events up to k are known.  One round
+// of loads: the captured cell's row by lanes 0..31, the entry's capture by lanes 32..43.
+template <bool GD>
+__device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh, Window& win, const Liveness<GD>& live,
+                                         int ent, int k, int ns_pre, int nm0) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63;
+  auto& p = d.p;
+  const int evi = lane <= k ? ((volatile int2*)win.ev)[lane].y : -1;  // lane j: voxel of event j
+  const int i1 = __builtin_amdgcn_readlane(evi, k), scan = uni(win.scan0) + k;
+  const int cand = ent >= 0 ? uni(win.cand[ent]) : -1, sw = ent >= 0 ? uni(win.own[ent]) : -1;
+  // an entry of a list the set-up built (the cells' own, and those ahead)
+  const bool first = cand >= 0 && (cand < ns_pre * AMCD_NB || cand >= d.acap * AMCD_NB);
+  const int* at = (const int*)(d.aRow + i1) + (lane & 31);
+  if (lane >= 32) at = first ? (const int*)(d.cap + cand) + min(lane - 32, 11) : at;
+  const int x = gmem(at)[0];
+  const int tn = lane < AMCD_NB ? x : -1;
+  bool liq = tn >= 0 && !live.dead(tn >= 0 ? tn : 0);
+  for (int j = 0; j < k; ++j) liq &= tn != __builtin_amdgcn_readlane(evi, j);
+  const unsigned long long bal = __ballot(liq);  // liquid just after the event
+  const int v1 = __builtin_amdgcn_readlane(x, 26), cold = __builtin_amdgcn_readlane(x, 27);
+  auto word2 = [&](int l) {
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane(x, l + 1) << 32) |
+                                            (unsigned)__builtin_amdgcn_readlane(x, l)));
   };
-  for (int s = me; s < ns; s += NO) {
-    const SlotHead h = slot_head(d, dead, s, 0, -1);
-    float lo = fInf, hi = fInf;
-    if (h.tgt1 >= 0) tau_bounds(h.D1, gmem(d.gExt)[s], gmem(d.gVhat)[s], T, lo, hi);
-    gstore8(d.gHd + s, make_int2(h.c1, h.tgt1));
-    gstore8(d.gLH + s, make_float2(lo, hi));
-    note(s, make_float2(lo, hi));
+  const double T1 = word2(28);
+  double cen[3], E0;
+  int G, pre = -1;
+  if (first) {            // capture (S/VoxelsCA.C:507-605)
+    cen[0] = word2(32);
+    cen[1] = word2(34);
+    cen[2] = word2(36);
+    E0 = word2(38);
+    pre = __builtin_amdgcn_readlane(x, 40);
+    G = __builtin_amdgcn_readlane(x, 41);
+  } else if (ent >= 0) {  // by a cell made in this launch
+    G = uni(gmem(d.slots)[sw].G);
+    const Octahedron o = recentre_out(I, sw, cand, v1);
+    cen[0] = uni(o.x);
+    cen[1] = uni(o.y);
+    cen[2] = uni(o.z);
+    E0 = uni(o.E);
+  } else {                // nucleation (S/VoxelsCA.C:486-506)
+    G = uni(win.G);
+    centre(d, v1, cen);
+    E0 = 0.0;
+    if (lane < 9) gmem(d.rot)[9 * (size_t)(G - 1) + lane] = gmem(d.pool)[9 * (size_t)uni(win.pool) + lane];
   }
-  int skip = -1;
-  int par = 0;
-  int nd = 0;
-  int nev = 0;
-  Decision x;
-  x.stop = 0;
-  x.nuc = 1;
-  x.i1 = sh.r_i1;
-  x.dt = 0.0;
-  bool apply_first = go == 2;
-  // the lane's cells are streamed MB at a time: all loads of a batch are issued before
-  // any of them is used
-  constexpr int MB = 8;
-  while (go > 0) {
-    if (!apply_first) {
-      // ---- EVAL: the wave's smallest upper bound, then the cells whose lower bound reaches it
-      const float u = wave_min(hmin);
-      Best b = best_none();
-      auto evaluate = [&](int s) {  // exact capture time of slot s's head (S/VoxelsCA.C:420-440)
-        const int2 hd = gload8(d.gHd + s);
-        const int c = hd.x;
-        const int pos = c - s * AMCD_NB;
-        const double e = gmem(d.gExt)[s], v = gmem(d.gVhat)[s];
-        const double D1 = gmem(d.cD)[c];
-        const double Dn = (pos + 1 < AMCD_NB) ? gmem(d.cD)[c + 1] : __builtin_inf();
-        const double rr = gmem(d.cR)[c];
-        const int kb = gmem(d.gScan)[s] * 32;
-        const int kk = gmem(d.cK)[c];
-        visits++;
-        evals++;
-        const double t1 = (D1 - e) / v;
-        if (t1 <= 1e6) {
-          Best y;
-          y.t = t1;
-          y.r = rr;
-          y.key = kb + kk;
-          y.cand = c;
-          y.tgt = hd.y;
-          if ((Dn - e) / v == t1) {
-            const int n = gmem(d.gN)[s];
-            for (int q = pos + 1; q < n; ++q) {
-              const int tq = gmem(d.cTgt)[c - pos + q];
-              if (!live_target(dead, tq, skip)) continue;
-              evals++;
-              const double tt = (gmem(d.cD)[c - pos + q] - e) / v;
-              if (!(tt == t1)) break;
-              Best z;
-              z.t = tt;
-              z.r = gmem(d.cR)[c - pos + q];
-              z.key = kb + gmem(d.cK)[c - pos + q];
-              z.cand = c - pos + q;
-              z.tgt = tq;
-              if (better(z, y)) y = z;
-            }
-          }
-          if (better(y, b)) b = y;
-        }
-      };
-      if (l2 <= u) {  // a third cell may reach u: every cell of the lane, MB at a time
-        for (int s0 = me; s0 < ns; s0 += MB * NO) {
-          float lob[MB];
-#pragma unroll
-          for (int q = 0; q < MB; ++q) {
-            const int s = s0 + q * NO;
-            lob[q] = s < ns ? gload8(d.gLH + s).x : fInf;
-          }
-#pragma unroll
-          for (int q = 0; q < MB; ++q)
-            if (lob[q] != fInf && lob[q] <= u) evaluate(s0 + q * NO);
-        }
-      } else {
-        if (f0 >= 0 && l0 != fInf && l0 <= u) evaluate(f0);
-        if (f1 >= 0 && l1 != fInf && l1 <= u) evaluate(f1);
-      }
-      b = wave_best(b);
-      if (lane == 0) sh.sb[par][w] = b;
-      __syncthreads();
-      x = decide<NW>(sh, par, T, DelT, rX, nd);
-      if (x.stop) break;
-      ++nd;
+  int slot = -1, cb = 0;
+  const bool grows = cold && bal;
+  if (grows) {
+    if (lane == 0) slot = atomicAdd(&sh.nslots, 1);
+    slot = uni(slot);
+    cb = pre >= 0 ? pre : slot * AMCD_NB;
+    if (pre < 0) {
+      if (ent < 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the nucleus's rotation, read back
+      list_out(I, cb, i1, G, v1, tn, liq, cen[0], cen[1], cen[2]);
     }
-    apply_first = false;
-    // ---- APPLY
-    const double Dt = x.dt;
-    const int i1 = x.i1;
-    // the cell created by the previous event joins its owner's slots ungrown; the pass
-    // below grows it like every other cell and computes its bounds
-    const NewCell& nc = sh.mb[par];
-    if (nc.valid && nc.slot % NO == me) {
-      gmem(d.gExt)[nc.slot] = nc.E;
-      gmem(d.gVhat)[nc.slot] = nc.V;
-      gstore8(d.gHd + nc.slot, make_int2(nc.c1, nc.tgt1));
-      gstore8(d.gLH + nc.slot, make_float2(-fInf, fInf));
+    const double V0 = (T1 == p.tS) & (T1 < p.tL) ? p.vhat_tS : velocity_out(I, T1);
+    if (lane == 0) {
+      win.base[k] = cb;
+      win.E0[k] = E0;
+      win.V0[k] = V0;
     }
-    if (nc.valid) ns = max(ns, nc.slot + 1);
-    T = T + Dt;
-    ++nev;
-    const bool all = nev >= (1 << 20);
-    if (all) nev = 0;
-    hmin = l0 = l1 = l2 = fInf;
-    f0 = f1 = -1;
-    for (int s0 = me; s0 < ns; s0 += MB * NO) {
-      int2 hdb[MB];
-      float2 lhb[MB];
-      double eb[MB], vb[MB];
-#pragma unroll
-      for (int q = 0; q < MB; ++q) {
-        const int s = s0 + q * NO;
-        const bool in = s < ns;
-        hdb[q] = in ? gload8(d.gHd + s) : make_int2(0, -1);
-        lhb[q] = in ? gload8(d.gLH + s) : make_float2(fInf, fInf);
-        eb[q] = in ? gmem(d.gExt)[s] : 0.0;
-        vb[q] = in ? gmem(d.gVhat)[s] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < MB; ++q) {
-        const int s = s0 + q * NO;
-        int2 hd = hdb[q];
-        if (hd.y < 0) continue;
-        float2 lh = lhb[q];
-        double e = eb[q];
-        const double v = vb[q];
-        if (!x.nuc) {  // growth (S/VoxelsCA.C:511-516)
-          const double g = e + v * Dt;
-          if (g < 0.0) {
-            e = 0.0;
-            lh.x = -fInf;
-          } else {
-            e = g;
-          }
-          gmem(d.gExt)[s] = e;
-        }
-        if (hd.y == i1) {
-          const SlotHead h = slot_head(d, dead, s, hd.x - s * AMCD_NB + 1, i1);
-          hd = make_int2(h.c1, h.tgt1);
-          lh = make_float2(fInf, fInf);
-          if (h.tgt1 >= 0) tau_bounds(h.D1, e, v, T, lh.x, lh.y);
-          gstore8(d.gHd + s, hd);
-          gstore8(d.gLH + s, lh);
-        } else if (lh.x == -fInf || all) {
-          tau_bounds(gmem(d.cD)[hd.x], e, v, T, lh.x, lh.y);
-          gstore8(d.gLH + s, lh);
-        }
-        note(s, lh);
-      }
-    }
-    skip = i1;
-    par ^= 1;
   }
-  visits_out += visits;
-  evals_out += evals;
+  if (lane == 0) win.slot[k] = slot;
+  // the slot's record by lanes 0..2 and the event's by lanes 3..5, 16 bytes each
+  const int q = lane < 3 ? lane : lane - 3;
+  const double c02 = q == 0 ? cen[0] : cen[2];
+  const double a = lane < 3 ? (q == 2 ? pack2(i1, scan) : c02) : (q == 0 ? pack2(i1, G) : q == 1 ? cen[0] : cen[2]);
+  const double b = lane < 3 ? (q == 0 ? cen[1] : q == 1 ? pack2(v1, G) : pack2(cb, 1))
+                            : (q == 0 ? E0 : q == 1 ? cen[1] : 0.0);
+  if (lane < 6 && (lane >= 3 || grows)) {
+    v2d* to = lane < 3 ? (v2d*)(d.slots + slot) + q : (v2d*)(d.events + (scan - nm0)) + q;
+    gmem(to)[0] = v2d{a, b};
+  }
+}
+// BUILD for a wave's share of a window's events, as the engine publishes them (or all of them,
+// when it is done); out of line: its registers do not add to those that hold the cells.  The
+// engine ends after at most WCAP events whatever these waves do, so the wait ends.
+template <bool GD>
+__device__ __attribute__((noinline)) static void build_cells(const Inst* I, int first, int step, int ns_pre, int nm0) {
+  CInst& d = *(CInst*)I;
+  Window& win = s_loop.win;
+  const Liveness<GD> live = {s_dead_bits, d.aVS};
+  for (int k = first; k < WCAP; k += step) {
+    int ent;
+    for (;;) {
+      const int done = uni(*(volatile int*)&win.done);
+      ent = uni(((volatile int2*)win.ev)[k].x);  // (read after `done`: a set flag means all is published)
+      if (ent != -2 || done) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    if (ent == -2) break;
+    build_cell<GD>(d, I, s_loop, win, live, ent, k, ns_pre, nm0);
+  }
 }
 
-// GD: the liveness bitmap lives in memory (d.gdead) instead of LDS, for interfaces of more
-// than AMCD_DEAD_BITS cells (instantiated with the memory-resident tier only).
+// A cell whose last candidate died in this window grows through the event that took it: the
+// largest event of its targets from the former head on (those before it died in earlier windows).
+__device__ static inline int last_event(CInst& d, int from, int scan0) {
+  int mx = -1;
+  for (int p = from;; p += 4) {
+    CandRec e[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) e[q] = load_rec(d.cand + p + q);
+    const int n = e[0].n;
+    int sc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sc[q] = gmem(d.aScan)[q < n ? e[q].tgt : e[0].tgt] - scan0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) mx = max(mx, sc[q]);
+    if (n <= 4) break;
+  }
+  return mx;
+}
+
+// One cell after a window: its head moves from entry c0 to the next live candidate; bounds for it.  e is the
+// half-diagonal before the window's growth (of a cell that event k0 created: after that event);
+// `grown` returns it with the window's growth, through the event that took the last candidate
+// when there is none left.  dtl: lane j holds the growth time of event j (whole waves call this).
+struct Refreshed {
+  double grown;
+  float lo, hi;
+  int c1, tgt;
+};
+template <bool GD>
+__device__ static inline Refreshed refresh_cell(CInst& d, const Liveness<GD>& live, bool on, int c0, double e, double v,
+                                                int k0, int m, int scan0, double dtl, double T0, double T) {
+  Refreshed o;
+  o.lo = o.hi = __builtin_inff();
+  o.c1 = 0;
+  o.tgt = -1;
+  o.grown = e;
+  double D1 = 0.0;
+  int last = -1;
+  if (on) {
+    const SlotHead h = slot_head<GD>(d, live, c0);
+    o.c1 = h.c1;
+    o.tgt = h.tgt1;
+    D1 = h.D1;
+    last = h.tgt1 >= 0 ? m - 1 : last_event(d, c0, scan0);
+  }
+  if (__any(on && (k0 >= 0 || o.tgt < 0))) {
+    for (int j = 0; j < m; ++j) {
+      const double g = o.grown + v * lane_f64(dtl, j);
+      o.grown = (j > k0) & (j <= last) ? g : o.grown;
+    }
+    if (o.grown < 0.0) o.grown = 0.0;  // (only a window's last event can step back)
+  }
+  // tau is the same before and after the growth; a new cell's is taken after it
+  if (o.tgt >= 0) tau_bounds(D1, k0 >= 0 ? o.grown : e, v, k0 >= 0 ? T : T0, o.lo, o.hi);
+  return o;
+}
+
+// A cell's entries up to clock W into the window: its head, and the live candidates after it
+// while their bounds reach W (two list positions per round of loads; the one past the list's end
+// is masked).
+__device__ static inline int put_entry(Window& win, const CandRec& e, double E, double V, int key, int cand, int own,
+                                       int parent, int lo, int hi) {
+  const int i = atomicAdd(&win.n, 1);
+  if (i >= WCAP) return -1;
+  win.D[i] = e.D;
+  win.E[i] = E;
+  win.V[i] = V;
+  win.r[i] = e.r;
+  win.tgt[i] = e.tgt;
+  win.key[i] = key;
+  win.cand[i] = cand;
+  win.own[i] = own;
+  win.parent[i] = parent;
+  win.lo[i] = lo;
+  win.hi[i] = hi;
+  return i;
+}
+template <bool GD>
+__device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Window& win, int s, double E, double V,
+                                        int c1, float lo, float hi, double T, float W, int ns_pre) {
+  const int scan = gmem(d.slots)[s].scan;
+  bool first = true;
+  for (int p = c1;; p += 2) {
+    CandRec e[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) e[q] = load_rec(d.cand + p + q);
+    const int n = e[0].n;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (q >= n) return;
+      if (!first) {
+        tau_bounds(e[q].D, E, V, T, lo, hi);
+        if (!(lo <= W) || lo == __builtin_inff()) return;  // and so are all later ones
+        if (live.dead(e[q].tgt)) continue;
+      }
+      first = false;
+      const int i = put_entry(win, e[q], E, V, scan * 32 + e[q].nb, p + q, s, -1, order_key(lo), order_key(hi));
+      if (i < 0) return;
+      // the clock after the capture is at least lo: when the new cell may capture within the
+      // window, its candidates join it
+      const float tn = e[q].tn;
+      const float x = lo + tn - 0x1p-20f * (fabsf(lo) + fabsf(tn));
+      int lim = tn == -__builtin_inff() ? (int)0x80000000 : tn == __builtin_inff() ? kKeyNone : order_key(x) - 2;
+      if (lim < order_key(W) && (p + q < ns_pre * AMCD_NB)) {
+        const CapRec cr = d.cap[p + q];
+        if (cr.pre >= 0) {
+          lim = kKeyNone;
+          for (int pc = cr.pre;; ++pc) {
+            const CandRec ec = load_rec(d.cand + pc);
+            float l, h;
+            tau_bounds(ec.D, cr.E, cr.V, 0.0, l, h);
+            const int lk = order_key(lo + l) - 1, hk = order_key(hi + h) + 1;
+            if (l == __builtin_inff() || lk > order_key(W)) break;
+            if (l == -__builtin_inff()) {  // (no bound: the window ends with the capture)
+              lim = (int)0x80000000;
+              break;
+            }
+            if (!live.dead(ec.tgt)) {
+              const int ic = put_entry(win, ec, cr.E, cr.V, ec.nb, pc, -1, i, lk, hk);
+              if (ic < 0) return;
+              const float xc = lo + l + ec.tn - 0x1p-20f * (fabsf(lo) + fabsf(l) + fabsf(ec.tn));
+              win.lim[ic] = ec.tn == -__builtin_inff() ? (int)0x80000000
+                                                       : ec.tn == __builtin_inff() ? kKeyNone : order_key(xc) - 2;
+            }
+            if (ec.n <= 1) break;
+          }
+        }
+      }
+      win.lim[i] = lim;
+    }
+    if (n <= 2) return;
+  }
+}
+
+// The exact best candidate of one cell (its head and the entries tied with it in time) against
+// b (S/VoxelsCA.C:420-440).
+template <bool GD>
+__device__ static inline void exact_cell(CInst& d, const Liveness<GD>& live, int s, double E, double V, int c1, Best& b,
+                                         int& bs, double& be, double& bv) {
+  const int scan = gmem(d.slots)[s].scan;
+  double t1 = 0.0;
+  for (int p = c1;; ++p) {
+    const CandRec e = load_rec(d.cand + p);
+    const double t = (e.D - E) / V;
+    if (p == c1) {
+      t1 = t;
+      if (!(t1 <= 1e6)) break;
+    }
+    if (!(t == t1)) break;
+    Best z;
+    z.t = t;
+    z.r = e.r;
+    z.key = scan * 32 + e.nb;
+    z.cand = p;
+    z.tgt = e.tgt;
+    if (!live.dead(e.tgt) && better(z, b)) {
+      b = z;
+      bs = s;
+      be = E;
+      bv = V;
+    }
+    if (e.n <= 1) break;
+  }
+}
+
+// GD: an interface of more than AMCD_DEAD_BITS cells, whose liveness is read from the states
+// (instantiated with the memory-resident tier only).  K = 0: every cell's state in memory
+// (gExt, gVhat, gHd, gLH), streamed MB cells per thread at a time, for growing lists larger
+// than the register tiers hold.
 template <int NT, int K, bool GD = false>
 __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, amcd_out* O) {
   constexpr int NW = NT / 64;
-  // slots this tier holds: K per owner thread in registers, or (K = 0) every slot of the
-  // domain's arrays in memory
-  const int CAP = K > 0 ? (NT - 64) * K : I[blockIdx.x].acap;
-  __shared__ EngineShared sh;
-  __shared__ int s_go;
-  constexpr int DB = DeadBits<K, GD>::n;
-  __shared__ unsigned s_dead[DB / 32];
-  __shared__ double s_hc[HeadCache<K>::on ? HeadCache<K>::words * (NT - 64) * K : 1];
-  // The descriptor and step record are copied to LDS: every event ends in a barrier, after
-  // which the compiler must re-read anything in global memory, and each array access would
-  // otherwise wait for its base pointer to come back from global memory first.
-  __shared__ Inst s_inst;
-  __shared__ amcd_step s_step;
+  constexpr bool MEM = K == 0;                  // half-diagonals and velocities in memory
+  constexpr bool HM = MEM || NT * K > LDS_CELLS;  // bounds and heads in memory
+  constexpr int KR = MEM ? 4 : K;  // cells a thread holds in registers at a time
+  // slots this tier holds: K per thread in registers, or every slot of the domain's arrays
+  const int CAP = MEM ? I[blockIdx.x].acap : NT * K;
+  LoopShared& sh = s_loop;
   if (I[blockIdx.x].ls->done) return;
-  if (threadIdx.x == 0) {
-    s_inst = I[blockIdx.x];
-    s_step = S[blockIdx.x];
-  }
-  __syncthreads();
-  const Inst& d = s_inst;
+  // The descriptor through the constant address space (no launch writes it while it is read): its
+  // fields are scalar loads that no store can alias, so the compiler keeps or repeats them as its
+  // registers allow; as a copy they spilled 420 scalar registers.
+  CInst& d = *(CInst*)(I + blockIdx.x);
   LoopState* ls = d.ls;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const amcd_params& p = d.p;
-  // loop constants held in registers (a read through the descriptor in LDS would be
-  // repeated after every barrier)
-  const double DelT = p.DelT, rX = p.rX;
-  const amcd_step& st = s_step;
+  const float fInf = __builtin_inff();
+  const double DelT = d.p.DelT, rX = d.p.rX;
+  const int n_pool = S[blockIdx.x].n_pool;
   const int Na = ls->Na;
-  unsigned* const dead = GD ? d.gdead : s_dead;
-  if (GD || Na <= DB) {  // liveness bitmap from the current states
+  const int ns_first = ls->nslots;
+  const int ns_pre = ls->nslots_pre < 0 ? ns_first : ls->nslots_pre;  // slots the set-up made
+  const Liveness<GD> live = {s_dead_bits, d.aVS};
+  if (!GD && Na <= AMCD_DEAD_BITS) {  // liveness bitmap from the current states
     for (int wd = tid; wd < (Na + 31) / 32; wd += NT) {
-      unsigned m = 0;
-      for (int q = 0; q < 32; ++q) {
-        const int a = 32 * wd + q;
-        if (a >= Na || d.aVS[a] != 1) m |= 1u << q;
+      typedef unsigned v4u __attribute__((ext_vector_type(4)));
+      const auto q = gmem((const v4u*)(d.aVS + 32 * (size_t)wd));  // (256 bytes are allocated beyond the end)
+      const v4u x = q[0], y = q[1];
+      unsigned b = 0;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        const unsigned v = j < 16 ? x[j / 4] : y[(j - 16) / 4];
+        b |= (((v >> (8 * (j & 3))) & 0xffu) != 1u ? 1u : 0u) << j;
       }
-      dead[wd] = m;
+      const int left = Na - 32 * wd;
+      s_dead_bits[wd] = left < 32 ? b | ~0u << left : b;
     }
   }
+  const unsigned long long c_start = clock64();  // the loop's own duration (stats)
   if (tid == 0) {
-    if (ls->nslots_pre < 0) ls->nslots_pre = ls->nslots;  // the step's first launch
-    sh.nslots = ls->nslots;
-    sh.mb[0].valid = sh.mb[1].valid = 0;
-    sh.susp[0] = sh.susp[1] = 0;
-    for (int q = 0; q < 16; ++q) sh.sb[0][q] = sh.sb[1][q] = best_none();
-    sh.fin = 0;
-    sh.r_i1 = -1;
-    s_go = 1;
-    if (!GD && Na > DB) {
-      s_go = -3;  // more interface cells than the LDS bitmap holds: the host relaunches with GD
-    } else if (ls->nslots > CAP) {
-      s_go = -2;  // more growing cells than this tier holds
-    } else if (ls->pending) {
-      sh.r_i1 = ls->pend_tgt;
-      s_go = 2;   // resume with the pending nucleation
-    } else if (ls->events == 0 && ls->Na == ls->nmushy0) {
-      s_go = 0;   // loop condition vSind2 != countS fails at once (S/VoxelsCA.C:381)
-    }
+    int go = 1;
+    if (!GD && Na > AMCD_DEAD_BITS)
+      go = -3;  // more interface cells than the LDS bitmap holds: the host relaunches with GD
+    else if (ns_first > CAP)
+      go = -2;  // more growing cells than this tier holds
+    else if (ls->pending)
+      go = 2;   // resume with the pending nucleation
+    else if (ls->events == 0 && Na == ls->nmushy0)
+      go = 0;   // loop condition vSind2 != countS fails at once (S/VoxelsCA.C:381)
+    sh.go = go;
+    sh.r_i1 = ls->pend_tgt;
+    sh.nslots = ns_first;
+    sh.T = ls->tinc;
+    sh.fin = go > 0 ? 1 : (go == 0 ? 0 : -2);
+    sh.units = 0;
+    sh.cur = ls->rng;
   }
+  if (tid < 32) sh.hist[tid] = 0;
   __syncthreads();
-  const int go = s_go;
-  long long visits = 0, evals = 0;
-  if (w > 0) {
-    if constexpr (K > 0)
-      owner_loop<NT, K>(d, sh, dead, s_hc, go, ls->tinc, visits, evals);
-    else
-      owner_loop_mem<NT>(d, sh, dead, go, ls->tinc, visits, evals);
-  } else {
-    // engine state, identical in every lane of wave 0
-    long long e_visits = 0, e_evals = 0, e_units = 0;
-    double tinc = ls->tinc;
-    int vSind2 = ls->vSind2, nGrain = ls->nGrain, pool_used = ls->pool_used;
-    int events = ls->events, captures = ls->captures, nucs = ls->nucs;
-    int nslots = ls->nslots;
-    const int ns_pre = ls->nslots_pre;
-    // the uniforms, 64 per batch, drawn ahead by jump-ahead (S/VoxelsCA.C:483)
-    const unsigned int x0 = ls->rng;
-    const long long draws0 = ls->draws;
-    const unsigned int aj = lcg_pow(2ull * lane + 1), c128 = lcg_pow(128);
-    unsigned int cb = 1;  // 16807^(128 b) for the next batch b to write
-    int nd = 0;
-    if (go > 0) {
-      sh.ubuf[0][lane] = draw_batch(x0, cb, aj);
-      cb = mod_m((unsigned long long)cb * c128);
-    }
-    int par = 0, fin = 0;
-    const unsigned long long c_start = clock64();  // the loop's own duration (stats)
-    Decision x;
-    x.stop = 0;
-    x.nuc = 1;
-    x.i1 = sh.r_i1;
-    x.cand = -1;
-    x.wave = 0;
-    x.dt = 0.0;
-    bool apply_first = go == 2;
-    EnginePrefetch pf;
-    bool have_pf = false;  // the event's inputs were prefetched with its decision
-    PHASE_FLAGS(eflag);
-    PHASE_INIT(et);
-    while (go > 0) {
-      if (!apply_first) {
-        PHASE(et, 0, tid == 0);
-        PHASE_ARRIVE(sh, par, 0, eflag);
-        PHASE_FLAGS_CLEAR(eflag);
-        __syncthreads();
-        PHASE(et, 1, tid == 0);
-        PHASE_LAST(sh, par, NW);
-        {
-          const Best me = lane_entry<NW>(sh, par);
-          pf = engine_prefetch<NW>(d, sh, me, par, ns_pre);
-          x = decide_from<NW>(sh, me, par, tinc, DelT, rX, nd);
-          prefetch_landed(pf);
-        }
-        have_pf = true;
-        if (x.stop) {
-          fin = x.stop < 0 ? x.stop : 0;
-          break;
-        }
-        events++;
-        e_units += nslots;  // the growing list this event's decision covered
-        if ((nd & 63) == 0) {  // first draw of batch nd/64: write batch nd/64 + 1
-          sh.ubuf[((nd >> 6) + 1) & 1][lane] = draw_batch(x0, cb, aj);
-          cb = mod_m((unsigned long long)cb * c128);
-        }
-        ++nd;
-        PHASE(et, 2, tid == 0);
-      }
-      apply_first = false;
-      // ---- APPLY: the event on voxel i1
-      const int i1 = x.i1;
-      NewCell& nc = sh.mb[par ^ 1];
-      int susp = 0;
-      Best nb = best_none();
-      if (lane == 0) nc.valid = 0;
-      if (x.nuc && (pool_used >= st.n_pool || pool_used >= d.poolcap || nGrain >= d.gcap)) {
-        if (lane == 0) {
-          *gmem(&ls->pending) = 1;  // the host refills the pool and resumes
-          *gmem(&ls->pend_tgt) = i1;
-        }
-        susp = -1;
-      } else {
-        // the event's inputs: the captured voxel's neighbour table and pair ruqs, its cold
-        // flag and temperature, the winning entry's voxel, and the capturing cell's grain
-        // and rotation -- from the lanes that prefetched them with the decision (a resumed
-        // nucleation loads them here)
-        const int cand = x.cand, sw = cand >= 0 ? cand / AMCD_NB : 0;
-        // an entry of a list the set-up built carries its capture's re-centring
-        const bool pre = !x.nuc && sw < ns_pre;
-        int tn, cold, v1, vjs = 0, G = 1;
-        double rpair, T1, fcap = 0.0, R[9], c0[3], cen[3], E0;
-        double4 rc = make_double4(0.0, 0.0, 0.0, 0.0);
-        if (have_pf) {
-          const int wq = x.wave;
-          take_row(pf, wq, lane, tn, rpair);
-          cold = __builtin_amdgcn_readlane(pf.cold, wq);
-          T1 = lane_f64(pf.T1, wq);
-          v1 = __builtin_amdgcn_readlane(pf.v1, wq);
-          if (!x.nuc) {
+  const int go = sh.go;
+  const int nm0 = ls->nmushy0;
+  // engine state (meaningful in wave 0 only)
+  EngineState es;
+  es.T = sh.T;
+  es.vSind2 = ls->vSind2;
+  es.nGrain = ls->nGrain;
+  es.pool_used = ls->pool_used;
+  es.events = ls->events;
+  es.captures = ls->captures;
+  es.nucs = ls->nucs;
+  es.nd = 0;
+  es.visits = 0;
+  unsigned long long units = 0;
+  Cells<KR> c;
+  if (go > 0) {
+    const unsigned int aj = lcg_pow(2ull * lane + 1);
+    Window& win = sh.win;
+    double T = sh.T;
 #pragma unroll
-            for (int q = 0; q < 9; ++q) R[q] = lane_f64(pf.R[q], wq);
-            G = __builtin_amdgcn_readlane(pf.G, wq);
-            if (pre)
-              rc = make_double4(lane_f64(pf.rc.x, wq), lane_f64(pf.rc.y, wq), lane_f64(pf.rc.z, wq),
-                                lane_f64(pf.rc.w, wq));
-          }
+    for (int k = 0; k < KR; ++k) c.E[k] = c.V[k] = 0.0;
+    int ns = ns_first;  // slots the threads have taken over
+    // Refresh of every cell whose head died (or of all) by its own thread.
+    auto refresh_own = [&](bool all, int m, int scan0, double dtl, double T0) {
+      for (int it = 0, s0 = w * 64; s0 < ns; ++it, s0 += NT) {
+        const int s = s0 + lane;
+        const int2 h = s < ns ? get_hd<HM>(d, s) : make_int2(0, -1);
+        const bool on = h.y >= 0 && (all || live.dead(h.y));
+        if (!__any(on)) continue;
+        double e = 0.0, v = 0.0;
+        if constexpr (MEM) {
+          e = on ? gmem(d.gExt)[s] : 0.0;
+          v = on ? gmem(d.gVhat)[s] : 0.0;
         } else {
-          tn = (lane < AMCD_NB) ? gmem(d.aNbr)[(size_t)i1 * AMCD_NB + lane] : -1;
-          rpair = (lane < AMCD_NB) ? gmem(d.aRN)[(size_t)i1 * AMCD_NB + lane] : 0.0;
-          cold = gmem(d.aCold)[i1];
-          T1 = gmem(d.aT)[i1];
-          v1 = cand >= 0 ? gmem(d.cV)[cand] : gmem(d.aVox)[i1];  // (no entry: a resumed nucleation)
-          if (!x.nuc) {
 #pragma unroll
-            for (int q = 0; q < 9; ++q) R[q] = gmem(d.gR)[9 * (size_t)sw + q];
-            G = gmem(d.gG)[sw];
-            if (pre) {
-              const auto q = gmem((double*)(d.cRC + cand));
-              rc = make_double4(q[0], q[1], q[2], q[3]);
+          for (int k = 0; k < KR; ++k) {
+            e = k == it ? c.E[k] : e;
+            v = k == it ? c.V[k] : v;
+          }
+        }
+        const Refreshed o = refresh_cell<GD>(d, live, on, h.x, e, v, -1, m, scan0, dtl, T0, T);
+        if (on) {
+          set_hd<HM>(d, s, o.c1, o.tgt);
+          set_lh<HM>(d, s, o.lo, o.hi);
+          if (o.tgt < 0) {
+            if constexpr (MEM) {
+              gmem(d.gExt)[s] = o.grown;
+              gmem(d.gVhat)[s] = 0.0;
+            } else {
+#pragma unroll
+              for (int k = 0; k < KR; ++k) {
+                c.E[k] = k == it ? o.grown : c.E[k];
+                c.V[k] = k == it ? 0.0 : c.V[k];
+              }
             }
           }
         }
-        PHASE(et, 9, tid == 0);
-        if (!x.nuc && !pre) {  // a cell made in this launch: re-centred below
+      }
+    };
+    // every cell starts at its list's first entry
+    for (int s = tid; s < ns; s += NT) {
+      const bool any = gmem(d.slots)[s].n > 0;
+      set_hd<HM>(d, s, any ? gmem(d.slots)[s].base : 0, any ? 0 : -1);
+      set_lh<HM>(d, s, fInf, fInf);
+      if (MEM && !any) gmem(d.gVhat)[s] = 0.0;
+    }
+    if constexpr (!MEM) {
 #pragma unroll
-          for (int q = 0; q < 3; ++q) c0[q] = gmem(d.gC)[3 * (size_t)sw + q];
-          fcap = gmem(d.cF)[cand];
-          vjs = gmem(d.gV)[sw];
+      for (int k = 0; k < KR; ++k) {
+        const int s = tid + k * NT;
+        if (s < ns) {
+          c.E[k] = gmem(d.gExt)[s];
+          c.V[k] = get_hd<HM>(d, s).y >= 0 ? gmem(d.gVhat)[s] : 0.0;
         }
-        if (x.nuc) {  // S/VoxelsCA.C:486-506
-          PHASE_FLAG(eflag, 8);
-          const auto P = gmem(d.pool) + 9 * (size_t)pool_used;
-          for (int q = 0; q < 9; ++q) R[q] = P[q];
-          G = nGrain + 1;
-          centre(d, v1, cen);
-          E0 = 0.0;
-          if (lane < 9) gmem(d.rot)[9 * (size_t)(G - 1) + lane] = P[lane];
-          nGrain = G;
-          pool_used++;
-          nucs++;
-          if (lane == 0) *gmem(&ls->pending) = 0;
-        } else {      // S/VoxelsCA.C:507-605
-          if (pre) {
-            cen[0] = rc.x;
-            cen[1] = rc.y;
-            cen[2] = rc.z;
-            E0 = rc.w;
-            PHASE_FLAG(eflag, 1);
-          } else {
-            PHASE_FLAG(eflag, 2);
-            recentre(d, vjs, v1, c0, R, fcap, cen, &E0);
+      }
+    }
+    refresh_own(true, 0, 0, 0.0, T);
+    // clock span of a window, adapted to the entries it gets (about half of the growing cells
+    // have a candidate within a step)
+    double step = DelT * fmin(1.0, 80.0 / (double)max(ns_first, 1));
+    int nev = 0;  // events since the bounds were last recomputed
+    int want = 44;  // heads asked for
+    bool resume = go == 2;
+    PHASE_INIT(pt);
+    for (;;) {
+      const double T0 = T;
+      // ---- SELECT
+      float u = fInf;
+      const float Tf = (float)T, ibin = (float)(16.0 / step), top = Tf + 2.0f * (float)step;
+      for (int s0 = w * 64; s0 < ns; s0 += 4 * NT) {
+        float2 b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int s = s0 + lane + q * NT;
+          b[q] = s < ns ? get_lh<HM>(d, s) : make_float2(fInf, fInf);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          u = fminf(u, b[q].y);
+          if (b[q].x <= top) atomicAdd(&sh.hist[max(0, min(31, (int)((b[q].x - Tf) * ibin)))], 1);
+        }
+      }
+      u = wave_min(u);
+      if (lane == 0) sh.red[w] = u;
+      if (tid < WCAP) {
+        win.ev[tid] = make_int2(-2, -1);
+        win.rank[tid] = 0;
+      }
+      if (w == 1) {  // the window's uniforms, one per lane (S/VoxelsCA.C:483)
+        const unsigned int x1 = mod_m((unsigned long long)sh.cur * aj), x2 = lcg_next(x1);
+        const unsigned long long nuc = __ballot(canonical(x1, x2) < rX);
+        win.x2[lane] = x2;
+        if (lane == 0) win.draws = nuc;
+      }
+      if (tid == 0) {
+        win.n = 0;
+        win.done = 0;
+        win.scan0 = es.vSind2;
+        sh.tn = 0;
+      }
+      __syncthreads();
+      PHASE(pt, 0);
+      if (!resume) {
+        u = wave_min(lane < NW ? sh.red[lane] : fInf);
+        // the span that takes `want` heads (later entries of their cells and new cells' come on
+        // top); the spans of the next windows follow it
+        int cum = lane < 32 ? sh.hist[lane] : 0;
+        cum += __builtin_amdgcn_update_dpp(0, cum, 0x111, 0xf, 0xf, false);
+        cum += __builtin_amdgcn_update_dpp(0, cum, 0x112, 0xf, 0xf, false);
+        cum += __builtin_amdgcn_update_dpp(0, cum, 0x114, 0xf, 0xf, false);
+        cum += __builtin_amdgcn_update_dpp(0, cum, 0x118, 0xf, 0xf, false);
+        cum += __builtin_amdgcn_update_dpp(0, cum, kBcast15, 0xa, 0xf, false);
+        const int bins = __popcll(__ballot(lane < 32 && cum <= want));
+        float W = fmaxf(Tf + (float)bins / ibin, u);
+        step *= bins >= 32 ? 1.6 : fmax(0.4, (bins + 8) / 26.0);
+        // ---- the window's entries
+        int mode = 0;  // 0: clock span, 1: less of it, 2: up to u, 3: exact best of every wave, one event
+        for (;; ++mode) {
+          if (mode > 0) W = mode == 1 ? fmaxf(Tf + 0.4f * (W - Tf), u) : u;
+          if (mode < 3) {
+            for (int s0 = tid; s0 < ns; s0 += KR * NT) {
+              unsigned todo = 0;
+#pragma unroll
+              for (int k = 0; k < KR; ++k) {
+                const int s = s0 + k * NT;
+                const float lo = s < ns ? get_lh<HM>(d, s).x : fInf;
+                todo |= (unsigned)(lo != fInf && lo <= W) << k;
+              }
+              while (todo != 0) {
+                const int k1 = __builtin_ctz(todo);
+                todo &= todo - 1;
+                const int s = s0 + k1 * NT;
+                double E = 0, V = 0;
+                if constexpr (MEM) {
+                  E = gmem(d.gExt)[s];
+                  V = gmem(d.gVhat)[s];
+                } else {
+#pragma unroll
+                  for (int k = 0; k < KR; ++k) {
+                    E = k == k1 ? c.E[k] : E;
+                    V = k == k1 ? c.V[k] : V;
+                  }
+                }
+                const float2 b = get_lh<HM>(d, s);
+                push_cell<GD>(d, live, win, s, E, V, get_hd<HM>(d, s).x, b.x, b.y, T, W, ns_pre);
+              }
+              if (!MEM) break;
+            }
+          } else {  // exact best of every wave
+            Best b = best_none();
+            int bs = 0;
+            double be = 0, bv = 0;
+            for (int s0 = tid; s0 < ns; s0 += KR * NT) {
+#pragma unroll
+              for (int k = 0; k < KR; ++k) {
+                const int s = s0 + k * NT;
+                const float lo = s < ns ? get_lh<HM>(d, s).x : fInf;
+                if (lo != fInf && lo <= u)
+                  exact_cell<GD>(d, live, s, MEM ? gmem(d.gExt)[s] : c.E[k], MEM ? gmem(d.gVhat)[s] : c.V[k],
+                                 get_hd<HM>(d, s).x, b, bs, be, bv);
+              }
+              if (!MEM) break;
+            }
+            const Best wb = wave_best(b);
+            if (wb.cand >= 0 && wb.cand == b.cand) {
+              const int i = put_entry(win, load_rec(d.cand + b.cand), be, bv, b.key, b.cand, bs, -1, order_key(-fInf),
+                                      order_key(u));
+              win.lim[i] = (int)0x80000000;
+            }
           }
-          captures++;
+          __syncthreads();
+          if (win.n <= WCAP) break;
+          __syncthreads();
+          if (tid == 0) win.n = 0;
+          __syncthreads();
         }
-        PHASE(et, 10, tid == 0);
-        const int scan = vSind2;
+        // (as many heads as leave room for what comes on top of them)
+        want = mode > 0 ? max(8, want * 5 / 8) : win.n < 44 ? min(56, want + 2) : win.n > 56 ? want - 1 : want;
+        {
+          // every entry's position by its upper bound: each wave counts a share of the others
+          const int n = win.n, j0 = w * (WCAP / NW);
+          if (lane < n && j0 < n) {
+            const int h = win.hi[lane];
+            int before = 0;
+#pragma unroll
+            for (int j = 0; j < WCAP / NW; ++j) {
+              const int hj = win.hi[j0 + j];
+              before += (j0 + j < n) & ((hj < h) | ((hj == h) & (j0 + j < lane))) ? 1 : 0;
+            }
+            if (before) atomicAdd(&win.rank[lane], before);
+          }
+          if (w == NW - 1 && lane < n) win.y[lane] = 1.0 / win.V[lane];
+        }
+        __syncthreads();
+        PHASE(pt, 1);
+        // ---- ENGINE
+        if (w == 0) {
+          __builtin_amdgcn_s_setprio(3);
+          engine_window(d, sh, win, es, W, mode == 3 ? 1 : WCAP, DelT, n_pool, ls);
+          __builtin_amdgcn_s_setprio(0);
+        }
+      } else if (w == 0) {
+        // a resumed nucleation: the window's one event, decided before the suspension
+        es.nGrain++;
         if (lane == 0) {
-          gmem(d.aG)[i1] = G;
-          gmem(d.aCx)[i1] = cen[0];
-          gmem(d.aCy)[i1] = cen[1];
-          gmem(d.aCz)[i1] = cen[2];
-          gmem(d.aExt)[i1] = E0;
+          const int i1 = sh.r_i1;
+          win.dt[0] = 0.0;
+          win.G = es.nGrain;
+          win.pool = es.pool_used;
+          win.m = 1;
+          win.decided = 0;
+          gmem(d.aScan)[i1] = es.vSind2;
+          *gmem(&ls->pending) = 0;
+          publish(win, 0, -1, i1);
+          *(volatile int*)&win.done = 1;
+        }
+        es.vSind2++;
+        es.pool_used++;
+        es.nucs++;
+      }
+      resume = false;
+      PHASE(pt, 2);
+      // ---- BUILD, while the engine goes on
+      if (w > 0) build_cells<GD>(I + blockIdx.x, w - 1, NW - 1, ns_pre, nm0);
+      __syncthreads();
+      PHASE(pt, 3);
+      T = sh.T;
+      int fin = sh.fin;
+      const int m = uni(win.m), scan0 = uni(win.scan0), ns1 = sh.nslots;
+      if (w == 0) {
+        units += (unsigned long long)win.decided * (unsigned)ns;
+        if (lane < m) {
+          const int i1 = win.ev[lane].y;
+          live.kill(i1);
           gmem(d.aVS)[i1] = 2;
-          gmem(d.aScan)[i1] = scan;
-          dead[i1 >> 5] |= 1u << (i1 & 31);
+          const int later = win.decided - 1 - lane;  // events that the reference scans its cell for
+          if (win.slot[lane] >= 0 && later > 0) atomicAdd(&sh.units, (unsigned long long)later);
         }
-        vSind2++;
-        tinc += x.dt;
-        PHASE(et, 3, tid == 0);
-        // the new mushy voxel joins the growing list if it has liquid neighbours
-        const bool liq = live_target(dead, tn, i1);
-        const unsigned long long bal = __ballot(liq);
-        if (cold && bal) {
-          PHASE_FLAG(eflag, 4);
-          const int slot = nslots;
-          const size_t cb = (size_t)slot * AMCD_NB;
-          const double V0 = growth_velocity(p, T1);
-          double D = __builtin_inf(), f = 0, r = __builtin_inf();
-          int key = 0x7fffffff;
-          // neighbour lane of v1, in the order of the active-neighbour table
-          int vi, vj, vk;
-          decode(d, v1, vi, vj, vk);
-          const int qq = lane < 13 ? lane : lane + 1;
-          const int ddx = qq % 3 - 1, ddy = (qq / 3) % 3 - 1, ddz = qq / 9 - 1;
-          const int vt = v1 + ddz * d.nxy + ddy * p.nx + ddx;
-          if (liq) {
-            const double ct[3] = {((double)(vi + ddx) + .5) * p.dx, ((double)(vj + ddy) + .5) * p.dy,
-                                  ((double)(vk + ddz) + .5) * p.dz};
-            candidate_at(ct, cen, R, &D, &f);
-            r = rpair;
-            key = scan * 32 + lane;
-          }
-          // position in (D, ruqs, key) order among the liquid neighbours (cand_less): a
-          // uniform loop over the ballot's set bits that broadcasts only D counts the
-          // neighbours strictly before by D (NaN last) and marks those with an equal D;
-          // a second loop over the lanes in some tie orders those by (ruqs, key)
-          int rank = 0;
-          unsigned long long tie = 0;
-          const bool nan_me = D != D;
-          for (unsigned long long m = bal; m != 0; m &= m - 1) {
-            const int j = (int)__builtin_ctzll(m);
-            const double Dj = lane_f64(D, j);
-            const bool nan_j = Dj != Dj;
-            const bool before = (nan_me & !nan_j) | (!nan_me & !nan_j & (Dj < D));
-            const bool same = (j != lane) & ((nan_me & nan_j) | (!nan_me & !nan_j & (Dj == D)));
-            rank += before ? 1 : 0;
-            tie |= (unsigned long long)same << j;
-          }
-          for (unsigned long long m = __ballot(liq & (tie != 0)); m != 0; m &= m - 1) {
-            const int j = (int)__builtin_ctzll(m);
-            const double rj = lane_f64(r, j);
-            const int kj = __builtin_amdgcn_readlane(key, j);
-            const bool rne = rj != r;
-            const bool before = (rne & (rj < r)) | (!rne & (kj < key));
-            rank += (((tie >> j) & 1ull) != 0 && before) ? 1 : 0;
-          }
-          if (liq) {
-            gmem(d.cD)[cb + rank] = D;
-            gmem(d.cF)[cb + rank] = f;
-            gmem(d.cR)[cb + rank] = r;
-            gmem(d.cTgt)[cb + rank] = tn;
-            gmem(d.cV)[cb + rank] = vt;
-            gmem(d.cK)[cb + rank] = (uint8_t)lane;
-            if (rank == 0) {
-              nc.D1 = D;
-              nc.r1 = r;
-              nc.key1 = key;
-              nc.c1 = (int)cb;
-              nc.tgt1 = tn;
-              if (__popcll(bal) < 2) nc.Dn1 = __builtin_inf();
-            }
-            if (rank == 1) nc.Dn1 = D;
-            // this cell's exact best for the next event (all its targets are liquid)
-            const double tq = (D - E0) / V0;
-            if (tq <= 1e6) {
-              nb.t = tq;
-              nb.r = r;
-              nb.key = key;
-              nb.cand = (int)(cb + rank);
-              nb.tgt = tn;
+        nev += m;
+        if (lane == 0) {
+          sh.all = nev >= (1 << 20);
+          sh.neg = 0;
+        }
+        nev = nev >= (1 << 20) ? 0 : nev;
+      }
+      if (m == 0 && fin == 1) fin = -4;  // a window always performs an event or ends the loop
+      __syncthreads();
+      // ---- APPLY: the cells whose head died (or, now and then, all), listed so that their list
+      // reads run side by side over the workgroup
+      const bool all = sh.all;
+      if (tid < 32) sh.hist[tid] = 0;  // (read before ENGINE, filled again after APPLY)
+      unsigned touched = 0;  // the thread's listed cells (register tiers)
+      for (int s0 = w * 64; s0 < ns; s0 += KR * NT) {
+        unsigned bits = 0;
+        int total = 0;
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+          const int s = s0 + lane + k * NT;
+          const int tg = s < ns ? get_hd<HM>(d, s).y : -1;
+          const bool dd = live.dead(tg >= 0 ? tg : 0);
+          const bool on = tg >= 0 && (dd || all);
+          bits |= (unsigned)on << k;
+          total += __popcll(__ballot(on));
+        }
+        if (total != 0) {
+          int base = 0;
+          if (lane == 0) base = atomicAdd(&sh.tn, total);
+          base = uni(base);
+#pragma unroll
+          for (int k = 0; k < KR; ++k) {
+            const bool on = (bits >> k) & 1u;
+            const unsigned long long bal = __ballot(on);
+            if (bal == 0) continue;
+            const int i = base + __popcll(bal & ((1ull << lane) - 1));
+            base += __popcll(bal);
+            if (on && i < TCAP) {
+              const int s = s0 + lane + k * NT;
+              sh.tS[i] = s;
+              sh.tE[i] = MEM ? gmem(d.gExt)[s] : c.E[k];
+              sh.tV[i] = MEM ? gmem(d.gVhat)[s] : c.V[k];
             }
           }
-          nb = wave_best(nb);
-          e_visits++;
-          e_evals += __popcll(bal);
-          // the slot's static capture inputs (rotation, centroid, voxel)
-          double rv = 0.0;
-#pragma unroll
-          for (int q = 0; q < 9; ++q)
-            if (q == lane) rv = R[q];
-#pragma unroll
-          for (int q = 0; q < 3; ++q)
-            if (q + 9 == lane) rv = cen[q];
-          if (lane < 9) gmem(d.gR)[9 * (size_t)slot + lane] = rv;
-          if (lane >= 9 && lane < 12) gmem(d.gC)[3 * (size_t)slot + lane - 9] = rv;
-          if (lane == 0) {
-            gmem(d.gV)[slot] = v1;
-            gmem(d.gG)[slot] = G;
-            gmem(d.gAct)[slot] = i1;
-            gmem(d.gScan)[slot] = scan;
-            gmem(d.gExt)[slot] = E0;
-            gmem(d.gVhat)[slot] = V0;
-            gmem(d.gN)[slot] = (uint8_t)__popcll(bal);
-            gmem(d.gDead)[slot] = 0;
-            nc.E = E0;
-            nc.V = V0;
-            nc.slot = slot;
-            nc.valid = slot < CAP;  // beyond this tier: resume with a larger one
-          }
-          nslots = slot + 1;
-          if (slot >= CAP && tinc < DelT) susp = -2;
         }
-        PHASE(et, 4, tid == 0);
+        touched = bits;
+        if (!MEM) break;
       }
-      if (lane == 0) {
-        sh.sb[par ^ 1][0] = nb;
-        sh.susp[par ^ 1] = susp;
-        sh.nslots = nslots;
+      __syncthreads();
+      PHASE(pt, 4);
+      const double dtl = lane < m ? win.dt[lane] : 0.0;  // lane j: growth time of event j
+      int nt = sh.tn;
+      if (nt > TCAP || all) {  // more than the list holds
+        refresh_own(all, m, scan0, dtl, T0);
+        nt = 0;
+        touched = 0;
       }
-      par ^= 1;
+      // growth, event by event in the reference's order (S/VoxelsCA.C:511-516), of the cells of
+      // before the window; a nucleation's time is 0: E + V*0 = E
+      bool neg = false;
+      for (int s0 = w * 64; s0 < ns; s0 += KR * NT) {
+        if constexpr (MEM) {
+#pragma unroll
+          for (int k = 0; k < KR; ++k) {
+            const int s = s0 + lane + k * NT;
+            c.E[k] = s < ns ? gmem(d.gExt)[s] : 0.0;
+            c.V[k] = s < ns ? gmem(d.gVhat)[s] : 0.0;
+          }
+        }
+        for (int j = 0; j < m; ++j) {
+          const double dt = lane_f64(dtl, j);
+#pragma unroll
+          for (int k = 0; k < KR; ++k) c.E[k] = c.E[k] + c.V[k] * dt;
+        }
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+          neg |= c.E[k] < 0.0;
+          if constexpr (MEM) {
+            const int s = s0 + lane + k * NT;
+            if (s < ns) gmem(d.gExt)[s] = c.E[k];
+          }
+        }
+        if (!MEM) break;
+      }
+      int fixs = -1;  // a cell out of candidates, and its final half-diagonal (memory tier)
+      double fixe = 0.0;
+      static_assert(!MEM || TCAP + WCAP <= NT, "one round over the list");
+      for (int i0 = 0; i0 < nt + m; i0 += NT) {
+        const int i = i0 + lane * NW + w;  // spread over the waves
+        int s = -1, k0 = -1, c0 = 0;
+        double e = 0.0, v = 0.0;
+        if (i < nt) {
+          s = sh.tS[i];
+          e = sh.tE[i];
+          v = sh.tV[i];
+          c0 = get_hd<HM>(d, s).x;
+        } else if (i < nt + m) {
+          k0 = i - nt;
+          s = win.slot[k0];
+          if (s >= 0) {
+            c0 = win.base[k0];
+            e = win.E0[k0];
+            v = win.V0[k0];
+          }
+        }
+        const Refreshed o = refresh_cell<GD>(d, live, s >= 0, c0, e, v, k0, m, scan0, dtl, T0, T);
+        if (s >= 0) {
+          if (i < nt) {
+            sh.tE[i] = o.grown;
+          } else {
+            gmem(d.gExt)[s] = o.grown;
+            gmem(d.gVhat)[s] = v;
+          }
+          if (HM || s < CAP) {
+            set_hd<HM>(d, s, o.tgt >= 0 ? o.c1 : i, o.tgt);
+            set_lh<HM>(d, s, o.lo, o.hi);
+          }
+          if (MEM && o.tgt < 0) {
+            fixs = s;
+            fixe = o.grown;
+          }
+        }
+      }
+      if (neg) sh.neg = 1;
+      __syncthreads();
+      PHASE(pt, 5);
+      // what the list's threads found: cells out of candidates, and the new cells
+      if constexpr (MEM) {
+        if (fixs >= 0) {
+          gmem(d.gExt)[fixs] = fixe;
+          gmem(d.gVhat)[fixs] = 0.0;
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+          const int s = tid + k * NT;
+          if ((touched >> k) & 1u) {
+            const int2 h = get_hd<HM>(d, s);
+            if (h.y < 0) {
+              c.E[k] = sh.tE[h.x];
+              c.V[k] = 0.0;
+            }
+          }
+          if (s >= ns && s < ns1) {
+            c.E[k] = gmem(d.gExt)[s];
+            c.V[k] = get_hd<HM>(d, s).y >= 0 ? gmem(d.gVhat)[s] : 0.0;
+          }
+        }
+      }
+      if (sh.neg) {
+        // the reference's clamp at zero, which moves the cell's capture times: only a window's
+        // last event can step back in time (or grow by a negative velocity) and so need it
+        if constexpr (MEM) __syncthreads();
+        for (int s0 = tid; s0 < ns; s0 += KR * NT) {
+#pragma unroll
+          for (int k = 0; k < KR; ++k) {
+            const int s = s0 + k * NT;
+            if (s >= ns) continue;
+            if ((MEM ? gmem(d.gExt)[s] : c.E[k]) < 0.0) {
+              if constexpr (MEM) gmem(d.gExt)[s] = 0.0;
+              else c.E[k] = 0.0;
+              const int2 h = get_hd<HM>(d, s);
+              if (h.y >= 0) {
+                float lo, hi;
+                tau_bounds(load_rec(d.cand + h.x).D, 0.0, MEM ? gmem(d.gVhat)[s] : c.V[k], T, lo, hi);
+                set_lh<HM>(d, s, lo, hi);
+              }
+            }
+          }
+          if (!MEM) break;
+        }
+      }
+      if (MEM) __syncthreads();  // (another thread's stores of a cell's state)
+      ns = min(ns1, CAP);
+      PHASE(pt, 6);
+      if (ns1 > CAP && fin == 1) fin = T < DelT ? -2 : 0;  // cells beyond this tier: the host resumes
+      if (fin != 1) {
+        if (tid == 0) sh.fin = fin;
+        break;
+      }
     }
-    if (tid == 0) {
-      sh.fin = fin;
-      ls->tinc = tinc;
-      ls->vSind2 = vSind2;
-      ls->nGrain = nGrain;
-      ls->pool_used = pool_used;
-      ls->events = events;
-      ls->captures = captures;
-      ls->nucs = nucs;
-    }
-    if (tid == 1 && go != -2) {  // engine state after the nd draws of this launch
-      ls->rng = mod_m((unsigned long long)x0 * lcg_pow(2ull * nd));
-      ls->draws = draws0 + 2ll * nd;
-      O[blockIdx.x].draws = draws0 + 2ll * nd;
-    }
-    visits += e_visits;
-    evals += e_evals;
-    if (tid == 0) {
-      atomicAdd((unsigned long long*)&O[blockIdx.x].interface_events, (unsigned long long)e_units);
-      atomicAdd((unsigned long long*)&O[blockIdx.x].loop_cycles, clock64() - c_start);
+    // half-diagonals back to the growing list (the cells not taken over are current there)
+    if constexpr (!MEM) {
+#pragma unroll
+      for (int k = 0; k < KR; ++k) {
+        const int s = tid + k * NT;
+        if (s < ns) gmem(d.gExt)[s] = c.E[k];
+      }
     }
   }
+  if (tid == 0) sh.nexec = es.vSind2 - nm0;
   __syncthreads();
   // ---- loop state and counters
   const int ns = sh.nslots;
-  const int fin = sh.fin;  // 0 finished, -1 pool refill, -2 larger tier
-  const bool suspended = go == -2 || go == -3 || fin < 0;
-  if (!suspended)
-    for (int s = tid; s < ns; s += NT) d.aExt[d.gAct[s]] = d.gExt[s];
-  atomicAdd((unsigned long long*)&O[blockIdx.x].slot_visits, (unsigned long long)visits);
-  atomicAdd((unsigned long long*)&O[blockIdx.x].cand_evals, (unsigned long long)evals);
+  const int fin = sh.fin;
+  if (fin == 0) {
+    // the step's events, and the half-diagonals of every growing cell, to the active arrays
+    for (int q = tid; q < sh.nexec; q += NT) {
+      const EventRec e = d.events[q];
+      gmem(d.aG)[e.i1] = e.G;
+      gmem(d.aCx)[e.i1] = e.x;
+      gmem(d.aCy)[e.i1] = e.y;
+      gmem(d.aCz)[e.i1] = e.z;
+      gmem(d.aExt)[e.i1] = e.E;
+    }
+    __syncthreads();
+    for (int s = tid; s < ns; s += NT) gmem(d.aExt)[gmem(d.slots)[s].act] = gmem(d.gExt)[s];
+  }
   if (tid == 0) {
-    const int status = go == -3 ? -3 : (go == -2 ? 2 : (fin == -1 ? 1 : (fin == -2 ? 2 : 0)));
+    const int status = go == -3 ? -3 : fin == -1 ? 1 : fin == -2 ? 2 : fin == 0 ? 0 : -4;
+    ls->nslots_pre = ns_pre;
+    ls->tinc = es.T;
+    ls->vSind2 = es.vSind2;
+    ls->nGrain = es.nGrain;
+    ls->pool_used = es.pool_used;
+    ls->events = es.events;
+    ls->captures = es.captures;
+    ls->nucs = es.nucs;
+    ls->rng = sh.cur;
+    ls->draws += 2ll * es.nd;
     ls->nslots = ns;
     ls->done = status == 0 ? 1 : 0;
     amcd_out& o = O[blockIdx.x];
     o.status = status;
-    o.n_events = ls->events;
-    o.n_captures = ls->captures;
-    o.n_nucleations = ls->nucs;
+    o.n_events = es.events;
+    o.n_captures = es.captures;
+    o.n_nucleations = es.nucs;
     o.n_slots = ns;
-    o.nGrain = ls->nGrain;
-    o.pool_used = ls->pool_used;
-    o.tinc = ls->tinc;
+    o.nGrain = es.nGrain;
+    o.pool_used = es.pool_used;
+    o.tinc = es.T;
+    o.draws = ls->draws;
+    o.interface_events += (long long)(units + sh.units);
+    o.slot_visits += es.visits;
+    o.cand_evals += es.visits;
+    o.loop_cycles += (long long)(clock64() - c_start);
   }
 }
 
@@ -2894,16 +3118,15 @@ static int dalloc(amcd_batch* b, T** p, size_t n) {
 static int alloc_active(amcd_batch* b, Inst& d, int acap) {
   d.acap = acap;
   size_t c = (size_t)acap;
+  // about 80 entries per growing cell, of which there are far fewer than active cells
+  d.precap = (int)std::min<size_t>(8 * c, (size_t)1 << 26);
+  if (c * AMCD_NB + (size_t)d.precap > 0x7fffff00ull) d.precap = 0;  // entries are counted in 32 bits
   if (dalloc(b, &d.aVox, c) || dalloc(b, &d.aVS, c) || dalloc(b, &d.aG, c) || dalloc(b, &d.aT, c) ||
       dalloc(b, &d.aExt, c) || dalloc(b, &d.aCx, c) || dalloc(b, &d.aCy, c) || dalloc(b, &d.aCz, c) ||
-      dalloc(b, &d.ruq, c) || dalloc(b, &d.aNbr, c * AMCD_NB) || dalloc(b, &d.aCold, c) ||
-      dalloc(b, &d.aScan, c) || dalloc(b, &d.gAct, c) || dalloc(b, &d.gScan, c) || dalloc(b, &d.gExt, c) ||
-      dalloc(b, &d.gVhat, c) || dalloc(b, &d.gN, c) || dalloc(b, &d.gDead, c) || dalloc(b, &d.gGrow, c) ||
-      dalloc(b, &d.cD, c * AMCD_NB) || dalloc(b, &d.cF, c * AMCD_NB) || dalloc(b, &d.cR, c * AMCD_NB) ||
-      dalloc(b, &d.cTgt, c * AMCD_NB) || dalloc(b, &d.cK, c * AMCD_NB) || dalloc(b, &d.aRN, c * AMCD_NB) ||
-      dalloc(b, &d.gR, c * 9) || dalloc(b, &d.gC, c * 3) || dalloc(b, &d.gV, c) || dalloc(b, &d.gG, c) ||
-      dalloc(b, &d.cV, c * AMCD_NB) || dalloc(b, &d.gLH, c) || dalloc(b, &d.gHd, c) ||
-      dalloc(b, &d.cRC, c * AMCD_NB) || dalloc(b, &d.gdead, (c + 31) / 32))
+      dalloc(b, &d.ruq, c) || dalloc(b, &d.aRow, c) || dalloc(b, &d.events, c) || dalloc(b, &d.aScan, c) ||
+      dalloc(b, &d.slots, c) || dalloc(b, &d.gExt, c) || dalloc(b, &d.gVhat, c) || dalloc(b, &d.gLH, c) ||
+      dalloc(b, &d.gHd, c) || dalloc(b, &d.cand, c * AMCD_NB + d.precap) ||
+      dalloc(b, &d.cF, c * AMCD_NB + d.precap) || dalloc(b, &d.cap, c * AMCD_NB + d.precap))
     return -1;
   return 0;
 }
@@ -3009,7 +3232,8 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
       amcd_destroy(b);
       return -1;
     }
-    int acap = (int)std::min<long long>(N, std::max<long long>(1 << 16, N / 8));
+    // (it grows on overflow; 2^23 interface cells are far more than a domain this size needs)
+    int acap = (int)std::min<long long>(N, std::max<long long>(1 << 16, std::min<long long>(N / 8, 1 << 23)));
     if (const char* ac = getenv("AMCAFE_ACTIVE_CAP_INIT"))  // tests: start small to exercise the growth path
       acap = (int)std::min<long long>(N, std::max(64, atoi(ac)));
     if (alloc_active(b, d, acap)) {
@@ -3335,43 +3559,28 @@ static int launch_update(amcd_batch* b, bool fused_temperature) {
   return 0;
 }
 
-// Capacity tiers of the capture loop: threads per workgroup x growing cells per thread.
-static int launch_event_loop_wide(amcd_batch* b);
+// Capacity tiers of the capture loop: threads per workgroup x growing cells per thread.  The
+// last but one keeps the cells in memory (no limit below the active capacity); the last one is
+// that with the liveness read from the states (interfaces beyond AMCD_DEAD_BITS).
+static const int kNTiers = 5;
+static const int kTierCap[kNTiers] = {256 * 4, 512 * 4, 512 * 8, 512 * 16, 0x7fffffff};
+extern "C++" template <int NT, int K, bool GD = false>
+static int launch_loop(amcd_batch* b) {
+  hipLaunchKernelGGL((k_event_loop<NT, K, GD>), dim3(b->n), dim3(NT), 0, b->stream, b->d_inst, b->d_steps, b->d_outs);
+  HIPT(hipGetLastError());
+  return 0;
+}
+static int launch_event_loop_wide(amcd_batch* b) { return launch_loop<512, 0, true>(b); }
 static int launch_event_loop(amcd_batch* b) {
-  const int n = b->n;
-  if (b->tier >= 5) return launch_event_loop_wide(b);
   switch (b->tier) {
-    case 0:
-      hipLaunchKernelGGL((k_event_loop<256, 4>), dim3(n), dim3(256), 0, b->stream, b->d_inst, b->d_steps, b->d_outs);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_event_loop<512, 4>), dim3(n), dim3(512), 0, b->stream, b->d_inst, b->d_steps, b->d_outs);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_event_loop<512, 8>), dim3(n), dim3(512), 0, b->stream, b->d_inst, b->d_steps,
-                         b->d_outs);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_event_loop<512, 16>), dim3(n), dim3(512), 0, b->stream, b->d_inst, b->d_steps,
-                         b->d_outs);
-      break;
-    default:
-      hipLaunchKernelGGL((k_event_loop<512, 0>), dim3(n), dim3(512), 0, b->stream, b->d_inst, b->d_steps,
-                         b->d_outs);
-      break;
+    case 0: return launch_loop<256, 4>(b);
+    case 1: return launch_loop<512, 4>(b);
+    case 2: return launch_loop<512, 8>(b);
+    case 3: return launch_loop<512, 16>(b);
+    case 4: return launch_loop<512, 0>(b);
+    default: return launch_event_loop_wide(b);
   }
-  HIPT(hipGetLastError());
-  return 0;
 }
-// the memory-resident tier with the liveness bitmap in memory (interfaces beyond AMCD_DEAD_BITS)
-static int launch_event_loop_wide(amcd_batch* b) {
-  hipLaunchKernelGGL((k_event_loop<512, 0, true>), dim3(b->n), dim3(512), 0, b->stream, b->d_inst, b->d_steps,
-                     b->d_outs);
-  HIPT(hipGetLastError());
-  return 0;
-}
-static const int kNTiers = 5;  // the last one keeps the cells in memory: no limit below the active capacity
-static const int kTierCap[kNTiers] = {192 * 4, 448 * 4, 448 * 8, 448 * 16, 0x7fffffff};
 
 static int read_outs(amcd_batch* b, amcd_out* outs) {
   HIPT(hipMemcpyAsync(b->h_outs, b->d_outs, sizeof(amcd_out) * b->n, hipMemcpyDeviceToHost, b->stream));
@@ -3594,10 +3803,11 @@ static int autotune_lists(amcd_batch* b) {
     ls[0] = 0;
     for (int i = 0; i < n; ++i) ls[i + 1] = ls[i] + std::min(kListCaps[c], (b->h[i].acap + 3) / 4);
     HIPT(hipMemcpyAsync(b->d_lstart, ls.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, b->stream));
-    hipLaunchKernelGGL(k_grow_lists, dim3(ls[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_lstart, n);
-    HIPT(hipEventRecord(b->ev[14], b->stream));
-    for (int r = 0; r < 3; ++r)
+    for (int r = 0; r < 4; ++r) {
+      if (r == 1) HIPT(hipEventRecord(b->ev[14], b->stream));
+      hipLaunchKernelGGL(k_clear_npre, dim3(n), dim3(64), 0, b->stream, b->d_inst);
       hipLaunchKernelGGL(k_grow_lists, dim3(ls[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_lstart, n);
+    }
     HIPT(hipEventRecord(b->ev[15], b->stream));
     HIPT(hipGetLastError());
     HIPT(hipEventSynchronize(b->ev[15]));
