@@ -241,7 +241,7 @@ __device__ static inline void decode(DI& d, int v, int& i, int& j, int& k) {
 //    quotient is >= 1 and so is the rounded sum of squares);
 //  * while tvalid holds, the previous T of a voxel is known from its hot flag and the
 //    previous laser plane, so T, the flag byte and BuildjID are stored only where they change;
-//  * a run of voxels whose row segment lies farther from the laser than the melt pool's
+//  * a run of voxels whose row segments lie farther from the laser than the melt pool's
 //    extent plus two voxels (in the unrotated frame: the rotation about the plate centre
 //    preserves distances up to rounding far below that margin) cannot reach tL, so in the
 //    planes the pool can reach it changes nothing unless one of its voxels was hot.
@@ -306,12 +306,14 @@ __global__ __launch_bounds__(GB) void k_temperature(Inst* I, const int* bstart, 
       for (int q = 0; q < TV; ++q) busy |= sv[q] & 0xbc;
       const double zp = ((double)k + .5) * p.dz;
       bool cold = k < kh0 || k > kh1 || zp > st.lz;  // no geometry reaches these voxels
-      if (!cold && i + TV <= p.nx) {  // a run inside one row: its distance to the laser
+      if (!cold) {  // the run's distance to the laser (of its rows' when it spans several)
         const double Lx = p.hx + st.cg * (st.lx - p.hx) - st.sg * (st.ly - p.hy);
         const double Ly = p.hy + st.sg * (st.lx - p.hx) + st.cg * (st.ly - p.hy);
-        const double xa = ((double)i + .5) * p.dx, xb = ((double)(i + TV - 1) + .5) * p.dx;
-        const double yc = ((double)j + .5) * p.dy;
-        const double ex = fmax(0.0, fmax(xa - Lx, Lx - xb)), ey = yc - Ly;
+        const bool one = i + TV <= p.nx;
+        const int ia = one ? i : 0, ib = one ? i + TV - 1 : p.nx - 1, jb = one ? j : j + (i + TV - 1) / p.nx;
+        const double xa = ((double)ia + .5) * p.dx, xb = ((double)ib + .5) * p.dx;
+        const double ya = ((double)j + .5) * p.dy, yb = ((double)jb + .5) * p.dy;
+        const double ex = fmax(0.0, fmax(xa - Lx, Lx - xb)), ey = fmax(0.0, fmax(ya - Ly, Ly - yb));
         const double A = fmax(p.bmDX0, p.a1[3]), B = fmax(p.a1[1], p.a1[4]);
         const double R = sqrt(A * A + B * B) + 2.0 * fmax(p.dx, p.dy);
         cold = ex * ex + ey * ey > R * R;
@@ -520,6 +522,84 @@ __global__ __launch_bounds__(GB) void k_setliquid(Inst* I, const int* bstart, in
   d.vs[v] = st | 0x80;
 }
 
+// A run of up to 16 consecutive voxels from v0 on, whatever rows it lies in: bit q of xlo, xhi, ylo,
+// yhi, zlo, zhi says that voxel v0 + q is on that side of the domain.
+struct RunEdges {
+  unsigned xlo, xhi, ylo, yhi, zlo, zhi;
+};
+__device__ static inline RunEdges run_edges(const Inst& d, int v0) {
+  const int nx = d.p.nx, ny = d.p.ny, nz = d.p.nz;
+  int i, j, k;
+  decode(d, v0, i, j, k);
+  RunEdges e = {0, 0, 0, 0, 0, 0};
+  if (i + 16 <= nx) {  // within a row
+    e.xlo = i == 0 ? 1u : 0u;
+    e.xhi = i + 16 == nx ? 1u << 15 : 0u;
+    e.ylo = j == 0 ? ~0u : 0u;
+    e.yhi = j == ny - 1 ? ~0u : 0u;
+    e.zlo = k == 0 ? ~0u : 0u;
+    e.zhi = k == nz - 1 ? ~0u : 0u;
+    return e;
+  }
+  for (int q = 0; q < 16;) {  // row by row
+    const int len = min(16 - q, nx - i);
+    const unsigned m = ((1u << len) - 1) << q;
+    e.xlo |= i == 0 ? 1u << q : 0u;
+    e.xhi |= i + len == nx ? 1u << (q + len - 1) : 0u;
+    e.ylo |= j == 0 ? m : 0u;
+    e.yhi |= j == ny - 1 ? m : 0u;
+    e.zlo |= k == 0 ? m : 0u;
+    e.zhi |= k >= nz - 1 ? m : 0u;
+    q += len;
+    i = 0;
+    if (++j == ny) {
+      j = 0;
+      ++k;
+    }
+  }
+  return e;
+}
+// Four state bytes at a time: bit 0 of each byte of the result is set for ...
+__device__ static inline unsigned bytes_liquid(unsigned x) { return x & ~(x >> 1) & 0x01010101u; }
+__device__ static inline unsigned bytes_solid(unsigned x) { return x & (x >> 1) & 0x01010101u; }
+__device__ static inline unsigned bytes_cool(unsigned x) {  // mushy, or liquid below tL
+  return ((x >> 1) & ~x & 0x01010101u) | (x & ~(x >> 1) & ~(x >> 7) & 0x01010101u);
+}
+// bit 0 of the four bytes to four adjacent bits
+__device__ static inline unsigned pack_bytes(unsigned b) { return (b * 0x10204080u) >> 28; }
+// Bit q: a Moore neighbour of voxel v0 + q has a state byte that `pred` marks.  Each of the nine rows
+// around the run is a run of 18 bytes itself (the run moved by the row's offset, and one byte to
+// either side), read with one 16-byte and one 4-byte load at whatever alignment it has; neighbours
+// across the domain's sides are masked out.  (Reads reach up to 20 bytes beyond the array, inside
+// the 256 that every device array is allocated beyond its length.)  Runs that span rows had gone
+// voxel by voxel, byte by byte: on 40x24x20 voxels k_solid_to_mushy 58 -> 4.8 us and k_active_flags
+// 62 -> 5.1 us; rows of a multiple of 16 (512x512x128, aligned loads before) 14.9 -> 15.3 and 20.3 ->
+// 16.8 us, so this is the only form.
+template <class Pred>
+__device__ static inline unsigned moore_marks(const Inst& d, int v0, const RunEdges& e, Pred pred) {
+  // (all nine rows' loads before the first use: one round of latency; a row outside the domain reads
+  // its nearest bytes and is masked)
+  uint4 w[9];
+  unsigned w4[9];
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    const int at = min(max(v0 + (r / 3 - 1) * d.nxy + (r % 3 - 1) * d.p.nx - 1, 0), d.N);
+    __builtin_memcpy(&w[r], d.vs + at, 16);
+    __builtin_memcpy(&w4[r], d.vs + at + 16, 4);
+  }
+  unsigned near = 0;
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    const int dz = r / 3 - 1, dy = r % 3 - 1, first = v0 + dz * d.nxy + dy * d.p.nx - 1;
+    const unsigned out = (dz < 0 ? e.zlo : dz > 0 ? e.zhi : 0u) | (dy < 0 ? e.ylo : dy > 0 ? e.yhi : 0u);
+    unsigned m = pack_bytes(pred(w[r].x)) | pack_bytes(pred(w[r].y)) << 4 | pack_bytes(pred(w[r].z)) << 8 |
+                 pack_bytes(pred(w[r].w)) << 12 | (pack_bytes(pred(w4[r])) & 3u) << 16;
+    m <<= min(max(-first, 0), 18);  // bit q: voxel v0 + q - 1 of the row
+    near |= ((m & ~e.xlo) | (m >> 1) | ((m >> 2) & ~e.xhi)) & ~out;
+  }
+  return near;
+}
+
 // ConvertSolid1(1): solid -> mushy when any Moore neighbour is liquid.  Updating in
 // place is equivalent to the reference's collect-then-apply, because the update
 // (3 -> 2) never changes the predicate (some neighbour == 1) of any other voxel.
@@ -527,7 +607,7 @@ __global__ __launch_bounds__(GB) void k_solid_to_mushy(Inst* I, const int* bstar
   int ii = find_inst(bstart, ninst, blockIdx.x);
   const Inst d = I[ii];  // a copy: stores in the loops cannot alias it
   if (S[ii].skip) return;
-  const int nx = d.p.nx, ny = d.p.ny, nz = d.p.nz;
+  const int nz = d.p.nz;
   const int b0 = (blockIdx.x - bstart[ii]) * SB;
   const int bend = min(d.N, b0 + SB);
   // liquid exists only in planes that held it at the last active-set pass or that the
@@ -538,80 +618,29 @@ __global__ __launch_bounds__(GB) void k_solid_to_mushy(Inst* I, const int* bstar
   bool any = false;
   for (int z = max(0, zb0 - 1); z <= min(nz - 1, zb1 + 1); ++z) any = any || (d.zliq[z] & 1u) || (z >= h0 && z <= h1);
   if (!any) return;
-  // A solid voxel with a liquid Moore neighbour turns mushy.  Each thread takes 16
-  // consecutive voxels; when they share a row it reads the 3x3 rows around them (16 bytes
-  // and the two end voxels each): the liquid voxels of each row, widened by one voxel to
-  // either side and or-ed over the nine rows, are the solid voxels of the run to mark.
-  // Liquid voxels are not changed by the pass, so every test reads settled states, and
-  // each thread writes its own voxels only.
+  // A solid voxel with a liquid Moore neighbour turns mushy.  Each thread takes 16 consecutive
+  // voxels and reads the nine rows around them (moore_marks).  Liquid voxels are not changed by
+  // the pass, so every test reads settled states, and each thread writes its own voxels only.
+  // Bound by latency: 15 us for 512x512x128 (mostly blocks that leave at once), 4.8 us for 40x24x20.
   constexpr int PT = SB / GB;
   const int v0 = b0 + (int)threadIdx.x * PT;
   if (v0 >= bend) return;
-  int i, j, k;
-  decode(d, v0, i, j, k);
-  if (nx % PT == 0 && v0 + PT <= d.N) {
-    const uint4 c = *reinterpret_cast<const uint4*>(d.vs + v0);
-    const unsigned cw[4] = {c.x, c.y, c.z, c.w};
-    unsigned sol = 0;
+  const uint4 c = *reinterpret_cast<const uint4*>(d.vs + v0);  // (beyond the domain's end: not solid)
+  const unsigned cw[4] = {c.x, c.y, c.z, c.w};
+  unsigned sol = 0;
 #pragma unroll
-    for (int q = 0; q < PT; ++q) sol |= (((cw[q >> 2] >> (8 * (q & 3))) & 3u) == 3u ? 1u : 0u) << q;
-    if (!sol) return;
-    unsigned near = 0;
-    for (int dz = -1; dz <= 1; ++dz) {
-      const int z = k + dz;
-      if (z < 0 || z >= nz) continue;
-      for (int dy = -1; dy <= 1; ++dy) {
-        const int y = j + dy;
-        if (y < 0 || y >= ny) continue;
-        const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * nx;
-        const uint4 w = *reinterpret_cast<const uint4*>(row + i);
-        const unsigned ww[4] = {w.x, w.y, w.z, w.w};
-        unsigned liq = 0;  // bit q + 1: voxel i + q of the row is liquid
+  for (int r = 0; r < 4; ++r) sol |= pack_bytes(bytes_solid(cw[r])) << (4 * r);
+  if (v0 + PT > d.N) sol &= (1u << (d.N - v0)) - 1;
+  if (!sol) return;
+  const unsigned m = sol & moore_marks(d, v0, run_edges(d, v0), bytes_liquid);
+  if (!m) return;
+  unsigned nw[4];
 #pragma unroll
-        for (int q = 0; q < PT; ++q) liq |= (((ww[q >> 2] >> (8 * (q & 3))) & 3u) == 1u ? 1u : 0u) << (q + 1);
-        if (i > 0 && (row[i - 1] & 3) == 1) liq |= 1u;
-        if (i + PT < nx && (row[i + PT] & 3) == 1) liq |= 1u << (PT + 1);
-        near |= liq | (liq >> 1) | (liq >> 2);
-      }
-    }
-    const unsigned m = sol & near & ((1u << PT) - 1);
-    if (!m) return;
-    unsigned nw[4] = {cw[0], cw[1], cw[2], cw[3]};
-#pragma unroll
-    for (int q = 0; q < PT; ++q)
-      if ((m >> q) & 1u) nw[q >> 2] = (nw[q >> 2] & ~(3u << (8 * (q & 3)))) | (2u << (8 * (q & 3)));
+  for (int r = 0; r < 4; ++r) nw[r] = cw[r] & ~(((m >> (4 * r)) & 15u) * 0x204081u & 0x01010101u);  // 3 -> 2
+  if (v0 + PT <= d.N) {
     *reinterpret_cast<uint4*>(d.vs + v0) = make_uint4(nw[0], nw[1], nw[2], nw[3]);
-    return;
-  }
-  // rows that are not a multiple of 16 voxels, and the end of the domain: voxel by voxel
-  for (int q = 0; q < PT; ++q) {
-    const int v = v0 + q;
-    if (v >= bend) break;
-    const uint8_t sv = d.vs[v];
-    if ((sv & 3) == 3) {
-      bool hit = false;
-      for (int dz = -1; dz <= 1 && !hit; ++dz) {
-        const int z = k + dz;
-        if (z < 0 || z >= nz) continue;
-        for (int dy = -1; dy <= 1 && !hit; ++dy) {
-          const int y = j + dy;
-          if (y < 0 || y >= ny) continue;
-          const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * nx;
-          for (int dx = -1; dx <= 1; ++dx) {
-            const int x = i + dx;
-            if (x >= 0 && x < nx && (row[x] & 3) == 1) hit = true;
-          }
-        }
-      }
-      if (hit) d.vs[v] = (sv & ~3) | 2;
-    }
-    if (++i == nx) {
-      i = 0;
-      if (++j == ny) {
-        j = 0;
-        ++k;
-      }
-    }
+  } else {
+    for (int q = 0; q < d.N - v0; ++q) d.vs[v0 + q] = (uint8_t)(nw[q >> 2] >> (8 * (q & 3)));
   }
 }
 
@@ -623,29 +652,6 @@ __global__ void k_zliq_clear(Inst* I, const amcd_step* S) {
 }
 // Active set: {mushy} U {liquid below tL} U {neighbours at or above tL of those}.
 // Writes bit 6 of vs and the per-block (ZB voxels) counts of active and mushy cells.
-// A hot voxel that is neither mushy nor cool liquid is active when a Moore neighbour
-// is mushy or cool liquid.
-__device__ static bool hot_voxel_active(const Inst& d, int v) {
-  int i, j, k;
-  decode(d, v, i, j, k);
-  for (int dz = -1; dz <= 1; ++dz) {
-    const int z = k + dz;
-    if (z < 0 || z >= d.p.nz) continue;
-    for (int dy = -1; dy <= 1; ++dy) {
-      const int y = j + dy;
-      if (y < 0 || y >= d.p.ny) continue;
-      const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * d.p.nx;
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int x = i + dx;
-        if (x < 0 || x >= d.p.nx || (dx == 0 && dy == 0 && dz == 0)) continue;
-        const uint8_t sn = row[x];
-        const int stn = sn & 3;
-        if (stn == 2 || (stn == 1 && !(sn & 0x80))) return true;
-      }
-    }
-  }
-  return false;
-}
 // One wave per block of ZB voxels (four per workgroup), 16 consecutive voxels per thread,
 // four state bytes at a time: per byte, bit 0 of lo/hi/hb is state bit 0, state bit 1
 // and the hot flag.
@@ -673,76 +679,29 @@ __global__ __launch_bounds__(256) void k_active_flags(Inst* I, const int* bstart
       for (int q = 0; q < nq; ++q) w[q >> 2] |= (unsigned)d.vs[v0 + q] << (8 * (q & 3));
     }
     const unsigned valid = nq == PT ? 0xffffu : (1u << nq) - 1;
-    // hot voxels that are neither mushy nor cool liquid ask their Moore neighbours; when
-    // the 16 voxels share a row, the 3x3 rows around them are read whole: their mushy or
-    // cool liquid voxels, widened by one voxel either way and or-ed over the nine rows
+    // hot voxels that are neither mushy nor cool liquid ask their Moore neighbours
     unsigned hotpend = 0;  // bit q: voxel v0 + q is hot and not active by itself
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const unsigned x = w[r];
-      const unsigned lo = x & 0x01010101u, hi = (x >> 1) & 0x01010101u, hb = (x >> 7) & 0x01010101u;
-      const unsigned self = (hi & ~lo) | (lo & ~hi & ~hb);
-      const unsigned pend = hb & ~self;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) hotpend |= ((pend >> (8 * q)) & 1u) << (4 * r + q);
-    }
+    for (int r = 0; r < 4; ++r) hotpend |= pack_bytes((w[r] >> 7) & 0x01010101u & ~bytes_cool(w[r])) << (4 * r);
     hotpend &= valid;
     unsigned nearA = 0;  // bit q: a Moore neighbour of voxel v0 + q is mushy or cool liquid
-    if (hotpend) {
-      if (d.p.nx % PT == 0 && nq == PT) {
-        int i, j, k;
-        decode(d, v0, i, j, k);
-        for (int dz = -1; dz <= 1; ++dz) {
-          const int z = k + dz;
-          if (z < 0 || z >= d.p.nz) continue;
-          for (int dy = -1; dy <= 1; ++dy) {
-            const int y = j + dy;
-            if (y < 0 || y >= d.p.ny) continue;
-            const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * d.p.nx;
-            const uint4 u = *reinterpret_cast<const uint4*>(row + i);
-            const unsigned uw[4] = {u.x, u.y, u.z, u.w};
-            unsigned am = 0;  // bit q + 1: voxel i + q of the row is mushy or cool liquid
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const unsigned x = uw[r];
-              const unsigned lo = x & 0x01010101u, hi = (x >> 1) & 0x01010101u, hb = (x >> 7) & 0x01010101u;
-              const unsigned a4 = (hi & ~lo) | (lo & ~hi & ~hb);
-#pragma unroll
-              for (int q = 0; q < 4; ++q) am |= ((a4 >> (8 * q)) & 1u) << (4 * r + q + 1);
-            }
-            auto edge = [](uint8_t sn) { const int st = sn & 3; return st == 2 || (st == 1 && !(sn & 0x80)); };
-            if (i > 0 && edge(row[i - 1])) am |= 1u;
-            if (i + PT < d.p.nx && edge(row[i + PT])) am |= 1u << (PT + 1);
-            nearA |= am | (am >> 1) | (am >> 2);
-          }
-        }
-      } else {
-        for (unsigned m = hotpend; m; m &= m - 1) {
-          const int q = __builtin_ctz(m);
-          if (hot_voxel_active(d, v0 + q)) nearA |= 1u << q;
-        }
-      }
-    }
+    if (hotpend) nearA = moore_marks(d, v0, run_edges(d, v0), bytes_cool);
     unsigned nw[4];
     bool changed = false;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const unsigned x = w[r];
       const unsigned lo = x & 0x01010101u, hi = (x >> 1) & 0x01010101u, hb = (x >> 7) & 0x01010101u;
-      unsigned vb = 0, nb = 0;  // bytes of this word inside the domain; hot bytes with an active neighbour
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        vb |= ((valid >> (4 * r + q)) & 1u) << (8 * q);
-        nb |= (((hotpend & nearA) >> (4 * r + q)) & 1u) << (8 * q);
-      }
+      // bytes of this word inside the domain; hot bytes with an active neighbour
+      const unsigned vb = ((valid >> (4 * r)) & 15u) * 0x204081u & 0x01010101u;
+      const unsigned nb = (((hotpend & nearA) >> (4 * r)) & 15u) * 0x204081u & 0x01010101u;
       const unsigned mu = hi & ~lo & vb, lq = lo & ~hi & vb;
       const unsigned ac = mu | (lq & ~hb) | nb;
       nw[r] = (x & ~0x40404040u) | (ac << 6);
       changed = changed || nw[r] != x;
       na += __popc(ac);
       nm += __popc(mu);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) liq |= ((lq >> (8 * q)) & 1u) << (4 * r + q);
+      liq |= pack_bytes(lq) << (4 * r);
     }
     if (changed) {
       if (nq == PT) {
