@@ -21,8 +21,8 @@
 // 2 (s - s*) s (1 - s) / width per voxel and step; it is contracted with dT/dtheta, whose
 // four components come from the same quadrature nodes (dT/dP = (T - T0)/P, dT/deta = (T - T0)/eta,
 // df/dv = f 2 dx (t - tau) / D1, df/dsigma = f (-2 sigma / A + 4 sigma (dx^2 + dy^2) / D1^2)).
-// FP32 arithmetic with FP32 accumulation per thread and per block; an FP64 instantiation of
-// the forward serves finite differences.
+// FP32 products on the matrix cores, FP64 sums over a thread's tiles and a block; the forward in FP64
+// serves finite differences.
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -36,24 +36,26 @@ namespace {
 
 thread_local unsigned long long g_last_evals = 0;
 
-template <typename F, bool GRAD, bool PRUNE>
+template <typename F, bool GRAD>
 int run(const amcafe_heat_desc* d, int nb, const double* theta, const double* target, int step0, int nsteps,
         double* loss, double* grad, float* ms, char* err, int errlen) {
-  const size_t nblk = (size_t)n_blocks(d);
-  std::vector<Src<F>> hs;
-  sources<F>(nb, theta, target, hs);
-  Bufs<F> B = {nullptr, nullptr, nullptr, nullptr};
-  HCHECK(hipMalloc(&B.src, sizeof(Src<F>) * 2 * nb));
-  HCHECK(hipMalloc(&B.part, sizeof(F) * 5 * nblk * nb));
-  HCHECK(hipMalloc(&B.out, sizeof(F) * 5 * nb));
-  HCHECK(hipMalloc(&B.evals, sizeof(unsigned long long)));
-  HCHECK(hipMemcpy(B.src, hs.data(), sizeof(Src<F>) * 2 * nb, hipMemcpyHostToDevice));
-  HCHECK(hipMemset(B.evals, 0, sizeof(unsigned long long)));
+  const Shape sp = shape_of<F>(d);
+  const size_t nblk = (size_t)sp.groups * sp.runs;
+  std::vector<Src> hs;
+  sources(nb, theta, target, hs);
+  // one allocation: sources and the evaluation counter (one upload), block slots, sums
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  const size_t nsrc = sizeof(Src) * 2 * (size_t)nb, at_part = up(nsrc + 8), at_out = at_part + up(sizeof(F) * 5 * nblk * nb);
+  hs.push_back({0, 0, 0, 0});
+  unsigned char* base = nullptr;
+  HCHECK(hipMalloc(&base, at_out + sizeof(F) * 5 * (size_t)nb));
+  const Bufs<F> B = {(Src*)base, (F*)(base + at_part), (F*)(base + at_out), (unsigned long long*)(base + nsrc)};
+  HCHECK(hipMemcpy(base, hs.data(), nsrc + 8, hipMemcpyHostToDevice));
   hipEvent_t e0, e1;
   HCHECK(hipEventCreate(&e0));
   HCHECK(hipEventCreate(&e1));
   HCHECK(hipEventRecord(e0, 0));
-  launch_all<F, GRAD, PRUNE>(d, nb, B, step0, nsteps, 0);
+  launch_all<F, GRAD>(d, nb, B, step0, nsteps, 0);
   HCHECK(hipGetLastError());
   HCHECK(hipEventRecord(e1, 0));
   std::vector<F> h(5 * (size_t)nb);
@@ -63,10 +65,7 @@ int run(const amcafe_heat_desc* d, int nb, const double* theta, const double* ta
   HCHECK(hipEventElapsedTime(&el, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  HCHECK(hipFree(B.src));
-  HCHECK(hipFree(B.part));
-  HCHECK(hipFree(B.out));
-  HCHECK(hipFree(B.evals));
+  HCHECK(hipFree(base));
   results<F>(nb, h, GRAD, loss, grad);
   if (ms) *ms = el;
   return 0;
@@ -78,8 +77,8 @@ int run(const amcafe_heat_desc* d, int nb, const double* theta, const double* ta
 // mode 0: FP32 loss, 1: FP32 loss and gradient, 2: FP64 loss (finite differences, no pruning)
 extern "C" int amcd_heat(const amcafe_heat_desc* d, int nb, const double* theta, const double* target, int step0,
                          int nsteps, int mode, double* loss, double* grad, float* ms, char* err, int errlen) {
-  if (mode == 0) return run<float, false, true>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
-  if (mode == 1) return run<float, true, true>(d, nb, theta, target, step0, nsteps, loss, grad, ms, err, errlen);
-  return run<double, false, false>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
+  if (mode == 0) return run<float, false>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
+  if (mode == 1) return run<float, true>(d, nb, theta, target, step0, nsteps, loss, grad, ms, err, errlen);
+  return run<double, false>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
 }
 extern "C" unsigned long long amcd_heat_last_evals(void) { return g_last_evals; }

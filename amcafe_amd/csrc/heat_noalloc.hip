@@ -16,8 +16,10 @@ using namespace amcafe_heat;
 // the first segment overwrites every block slot.  Host code never passes the array's name to
 // a kernel or a copy (on the host it is only a stand-in): it uses the device address that
 // hipGetSymbolAddress returns for the current device, fetched once per device.
+// A call is accepted by its share at 20 bytes per 256 voxels and instance; the array holds twice
+// that, for domains one voxel long (see Shape).
 constexpr size_t kScratchBytes = 8u << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[2 * kScratchBytes];
 
 namespace {
 
@@ -27,9 +29,10 @@ static std::mutex g_scratch_mu;
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// scratch bytes a call needs: sources, block slots, sums, counter
+// scratch bytes a call is accounted: sources, sums of 256 voxels each, sums, counter
 size_t noalloc_bytes(const amcafe_heat_desc* d, int nb) {
-  return align256(sizeof(Src<float>) * 2 * (size_t)nb) + align256(sizeof(float) * 5 * (size_t)n_blocks(d) * nb) +
+  const size_t nblk = ((size_t)d->nX[0] * d->nX[1] * d->nX[2] + 255) / 256;
+  return align256(4 * sizeof(float) * 2 * (size_t)nb) + align256(sizeof(float) * 5 * nblk * nb) +
          align256(sizeof(float) * 5 * (size_t)nb) + align256(sizeof(unsigned long long));
 }
 
@@ -57,19 +60,20 @@ int run_noalloc(const amcafe_heat_desc* d, int nb, const double* theta, const do
     }
     base = (unsigned char*)g_scratch_ptr[dev];
   }
-  std::vector<Src<float>> hs;
-  sources<float>(nb, theta, target, hs);
+  const Shape sp = shape_of<float>(d);
+  std::vector<Src> hs;
+  sources(nb, theta, target, hs);
   Bufs<float> B;
   size_t off = 0;
-  B.src = (Src<float>*)(base + off);
-  off += align256(sizeof(Src<float>) * 2 * (size_t)nb);
+  B.src = (Src*)(base + off);
+  off += align256(sizeof(Src) * 2 * (size_t)nb);
   B.part = (float*)(base + off);
-  off += align256(sizeof(float) * 5 * (size_t)n_blocks(d) * nb);
+  off += align256(sizeof(float) * 5 * (size_t)sp.groups * sp.runs * nb);
   B.out = (float*)(base + off);
   off += align256(sizeof(float) * 5 * (size_t)nb);
   B.evals = nullptr;
-  HCHECK(hipMemcpy(B.src, hs.data(), sizeof(Src<float>) * 2 * nb, hipMemcpyHostToDevice));
-  launch_all<float, true, true>(d, nb, B, step0, nsteps, 0);
+  HCHECK(hipMemcpy(B.src, hs.data(), sizeof(Src) * 2 * nb, hipMemcpyHostToDevice));
+  launch_all<float, true>(d, nb, B, step0, nsteps, 0);
   HCHECK(hipGetLastError());
   std::vector<float> h(5 * (size_t)nb);
   HCHECK(hipMemcpy(h.data(), B.out, sizeof(float) * 5 * nb, hipMemcpyDeviceToHost));

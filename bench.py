@@ -157,10 +157,10 @@ def adjoint_cost(fd_steps=2000):
     if fd_steps != 2000:
         _, grad, _ = f.loss_grad_f32(start, 0, fd_steps)
     rel = [abs(g - d) / abs(d) for g, d in zip(grad, fd)]
-    # FP32 operations per evaluated voxel-step, counted in the kernel's source: per quadrature
-    # node 6 for the field and 6 for the target's (x offset, square, scale, exp, weight, sum),
-    # 10 more for the two gradient sums; 25 nodes, plus the indicator and accumulation per step
-    ops_f, ops_g = 25 * 12 + 12, 25 * 22 + 20
+    # FP32 operations per evaluated voxel-step, counted in the kernel's source: 26 (padded) nodes
+    # of a product and a sum for the field and the target's, three more for the gradient's sums, plus
+    # the indicators and accumulation (the columns' exponentials, shared by 128 rows, are not counted)
+    ops_f, ops_g = 26 * 4 + 20, 26 * 10 + 30
     return {"workload": "c3_heat", "voxels": 256 * 256 * 64, "steps": 2000, "dtype": "f32",
             "loss": loss, "forward_ms": round(ms_f, 2), "forward_and_adjoint_ms": round(ms_g, 2),
             "cost_ratio": round(ms_g / ms_f, 3), "wall_forward_s": round(tf, 3), "wall_adjoint_s": round(tg, 3),
