@@ -2,24 +2,25 @@
 // the internal launcher API declared in amcafe_dev.h.
 //
 // One step of one or many independent domains ("instances") runs as:
+//   k_step_in          the step's records from the pinned staging area
 //   k_temperature      TempField::AnalyticTempCurr (S/TempField.C:139-217), optionally
-//                      fused with SetLiquid3 (S/VoxelsCA.C:1098-1116); k_temp_commit
-//                      records the laser plane the field now matches.  (k_easm: the
-//                      EASM temperature, S/TempField.C:79-137, when asked for.)
+//                      fused with SetLiquid3 (S/VoxelsCA.C:1098-1116).  (k_easm: the
+//                      EASM temperature, S/TempField.C:79-137, when asked for;
+//                      k_temp_commit after a temperature on its own.)
 //   k_setliquid        SetLiquid3 alone, when the temperature was a separate call
 //   k_solid_to_mushy   ConvertSolid1(1) (S/VoxelsCA.C:780-797)
 //   k_active_flags     active-set membership (S/VoxelsCA.C:262-273) + per-block counts
-//   k_scan_chunks,     two-level exclusive scan of the block counts
-//   k_scan
+//   k_scan             two-level exclusive scan of the block counts, the step's loop state
 //   k_compact          ordered active list, voxel->active map, gathers, ruq draws
-//                      (S/VoxelsCA.C:274-303, 336-380); k_loop_rng seeds the loop's engine
+//                      (S/VoxelsCA.C:274-303, 336-380)
 //   k_active_setup     active-neighbour table (S/VoxelsCA.C:304-335) and growing list;
 //   k_grow_lists       the growing cells' sorted candidate lists (the per-pair part of
 //                      S/VoxelsCA.C:386-445) with each entry's capture re-centring
 //   k_event_loop       the serial capture/nucleation loop (S/VoxelsCA.C:381-610), one
 //                      workgroup per instance, FP64 throughout
-//   k_scatter          active arrays back to the grid (S/VoxelsCA.C:633-643)
-//   k_mushy_to_solid   ConvertSolid1(0) over the active cells (S/VoxelsCA.C:739-758)
+//   k_finish           active arrays back to the grid (S/VoxelsCA.C:633-643) and
+//                      ConvertSolid1(0) over the active cells (S/VoxelsCA.C:739-758)
+//   k_step_out         the output records to the pinned staging area
 // Per-voxel passes take runs of 16 voxels per thread (one 16-byte state load).  Layer
 // kernels: k_voronoi, k_site_rank, k_write_layer (base plate and powder layers,
 // S/BasePlate.C, S/VoxelsCA.C AddLayer1/CleanLayer); k_grain_presence, k_remap (grain
@@ -97,8 +98,11 @@ struct LoopState {
   int zhot0, zhot1;  // z planes the last temperature evaluation could have melted
   // T holds the analytic field of a laser plane at lz_prev (tvalid = 1): every voxel is xi
   // where its hot flag (vs bit 7) is set, else T0 above lz_prev and tS below it
-  int tvalid, pad1;
+  int tvalid;
+  int fin;      // the step's loop has finished: its results may go to the grid
   double lz_prev;
+  int zpar;     // which half of zliq the last active-set pass wrote
+  int chunks;   // chunks of the active-set scan that are done
 };
 
 // One entry of a growing cell's candidate list: everything the capture loop reads of it in one
@@ -147,7 +151,9 @@ struct Inst {
   uint8_t* bj;
   uint8_t* build;  // VoxelsCA::Build (changes only where the driver calls SetBuild)
   int* amap;
-  unsigned* zliq;  // per z plane: bit 0 = had liquid at the last active-set pass (or unknown)
+  // per z plane: bit 0 = had liquid at the last active-set pass (or unknown); two halves of nz planes,
+  // the pass writes the one that ls->zpar does not name, which is clear
+  unsigned* zliq;
   int *bcA, *bcM;  // per-ZB-block counts -> exclusive offsets within chunks of 1024 blocks
   int *chA, *chM;  // per chunk: totals -> exclusive offsets
   // active list
@@ -202,6 +208,29 @@ __host__ __device__ static inline unsigned int lcg_pow(unsigned long long e) {  
 __host__ __device__ static inline unsigned int rng_back(unsigned int x) {
   const unsigned long long inv = 1407677000ull;
   return mod_m(mod_m((unsigned long long)x * inv) * inv);
+}
+// 16807^(2 d 256^q) mod m: digit q (base 256) of a cell's index, so that the engine is at a cell's two
+// outputs after four products (by squaring, up to 18 cells' index bits took as many dependent pairs)
+struct LcgTable {
+  unsigned p[4][256];
+};
+constexpr LcgTable lcg_table() {
+  LcgTable t = {};
+  unsigned long long base = 16807ull * 16807ull % MINSTD_M;
+  for (int q = 0; q < 4; ++q) {
+    unsigned long long x = 1;
+    for (int d = 0; d < 256; ++d) {
+      t.p[q][d] = (unsigned)x;
+      x = x * base % MINSTD_M;
+    }
+    base = x;
+  }
+  return t;
+}
+__constant__ LcgTable kLcg = lcg_table();
+__device__ static inline unsigned lcg_skip_cells(unsigned x, unsigned a) {  // x 16807^(2a)
+  for (int q = 0; q < 4 && (a >> (8 * q)) != 0; ++q) x = mod_m((unsigned long long)x * kLcg.p[q][(a >> (8 * q)) & 255u]);
+  return x;
 }
 __host__ __device__ static inline unsigned int lcg_seed(unsigned long long s) {
   unsigned int x = (unsigned int)(s % MINSTD_M);
@@ -616,7 +645,8 @@ __global__ __launch_bounds__(GB) void k_solid_to_mushy(Inst* I, const int* bstar
   const int h0 = d.ls->zhot0, h1 = d.ls->zhot1;
   const int zb0 = b0 / d.nxy, zb1 = (bend - 1) / d.nxy;
   bool any = false;
-  for (int z = max(0, zb0 - 1); z <= min(nz - 1, zb1 + 1); ++z) any = any || (d.zliq[z] & 1u) || (z >= h0 && z <= h1);
+  const unsigned* zliq = d.zliq + (size_t)d.ls->zpar * nz;
+  for (int z = max(0, zb0 - 1); z <= min(nz - 1, zb1 + 1); ++z) any = any || (zliq[z] & 1u) || (z >= h0 && z <= h1);
   if (!any) return;
   // A solid voxel with a liquid Moore neighbour turns mushy.  Each thread takes 16 consecutive
   // voxels and reads the nine rows around them (moore_marks).  Liquid voxels are not changed by
@@ -644,12 +674,6 @@ __global__ __launch_bounds__(GB) void k_solid_to_mushy(Inst* I, const int* bstar
   }
 }
 
-// The per-plane liquid flags are rebuilt by every active-set pass.
-__global__ void k_zliq_clear(Inst* I, const amcd_step* S) {
-  const Inst& d = I[blockIdx.x];
-  if (S[blockIdx.x].skip) return;
-  for (int z = threadIdx.x; z < d.p.nz; z += blockDim.x) d.zliq[z] = 0u;
-}
 // Active set: {mushy} U {liquid below tL} U {neighbours at or above tL of those}.
 // Writes bit 6 of vs and the per-block (ZB voxels) counts of active and mushy cells.
 // One wave per block of ZB voxels (four per workgroup), 16 consecutive voxels per thread,
@@ -714,6 +738,7 @@ __global__ __launch_bounds__(256) void k_active_flags(Inst* I, const int* bstart
   // planes holding liquid now (for the next step's solid->mushy pass): one atomic per
   // wave and plane, and none once the flag is seen set.  A run of 16 spans at most two
   // planes unless a plane holds fewer than 16 voxels.
+  unsigned* zliq = d.zliq + (size_t)(1 - d.ls->zpar) * d.p.nz;
   int lp0 = -1, lp1 = -1;
   if (liq) {
     lp0 = (v0 + __builtin_ctz(liq)) / d.nxy;
@@ -721,7 +746,7 @@ __global__ __launch_bounds__(256) void k_active_flags(Inst* I, const int* bstart
     if (d.nxy < PT)
       for (unsigned m = liq; m; m &= m - 1) {
         const int kz = (v0 + __builtin_ctz(m)) / d.nxy;
-        if (!(d.zliq[kz] & 1u)) atomicOr(&d.zliq[kz], 1u);
+        if (!(zliq[kz] & 1u)) atomicOr(&zliq[kz], 1u);
       }
   }
   for (int pass = 0; pass < 2; ++pass) {
@@ -731,7 +756,7 @@ __global__ __launch_bounds__(256) void k_active_flags(Inst* I, const int* bstart
       const int leader = __builtin_ctzll(pend);
       const int zl = __builtin_amdgcn_readlane(pz, leader);
       pend &= ~__ballot(pz == zl);
-      if (lane == leader && !(d.zliq[zl] & 1u)) atomicOr(&d.zliq[zl], 1u);
+      if (lane == leader && !(zliq[zl] & 1u)) atomicOr(&zliq[zl], 1u);
     }
   }
   for (int o = 32; o >= 1; o >>= 1) {
@@ -744,16 +769,22 @@ __global__ __launch_bounds__(256) void k_active_flags(Inst* I, const int* bstart
   }
 }
 
-// Exclusive scan of the per-block counts in two levels: chunks of 1024 blocks scanned
-// by one workgroup each (offsets within the chunk, chunk totals), then one workgroup
-// per instance over the chunk totals.
-__global__ __launch_bounds__(1024) void k_scan_chunks(Inst* I, const int* cstart, int ninst) {
-  __shared__ int wa[16], wm[16];
+// Exclusive scan of the per-block counts in two levels, and the step's loop state: chunks of 1024
+// blocks scanned by one workgroup each (offsets within the chunk, chunk totals); the instance's last
+// chunk to be done scans the totals.  It also seeds the loop's engine (after the Na cells' two
+// draws each, S/VoxelsCA.C:380), takes over the laser plane of the temperature (`commit`) and swaps
+// the liquid-plane marks.  A pass of a few microseconds that is launch latency, so everything
+// that is one workgroup's work between the flags and the compaction is in it: as five launches
+// (chunks, totals, engine, laser plane, marks) it took 23 us of a step.
+__global__ __launch_bounds__(1024) void k_scan(Inst* I, const int* cstart, int ninst, const amcd_step* S, amcd_out* O,
+                                               int commit) {
+  __shared__ int wa[16], wm[16], last;
   const int ii = find_inst(cstart, ninst, blockIdx.x);
   const Inst& d = I[ii];
-  const int c = blockIdx.x - cstart[ii];
+  const int c = blockIdx.x - cstart[ii], nc = cstart[ii + 1] - cstart[ii];
   const int b = c * 1024 + (int)threadIdx.x;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  LoopState* ls = d.ls;
   int a = 0, m = 0;
   if (b < d.nblkZ) {
     a = d.bcA[b];
@@ -782,43 +813,51 @@ __global__ __launch_bounds__(1024) void k_scan_chunks(Inst* I, const int* cstart
     d.bcM[b] = pm + im - m;
   }
   if (threadIdx.x == 1023) {
-    d.chA[c] = pa + ia;
-    d.chM[c] = pm + im;
+    __hip_atomic_store(&d.chA[c], pa + ia, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&d.chM[c], pm + im, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // every chunk's totals are there when the count is complete
+    last = nc == 1 || __hip_atomic_fetch_add(&ls->chunks, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nc - 1;
   }
-}
-__global__ __launch_bounds__(1024) void k_scan(Inst* I, const amcd_step* S, amcd_out* O) {
-  __shared__ int sA[1024], sM[1024];
-  const Inst& d = I[blockIdx.x];
-  const int nc = (d.nblkZ + 1023) / 1024, t = threadIdx.x;
-  const int per = (nc + 1023) / 1024;
-  const int c0 = t * per, c1 = min(nc, c0 + per);
-  int a = 0, m = 0;
-  for (int c = c0; c < c1; ++c) {
-    a += d.chA[c];
-    m += d.chM[c];
-  }
-  sA[t] = a;
-  sM[t] = m;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {  // Hillis-Steele inclusive scan
-    int xa = t >= off ? sA[t - off] : 0, xm = t >= off ? sM[t - off] : 0;
+  if (!last) return;
+  const amcd_step st = S[ii];
+  if (!st.skip) {
+    const int zp = ls->zpar;
+    for (int z = threadIdx.x; z < d.p.nz; z += 1024) d.zliq[(size_t)zp * d.p.nz + z] = 0u;
     __syncthreads();
-    sA[t] += xa;
-    sM[t] += xm;
-    __syncthreads();
+    if (threadIdx.x == 0) {
+      ls->zpar = 1 - zp;
+      if (commit) {
+        ls->tvalid = 1;
+        ls->lz_prev = st.lz;
+      }
+    }
   }
-  int ra = sA[t] - a, rm = sM[t] - m;
-  for (int c = c0; c < c1; ++c) {
-    const int va = d.chA[c], vm = d.chM[c];
-    d.chA[c] = ra;
-    d.chM[c] = rm;
-    ra += va;
-    rm += vm;
+  if (w != 0) return;
+  // the chunk totals, 64 at a time
+  int Na = 0, Nm = 0;
+  for (int c0 = 0; c0 < nc; c0 += 64) {
+    const bool in = c0 + lane < nc;
+    const int va = in ? __hip_atomic_load(&d.chA[c0 + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    const int vm = in ? __hip_atomic_load(&d.chM[c0 + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    int xa = va, xm = vm;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int ta = __shfl_up(xa, o), tm = __shfl_up(xm, o);
+      if (lane >= o) {
+        xa += ta;
+        xm += tm;
+      }
+    }
+    if (in) {
+      d.chA[c0 + lane] = Na + xa - va;
+      d.chM[c0 + lane] = Nm + xm - vm;
+    }
+    Na += __shfl(xa, 63);
+    Nm += __shfl(xm, 63);
   }
-  if (t == 1023) {
-    int Na = sA[1023], Nm = sM[1023];
-    if (S[blockIdx.x].skip) Na = Nm = 0;
-    LoopState* ls = d.ls;
+  if (lane == 0) {
+    if (st.skip) Na = Nm = 0;
+    ls->chunks = 0;
     ls->Na = Na;
     ls->nmushy0 = Nm;
     ls->nslots = 0;
@@ -829,17 +868,20 @@ __global__ __launch_bounds__(1024) void k_scan(Inst* I, const amcd_step* S, amcd
     ls->events = ls->captures = ls->nucs = 0;
     ls->pool_used = 0;
     ls->pending = 0;
-    ls->done = 0;
-    ls->nGrain = S[blockIdx.x].nGrain;
-    amcd_out& o = O[blockIdx.x];
+    ls->fin = 0;
+    ls->done = st.skip || Na > d.acap;
+    ls->nGrain = st.nGrain;
+    if (!ls->done) {
+      ls->rng = lcg_skip_cells(lcg_seed(30ull * (unsigned long long)st.tInd + d.p.seed1), (unsigned)Na);
+      ls->draws = 2ll * Na;
+    }
+    amcd_out& o = O[ii];
     o.n_active = Na;
     o.n_mushy0 = Nm;
     if (Na > d.acap) {
       o.overflow = 1;
       o.status = -2;
-      ls->done = 1;
     }
-    if (S[blockIdx.x].skip) ls->done = 1;
   }
 }
 
@@ -918,14 +960,16 @@ __global__ __launch_bounds__(256) void k_compact(Inst* I, const int* bstart, int
     d.aVox[a] = v;
     d.amap[v] = a;
     d.aVS[a] = d.vs[v] & 3;
-    d.aG[a] = d.gid[v];
     d.aT[a] = d.T[v];
-    d.aExt[a] = d.ext[v];
-    d.aCx[a] = d.cx[v];
-    d.aCy[a] = d.cy[v];
-    d.aCz[a] = d.cz[v];
+    if (mushy) {  // (a liquid cell's are written when it is captured)
+      d.aG[a] = d.gid[v];
+      d.aExt[a] = d.ext[v];
+      d.aCx[a] = d.cx[v];
+      d.aCy[a] = d.cy[v];
+      d.aCz[a] = d.cz[v];
+    }
     d.aScan[a] = mushy ? m0 + emt + __popc(mmt & ((1u << q) - 1)) : -1;
-    const unsigned int x1 = mod_m((unsigned long long)x0 * lcg_pow(2ull * a + 1));
+    const unsigned int x1 = lcg_next(lcg_skip_cells(x0, (unsigned)a));
     const unsigned int x2 = lcg_next(x1);
     d.ruq[a] = (canonical(x1, x2) - .5) * d.p.dx / 100.;
   }
@@ -2792,7 +2836,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
     ls->rng = sh.cur;
     ls->draws += 2ll * es.nd;
     ls->nslots = ns;
-    ls->done = status == 0 ? 1 : 0;
+    ls->done = ls->fin = status == 0 ? 1 : 0;
     amcd_out& o = O[blockIdx.x];
     o.status = status;
     o.n_events = es.events;
@@ -2810,59 +2854,73 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
   }
 }
 
-// Active arrays back to the grid (S/VoxelsCA.C:633-643).
-__global__ __launch_bounds__(GB) void k_scatter(Inst* I, const int* astart, int ninst) {
+// The step's results back to the grid (S/VoxelsCA.C:633-643) and ConvertSolid1(0)
+// (S/VoxelsCA.C:739-758): mushy -> solid when every Moore neighbour is mushy or solid.  Every mushy
+// voxel is in the active list, so only those are visited, and so is every liquid neighbour of one: a
+// neighbour whose state in the grid is liquid has been captured when its active state is mushy,
+// whether its own thread has written the grid yet or not, and a state that has been written (2, or
+// 3 from 2) counts the same.  One pass instead of two: only what a step changes is written (the
+// octahedra of captured voxels, half-diagonals of mushy ones), 6.9 + 9.1 -> 12.8 us for the 512x512x128
+// raster.  Also clears the voxel -> active map for the next step.  The pass leaves the grid as it is
+// while the step will be run again (an overflow in any instance) or the loop be resumed; run a second
+// time it writes the same values.
+__global__ __launch_bounds__(GB) void k_finish(Inst* I, const int* astart, int ninst, const amcd_out* O) {
+  int again = 0;
+  for (int q = threadIdx.x; q < ninst; q += GB) again |= O[q].overflow;
+  if (__syncthreads_or(again)) return;
   int ii = find_inst(astart, ninst, blockIdx.x);
   const Inst d = I[ii];  // a copy: stores in the loops cannot alias it
-  int a = (blockIdx.x - astart[ii]) * GB + threadIdx.x;
-  if (d.ls->pending || a >= d.ls->Na || a >= d.acap) return;
-  int v = d.aVox[a];
-  d.vs[v] = (d.vs[v] & 0xC0) | d.aVS[a];
-  d.gid[v] = d.aG[a];
-  d.ext[v] = d.aExt[a];
-  d.cx[v] = d.aCx[a];
-  d.cy[v] = d.aCy[a];
-  d.cz[v] = d.aCz[a];
-}
-
-// ConvertSolid1(0) (S/VoxelsCA.C:739-758): mushy -> solid when every Moore neighbour
-// is mushy or solid.  Every mushy voxel is in the active list, so only those are
-// visited; in-place update is safe because 2 -> 3 keeps "neighbour >= 2" true.
-// Also clears the voxel -> active map for the next step.
-__global__ __launch_bounds__(GB) void k_mushy_to_solid(Inst* I, const int* astart, int ninst) {
-  int ii = find_inst(astart, ninst, blockIdx.x);
-  const Inst d = I[ii];  // a copy: stores in the loops cannot alias it
-  int a = (blockIdx.x - astart[ii]) * GB + threadIdx.x;
-  if (d.ls->pending || a >= d.ls->Na || a >= d.acap) return;
-  int v = d.aVox[a];
+  const int a = (blockIdx.x - astart[ii]) * GB + threadIdx.x;
+  if (!d.ls->fin || a >= d.ls->Na || a >= d.acap) return;
+  const int v = d.aVox[a];
   d.amap[v] = -1;
   if (d.aVS[a] != 2) return;
+  const uint8_t s0 = d.vs[v];
   int i, j, k;
   decode(d, v, i, j, k);
-  for (int dz = -1; dz <= 1; ++dz) {
-    int z = k + dz;
-    if (z < 0 || z >= d.p.nz) continue;
-    for (int dy = -1; dy <= 1; ++dy) {
-      int y = j + dy;
-      if (y < 0 || y >= d.p.ny) continue;
-      const uint8_t* row = d.vs + (size_t)z * d.nxy + (size_t)y * d.p.nx;
-      for (int dx = -1; dx <= 1; ++dx) {
-        int x = i + dx;
-        if (x < 0 || x >= d.p.nx || (dx == 0 && dy == 0 && dz == 0)) continue;
-        if ((row[x] & 3) < 2) return;
-      }
-    }
+  const int* nbr = d.aRow[a].nbr;
+  uint8_t sn[AMCD_NB];
+#pragma unroll
+  for (int q = 0; q < AMCD_NB; ++q) {  // (the nine rows' bytes side by side; outside the domain: solid)
+    const int qq = q < 13 ? q : q + 1, x = i + qq % 3 - 1, y = j + (qq / 3) % 3 - 1, z = k + qq / 9 - 1;
+    const bool in = x >= 0 && x < d.p.nx && y >= 0 && y < d.p.ny && z >= 0 && z < d.p.nz;
+    sn[q] = in ? d.vs[v + (qq / 9 - 1) * d.nxy + ((qq / 3) % 3 - 1) * d.p.nx + qq % 3 - 1] : 3;
   }
-  d.vs[v] = (d.vs[v] & 0xFC) | 3;
-  d.ext[v] = 0.0;
+  unsigned liq = 0, none = 0;
+#pragma unroll
+  for (int q = 0; q < AMCD_NB; ++q) {
+    liq |= ((sn[q] & 3) == 1 ? 1u : 0u) << q;
+    none |= (sn[q] & 3) == 0 ? 1u : 0u;
+  }
+  bool solid = none == 0;
+  for (; solid && liq != 0; liq &= liq - 1) {
+    const int n = nbr[__builtin_ctz(liq)];
+    solid = n >= 0 && d.aVS[n] == 2;
+  }
+  const uint8_t s1 = (s0 & 0xC0) | (solid ? 3 : 2);
+  if (s1 != s0) d.vs[v] = s1;
+  d.ext[v] = solid ? 0.0 : d.aExt[a];
+  if ((s0 & 3) == 1) {  // captured in this step
+    d.gid[v] = d.aG[a];
+    d.cx[v] = d.aCx[a];
+    d.cy[v] = d.aCy[a];
+    d.cz[v] = d.aCz[a];
+  }
 }
 
 // ---- per-layer helpers ---------------------------------------------------------------
 // After a host upload of vState: the "T >= tL" flag (bit 7) follows the device's current
 // temperature field, so SetLiquid3 still sees the caller's melt pool.
-// Fresh output records inside a captured step (a memset node is not used in graphs).
-__global__ void k_clear_outs(unsigned* o, int nwords) {
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < nwords; q += gridDim.x * blockDim.x) o[q] = 0u;
+// A step's records: in from the pinned staging area with fresh output records (`clear` words), and the
+// outputs back.  As kernels in the step's graph they cost 2 us each; as stream copies beside it, 10.
+__global__ void k_step_in(unsigned* steps, const unsigned* staged, int nwords, unsigned* outs, int clear) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nwords) steps[q] = staged[q];
+  if (q < clear) outs[q] = 0u;
+}
+__global__ void k_step_out(unsigned* staged, const unsigned* outs, int nwords) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nwords) staged[q] = outs[q];
 }
 __global__ void k_rehot(uint8_t* vs, const double* T, int N, double tL) {
   size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3033,9 +3091,9 @@ struct amcd_batch {
   size_t mark_cap = 0;
   std::vector<size_t> pool_off;
   hipEvent_t pool_ev = nullptr;  // the last staging copy (the staging area is rewritten after it)
-  // The driver's step as HIP graphs (AMCAFE_GRAPH=0 launches the stages one by one): the
-  // stages up to the capture loop, per capture tier, and the finishing pair; each is captured
-  // again when the block counts it was captured with change (capacity growth)
+  // The driver's step as HIP graphs (AMCAFE_GRAPH=0 launches the stages one by one): the stages up
+  // to the capture loop, per capture tier, and the finishing pass; each is captured again when the
+  // block counts it was captured with change (capacity growth)
   bool graphs = true;
   hipGraphExec_t gstep[6] = {};
   long long gstep_key[6] = {};
@@ -3164,7 +3222,7 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
         dalloc(b, &d.cy, Nn) || dalloc(b, &d.cz, Nn) || dalloc(b, &d.T, Nn) || dalloc(b, &d.bj, Nn) || dalloc(b, &d.build, Nn) ||
         dalloc(b, &d.amap, Nn) || dalloc(b, &d.bcA, (size_t)d.nblkZ) || dalloc(b, &d.bcM, (size_t)d.nblkZ) ||
         dalloc(b, &d.chA, (size_t)d.nblkZ / 1024 + 1) || dalloc(b, &d.chM, (size_t)d.nblkZ / 1024 + 1) ||
-        dalloc(b, &d.zliq, (size_t)p[i].nz) || dalloc(b, &d.ls, 1)) {
+        dalloc(b, &d.zliq, 2 * (size_t)p[i].nz) || dalloc(b, &d.ls, 1)) {
       snprintf(err, errlen, "%s", g_dev_err.c_str());
       amcd_destroy(b);
       return -1;
@@ -3183,7 +3241,7 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
     zero(d.T, 0, Nn * 8);
     zero(d.bj, 0, Nn);
     zero(d.build, 0, Nn);
-    zero(d.zliq, 0xff, (size_t)p[i].nz * 4);  // unknown: every plane may hold liquid
+    zero(d.zliq, 0xff, (size_t)p[i].nz * 8);  // unknown: every plane may hold liquid
     zero(d.amap, 0xff, Nn * 4);
     zero(d.ls, 0, sizeof(LoopState));
     if (me != hipSuccess) {
@@ -3277,7 +3335,7 @@ int amcd_upload(amcd_batch* b, int i, const int* gid, const int* vstate, const d
   if (vstate) {
     for (size_t v = 0; v < N; ++v) tmp[v] = (uint8_t)(vstate[v] & 3);
     HIPT(hipMemcpy(d.vs, tmp.data(), N, hipMemcpyHostToDevice));
-    HIPT(hipMemset(d.zliq, 0xff, (size_t)d.p.nz * 4));
+    HIPT(hipMemset(d.zliq, 0xff, (size_t)d.p.nz * 8));
     HIPT(hipMemset(&d.ls->tvalid, 0, sizeof(int)));
     hipLaunchKernelGGL(k_rehot, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, b->stream, d.vs, d.T, d.N, d.p.tL);
     HIPT(hipGetLastError());
@@ -3428,7 +3486,22 @@ int amcd_reserve_grains(amcd_batch* b, int i, int need) { return ensure_grains(b
 
 static int put_steps(amcd_batch* b, const amcd_step* steps) {
   memcpy(b->h_steps, steps, sizeof(amcd_step) * b->n);
-  HIPT(hipMemcpyAsync(b->d_steps, b->h_steps, sizeof(amcd_step) * b->n, hipMemcpyHostToDevice, b->stream));
+  return 0;
+}
+// the staged step records to the device, with fresh output records when `clear`
+static int launch_step_in(amcd_batch* b, bool clear) {
+  static_assert(sizeof(amcd_step) % 4 == 0 && sizeof(amcd_out) % 4 == 0, "records copied as words");
+  const int ns = (int)(sizeof(amcd_step) / 4) * b->n, no = clear ? (int)(sizeof(amcd_out) / 4) * b->n : 0;
+  hipLaunchKernelGGL(k_step_in, dim3((std::max(ns, no) + 255) / 256), dim3(256), 0, b->stream, (unsigned*)b->d_steps,
+                     (const unsigned*)b->h_steps, ns, (unsigned*)b->d_outs, no);
+  HIPT(hipGetLastError());
+  return 0;
+}
+static int launch_step_out(amcd_batch* b) {
+  const int no = (int)(sizeof(amcd_out) / 4) * b->n;
+  hipLaunchKernelGGL(k_step_out, dim3((no + 255) / 256), dim3(256), 0, b->stream, (unsigned*)b->h_outs,
+                     (const unsigned*)b->d_outs, no);
+  HIPT(hipGetLastError());
   return 0;
 }
 
@@ -3440,7 +3513,11 @@ static int run_temperature(amcd_batch* b, int setliquid) {
   int nb = b->bstartT[b->n];
   hipLaunchKernelGGL(k_temperature, dim3(nb), dim3(GB), 0, b->stream, b->d_inst, b->d_bstartT, b->n, b->d_steps,
                      b->d_outs, setliquid);
-  hipLaunchKernelGGL(k_temp_commit, dim3(b->n), dim3(64), 0, b->stream, b->d_inst, b->d_steps, 1);
+  HIPT(hipGetLastError());
+  return 0;
+}
+static int commit_temperature(amcd_batch* b, int valid) {  // (in the fused step the scan does it)
+  hipLaunchKernelGGL(k_temp_commit, dim3(b->n), dim3(64), 0, b->stream, b->d_inst, b->d_steps, valid);
   HIPT(hipGetLastError());
   return 0;
 }
@@ -3451,24 +3528,21 @@ static int invalidate_T(amcd_batch* b, int i) {
 }
 
 int amcd_temperature(amcd_batch* b, const amcd_step* steps) {
-  if (put_steps(b, steps)) return -1;
-  HIPT(hipMemsetAsync(b->d_outs, 0, sizeof(amcd_out) * b->n, b->stream));
-  return run_temperature(b, 0);
+  if (put_steps(b, steps) || launch_step_in(b, true) || run_temperature(b, 0)) return -1;
+  return commit_temperature(b, 1);
 }
 
 static int read_outs(amcd_batch* b, amcd_out* outs);
 int amcd_easm(amcd_batch* b, const amcd_step* steps, double Q, double layerT, amcd_out* outs,
               unsigned long long* n_evals) {
-  if (put_steps(b, steps)) return -1;
-  HIPT(hipMemsetAsync(b->d_outs, 0, sizeof(amcd_out) * b->n, b->stream));
+  if (put_steps(b, steps) || launch_step_in(b, true)) return -1;
   unsigned long long* dn = nullptr;
   HIPT(hipMalloc(&dn, sizeof(unsigned long long)));
   HIPT(hipMemsetAsync(dn, 0, sizeof(unsigned long long), b->stream));
   tmark(b, 0);
   hipLaunchKernelGGL(k_easm, dim3(b->bstartG[b->n]), dim3(GB), 0, b->stream, b->d_inst, b->d_bstartG, b->n,
                      b->d_steps, b->d_outs, Q, layerT, dn);
-  hipLaunchKernelGGL(k_temp_commit, dim3(b->n), dim3(64), 0, b->stream, b->d_inst, b->d_steps, 0);
-  HIPT(hipGetLastError());
+  if (commit_temperature(b, 0)) return -1;
   tmark(b, 1);
   unsigned long long hn = 0;
   HIPT(hipMemcpyAsync(&hn, dn, sizeof(hn), hipMemcpyDeviceToHost, b->stream));
@@ -3481,15 +3555,6 @@ int amcd_easm(amcd_batch* b, const amcd_step* steps, double Q, double layerT, am
   }
   if (n_evals) *n_evals = hn;
   return 0;
-}
-
-__global__ void k_loop_rng(Inst* I, const amcd_step* S) {
-  const Inst& d = I[blockIdx.x];
-  LoopState* ls = d.ls;
-  if (threadIdx.x != 0 || ls->done) return;
-  unsigned int x0 = lcg_seed(30ull * (unsigned long long)S[blockIdx.x].tInd + d.p.seed1);
-  ls->rng = mod_m((unsigned long long)x0 * lcg_pow(2ull * (unsigned long long)ls->Na));
-  ls->draws = 2ll * ls->Na;
 }
 
 static int launch_update(amcd_batch* b, bool fused_temperature) {
@@ -3505,14 +3570,12 @@ static int launch_update(amcd_batch* b, bool fused_temperature) {
   hipLaunchKernelGGL(k_solid_to_mushy, dim3(b->bstartS[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_bstartS, n,
                      b->d_steps);
   tmark(b, 2);
-  hipLaunchKernelGGL(k_zliq_clear, dim3(n), dim3(256), 0, b->stream, b->d_inst, b->d_steps);
   hipLaunchKernelGGL(k_active_flags, dim3(b->bstartF[n]), dim3(256), 0, b->stream, b->d_inst, b->d_bstartF, n,
                      b->d_steps);
-  hipLaunchKernelGGL(k_scan_chunks, dim3(b->cstart[n]), dim3(1024), 0, b->stream, b->d_inst, b->d_cstart, n);
-  hipLaunchKernelGGL(k_scan, dim3(n), dim3(1024), 0, b->stream, b->d_inst, b->d_steps, b->d_outs);
+  hipLaunchKernelGGL(k_scan, dim3(b->cstart[n]), dim3(1024), 0, b->stream, b->d_inst, b->d_cstart, n, b->d_steps,
+                     b->d_outs, fused_temperature ? 1 : 0);
   hipLaunchKernelGGL(k_compact, dim3(b->bstartF[n]), dim3(256), 0, b->stream, b->d_inst, b->d_bstartF, n,
                      b->d_steps);
-  hipLaunchKernelGGL(k_loop_rng, dim3(n), dim3(64), 0, b->stream, b->d_inst, b->d_steps);
   tmark(b, 3);
   HIPT(hipGetLastError());
   return 0;
@@ -3541,12 +3604,12 @@ static int launch_event_loop(amcd_batch* b) {
   }
 }
 
-static int read_outs(amcd_batch* b, amcd_out* outs) {
-  HIPT(hipMemcpyAsync(b->h_outs, b->d_outs, sizeof(amcd_out) * b->n, hipMemcpyDeviceToHost, b->stream));
+static int wait_outs(amcd_batch* b, amcd_out* outs) {
   HIPT(hipStreamSynchronize(b->stream));
   memcpy(outs, b->h_outs, sizeof(amcd_out) * b->n);
   return 0;
 }
+static int read_outs(amcd_batch* b, amcd_out* outs) { return launch_step_out(b) || wait_outs(b, outs); }
 
 // The active-cell block lists, sized by the capacities (idle threads exit, so no host round
 // trip is needed mid-step), uploaded when a capacity has changed.
@@ -3587,8 +3650,7 @@ static int launch_active(amcd_batch* b) { return prep_active(b) || launch_active
 
 static int launch_finish(amcd_batch* b) {
   const int n = b->n;
-  hipLaunchKernelGGL(k_scatter, dim3(b->astart[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_astart, n);
-  hipLaunchKernelGGL(k_mushy_to_solid, dim3(b->astart[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_astart, n);
+  hipLaunchKernelGGL(k_finish, dim3(b->astart[n]), dim3(GB), 0, b->stream, b->d_inst, b->d_astart, n, b->d_outs);
   tmark(b, 6);
   HIPT(hipGetLastError());
   return 0;
@@ -3681,24 +3743,15 @@ static void pick_tier(amcd_batch* b, const amcd_out* outs) {
   b->tier = std::max(t, b->min_tier);
 }
 
-// Capture of the step's stages into an executable graph: with `step` the output clear, the
-// temperature and state passes, the active-list and candidate-list passes and the capture loop
-// of the current tier; otherwise the scatter and mushy->solid pair.  (The step record's upload
-// and the outputs' download stay plain stream copies around the graph: as graph nodes they
-// made the step slower.)
-static int capture_graph(amcd_batch* b, bool step, bool fused, hipGraphExec_t* out) {
-  static_assert(sizeof(amcd_out) % 4 == 0, "outputs cleared as words");
-  const int n = b->n;
+// Capture of the step's stages into an executable graph: with `step` the step records in, the
+// temperature and state passes, the active-list and candidate-list passes and the capture loop of the
+// current tier; otherwise the results to the grid (of the instances whose loop has finished) and the
+// output records out.
+static int capture_graph(amcd_batch* b, bool step, hipGraphExec_t* out) {
   hipGraph_t g = nullptr;
   HIPT(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-  int rc = 0;
-  if (step) {
-    const int nw = (int)(sizeof(amcd_out) / 4) * n;
-    hipLaunchKernelGGL(k_clear_outs, dim3((nw + 255) / 256), dim3(256), 0, b->stream, (unsigned*)b->d_outs, nw);
-    rc = launch_update(b, fused) || launch_active_kernels(b);
-  } else {
-    rc = launch_finish(b);
-  }
+  const int rc = step ? launch_step_in(b, true) || launch_update(b, true) || launch_active_kernels(b)
+                      : launch_finish(b) || launch_step_out(b);
   const hipError_t e = hipStreamEndCapture(b->stream, &g);
   if (rc || e != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
@@ -3725,7 +3778,7 @@ static int launch_step_graph(amcd_batch* b) {
     g = nullptr;
   }
   if (!g) {
-    if (capture_graph(b, true, true, &g)) return -1;
+    if (capture_graph(b, true, &g)) return -1;
     b->gstep_key[t] = key;
   }
   HIPT(hipGraphLaunch(g, b->stream));
@@ -3739,7 +3792,7 @@ static int launch_finish_graph(amcd_batch* b) {
     b->gfin = nullptr;
   }
   if (!b->gfin) {
-    if (capture_graph(b, false, false, &b->gfin)) return -1;
+    if (capture_graph(b, false, &b->gfin)) return -1;
     b->gfin_key = key;
   }
   HIPT(hipGraphLaunch(b->gfin, b->stream));
@@ -3803,63 +3856,47 @@ int amcd_tuning(amcd_batch* b, int* list_cap, int* n_tunings, int* cells, float*
   return b->tuned ? 1 : 0;
 }
 
-// The step with its stages in graphs: one graph launch up to the capture loop's outputs, then,
-// when every instance has finished its loop, one for the finishing pair.  Suspensions (pool
-// refill, larger tier, wide bitmap) and capacity growth take the same host paths as the
-// stage-by-stage form.
-static int update_graph(amcd_batch* b, const amcd_step* steps, amcd_out* outs) {
-  if (put_steps(b, steps)) return -1;
-  for (int attempt = 0; attempt < 8; ++attempt) {
-    if (prep_active(b) || launch_step_graph(b) || read_outs(b, outs)) return -1;
-    bool ovf = false;
-    for (int i = 0; i < b->n; ++i) ovf = ovf || outs[i].overflow;
-    if (!ovf) break;
-    if (grow_active(b, outs)) return -1;
-  }
-  if (widen(b, outs) || regrow_tier(b, outs)) return -1;
-  bool pend = false;
-  for (int i = 0; i < b->n; ++i) pend = pend || outs[i].status == 1;
-  if (!pend) {
-    if (launch_finish_graph(b)) return -1;
-    HIPT(hipStreamSynchronize(b->stream));
-    pick_tier(b, outs);
-    if (maybe_autotune(b, outs)) return -1;
-  }
-  return 0;
+static bool all_finished(const amcd_batch* b, const amcd_out* outs) {
+  for (int i = 0; i < b->n; ++i)
+    if (outs[i].status != 0) return false;
+  return true;
 }
-
+// The step, as graphs (the driver's fused form) or stage by stage: per-stage timing needs events
+// between the stages, a tuning step runs the list pass several times, and the seam form keeps the
+// output records its temperature call wrote.  One synchronisation: the results of instances whose
+// loop has finished are in the grid when the output records are read.  Suspensions (pool refill,
+// larger tier, wide bitmap) take further launches, and the finishing pass then runs again (the same
+// values, for the instances that had finished).
 static int update_common(amcd_batch* b, const amcd_step* steps, amcd_out* outs, bool fused) {
-  // the driver's fused step runs as graphs; per-stage timing needs events between the stages,
-  // and the seam form keeps the output records its temperature call wrote: stage by stage
-  if (b->graphs && !b->timing && fused && !b->tune_pending) return update_graph(b, steps, outs);
+  const bool graph = b->graphs && !b->timing && fused && !b->tune_pending;
   if (put_steps(b, steps)) return -1;
   for (int attempt = 0; attempt < 8; ++attempt) {
-    if (fused || attempt > 0) {
-      // fresh output records; the temperature kernel sets any_melt
-      HIPT(hipMemsetAsync(b->d_outs, 0, sizeof(amcd_out) * b->n, b->stream));
+    if (graph) {
+      if (prep_active(b) || launch_step_graph(b) || launch_finish_graph(b) || wait_outs(b, outs)) return -1;
+    } else {
+      // A retry repeats the step's stages with the same temperature source: the fused form
+      // re-evaluates the same laser (idempotent), the seam form keeps the caller's field and
+      // re-applies SetLiquid3 to it (idempotent for the same T).
+      if (launch_step_in(b, fused || attempt > 0) || launch_update(b, fused) || launch_active(b) || launch_finish(b) ||
+          read_outs(b, outs))
+        return -1;
     }
-    // A retry repeats the step's stages with the same temperature source: the fused form
-    // re-evaluates the same laser (idempotent), the seam form keeps the caller's field and
-    // re-applies SetLiquid3 to it (idempotent for the same T).
-    if (launch_update(b, fused)) return -1;
-    if (launch_active(b)) return -1;
-    if (read_outs(b, outs)) return -1;
     bool ovf = false;
     for (int i = 0; i < b->n; ++i) ovf = ovf || outs[i].overflow;
     if (!ovf) break;
     if (grow_active(b, outs)) return -1;
   }
-  if (widen(b, outs) || regrow_tier(b, outs)) return -1;
-  bool pend = false;
-  for (int i = 0; i < b->n; ++i) pend = pend || outs[i].status == 1;
-  if (!pend) {
+  const bool finished = all_finished(b, outs);
+  if (!finished) {
+    if (widen(b, outs) || regrow_tier(b, outs)) return -1;
+    for (int i = 0; i < b->n; ++i)
+      if (outs[i].status == 1) return 0;  // (the caller refills the pool and resumes)
     if (launch_finish(b)) return -1;
     HIPT(hipStreamSynchronize(b->stream));
-    collect_timing(b);
-    pick_tier(b, outs);
-    if (maybe_autotune(b, outs)) return -1;
   }
-  return 0;
+  collect_timing(b);
+  pick_tier(b, outs);
+  return maybe_autotune(b, outs);
 }
 
 int amcd_update_voxels(amcd_batch* b, const amcd_step* steps, amcd_out* outs) {
@@ -3974,7 +4011,7 @@ int amcd_init_plate(amcd_batch* b, int i, int nzh, const double* xs, int ng) {
   hipLaunchKernelGGL(k_voronoi<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, b->stream, b->d_inst, i, 0,
                      nzh, dx, ng, nullptr, nullptr);
   HIPT(hipGetLastError());
-  HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 4, b->stream));
+  HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 8, b->stream));
   if (invalidate_T(b, i)) return -1;
   HIPT(hipStreamSynchronize(b->stream));
   HIPT(hipFree(dx));
@@ -4002,7 +4039,7 @@ int amcd_add_layer(amcd_batch* b, int i, int iz1, int ilaserLoc, int gbase, cons
   hipLaunchKernelGGL(k_write_layer, dim3((d.N + 255) / 256), dim3(256), 0, b->stream, b->d_inst, i, iz1, ilaserLoc,
                      gbase, lab, rank);
   HIPT(hipGetLastError());
-  HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 4, b->stream));
+  HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 8, b->stream));
   if (invalidate_T(b, i)) return -1;
   HIPT(hipMemcpyAsync(n_used, tot, sizeof(int), hipMemcpyDeviceToHost, b->stream));
   HIPT(hipStreamSynchronize(b->stream));

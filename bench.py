@@ -48,7 +48,7 @@ HBM_PEAK_GBS = 8000.0
 STAGES = ("temperature+SetLiquid3", "solid->mushy", "active list", "growing setup", "capture loop",
           "scatter+mushy->solid")
 KERNEL_NAMES = ("k_temperature", "k_solid_to_mushy", "k_active_flags/k_scan/k_compact", "k_active_setup",
-                "k_event_loop", "k_scatter/k_mushy_to_solid")
+                "k_event_loop", "k_finish")
 WORKLOADS = {
     "c1_raster": "512x512x128 voxels, dx 2.5 um, 4 layers of 30 um, 3-track bidirectional raster, "
                  "hatch 60 um, 90 deg rotation, 250 W, 1.0 m/s, FP64",
