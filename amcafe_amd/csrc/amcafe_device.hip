@@ -75,6 +75,22 @@ __device__ static inline double lane_f64(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// another lane's value by a DPP row operation
+template <int CTRL, int ROWS = 0xf>
+__device__ static inline int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ static inline float dpp(float v) {
+  return __int_as_float(dpp<CTRL, ROWS>(__float_as_int(v)));
+}
+template <int CTRL, int ROWS = 0xf>
+__device__ static inline double dpp(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)dpp<CTRL, ROWS>((int)b), hi = (unsigned)dpp<CTRL, ROWS>((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 #define ZB 1024     // voxels per compaction block (one wave, 16 per thread)
 #define GB 256      // threads per grid-wide block
 #define SB 4096     // voxels per solid->mushy block (GB threads, 16 voxels each)
@@ -423,13 +439,22 @@ __global__ void k_temp_commit(Inst* I, const amcd_step* S, int valid) {
 // -------------------------------------------------------------------------------------
 // TempField::EASM (S/TempField.C:79-137): the temperature of a Gaussian moving source with
 // 316L properties, Utilities::EASM_Temp_LG (S/Utilities.C:128-140).  Every voxel is an
-// independent FP64 fixed-point problem (FP64-VALU bound).
+// independent FP64 fixed-point problem: T -> (T + F(T))/2 with F the source integral, until a step is
+// at most 10 K, or 100 times.  The properties jump at 1660 K, so where F crosses that temperature
+// the iteration goes round for all 100 steps: 2.5% of the voxels of a 128x64x32 domain, the others
+// take 1 to 11.  With a thread to a voxel the launch lasted for those: 101 integrals of 25
+// nodes one after the other, 4250 us.  Now a thread takes its voxel through EASM_FIRST integrals, and
+// what is left of a block's voxels goes to groups of 16 lanes, one or two nodes a lane, until the
+// iteration repeats itself: the map has no other state than T, so a value that came back to the
+// bit gives every later one.  Per node one reciprocal and one exponential (a power, three divisions
+// and an exponential before).  A whole call now takes 220 us; bound by FP64 issue and the chain of
+// the last voxels.
 __constant__ double kGLx[AMC_GL25_N] = AMC_GL25_X;
 __constant__ double kGLw[AMC_GL25_N] = AMC_GL25_W;
 
-// Utilities::Materials_316L (S/Utilities.C:60-96): cP, k, rho, alpha at temperature T
+// Utilities::Materials_316L (S/Utilities.C:60-96): cP, k, rho at temperature T (alpha = k/(rho cP))
 // (pow(10, -n) written as the literal it folds to)
-__device__ static inline void mat316(double T, double& cP, double& k, double& rho, double& alpha) {
+__device__ static inline void mat316(double T, double& cP, double& k, double& rho) {
   if (T < 1660)
     rho = 8084.2 - 0.42086 * T - 3.8942 * 1e-5 * T * T;
   else if (T >= 1660 && T < 3090)
@@ -443,81 +468,186 @@ __device__ static inline void mat316(double T, double& cP, double& k, double& rh
     k = 12.41 + 3.279 * 1e-3 * T;
   else
     k = 21.6465;
-  alpha = k / (rho * cP);
+}
+
+// 1/x and 1/sqrt(x) for normal x by Newton's iteration on the hardware's estimates (within 1 ulp).
+__device__ static inline double rcp_f64(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+__device__ static inline double rsqrt_f64(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+// exp(x) for x <= 0: 2^n times the Taylor sum of the rest, |r| <= ln(2)/2, to r^13/13! (the next term
+// is 4e-18); ln(2) in two parts, the first short enough for exact products with n.
+__device__ static inline double exp_neg_f64(double x) {
+  x = fmax(x, -800.0);
+  const double n = rint(x * 0x1.71547652b82fep+0);
+  const double r = fma(-n, 0x1.ef35793c76730p-45, fma(-n, 0x1.62e42fefa3800p-1, x));
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return __builtin_amdgcn_ldexp(p, (int)n);
 }
 
 // Utilities::Integral (S/Utilities.C:105-124): 300 + the 25-point Gauss-Legendre sum over
 // s in [0, t] of Temp_Fun_G (S/Utilities.C:228-249), t = 8e-4 s, sigma 50 um, eta 0.56,
-// properties at the iterate T.  Nodes x = t/2 + (t/2) xi, weights (t/2) w, summed in order.
-__device__ static inline double easm_integral(const double L[3], double T, const double R[3], double Q, double bmV,
-                                              int* evals) {
-  const double t = 80.0e-5, sigma = 50.0e-6, eta = 0.56;
-  double cP, k, rho, alpha;
-  mat316(T, cP, k, rho, alpha);
-  const double C = eta * Q / (M_PI * rho * cP * sqrt(4 * M_PI * alpha));
-  const double x0 = L[0] - bmV * t;
-  const double slp = (t - 0.0) / 2.0, shft = (0.0 + t) / 2.0;
-  double sum = 0.0;
-  for (int i = 0; i < AMC_GL25_N; ++i) {
-    const double x = shft + slp * kGLx[i];
-    const double w = kGLw[i] * slp;
-    const double Lx = x0 + bmV * x;
-    const double dx = R[0] - Lx, dy = R[1] - L[1], dz = fabs(R[2] - L[2]);
-    const double f = C * pow(t - x, -0.5) / (2 * alpha * (t - x) + sigma * sigma) *
-                     exp(-1 * (dx * dx + dy * dy) / (4 * alpha * (t - x) + 2 * (sigma * sigma)) -
-                         dz * dz / (4 * alpha * (t - x)));
-    sum += w * f;
-  }
-  ++*evals;
-  return 300 + sum;
+// properties at the iterate T.  Nodes x = t/2 + (t/2) xi, weights (t/2) w.
+constexpr double kEasmT = 80.0e-5, kEasmSigma = 50.0e-6, kEasmEta = 0.56;
+struct EasmNodes {
+  double x[AMC_GL25_N];   // the source's position along the track
+  double ts[AMC_GL25_N];  // its age
+  double w[AMC_GL25_N];   // weight / sqrt(age)
+};
+struct EasmProps {
+  double a4;  // 4 alpha
+  double C2;  // twice eta Q / (pi rho cP sqrt(4 pi alpha))
+};
+__device__ static inline EasmProps easm_props(double T, double Q) {
+  double cP, k, rho;
+  mat316(T, cP, k, rho);
+  const double q = rho * cP;  // 2 / (pi rho cP sqrt(4 pi alpha)) = pi^(-3/2) / sqrt(k rho cP)
+  return {4 * k * rcp_f64(q), kEasmEta * Q * 0x1.6fcb5f827b97fp-3 * rsqrt_f64(k * q)};
 }
-
-// Utilities::EASM_Temp_LG (S/Utilities.C:128-140): damped Picard iteration from T
-__device__ static inline double easm_temp(const double L[3], const double R[3], double T, double Q, double bmV,
-                                          int* evals) {
-  double Told = T;
-  int n = 0;
-  const int nlim = 100;
-  const double tol = 10;
-  double Tnew = easm_integral(L, T, R, Q, bmV, evals);
-  while (fabs(Told - Tnew) > tol && n < nlim) {
-    Told = Tnew;
-    const double T_temp = easm_integral(L, Told, R, Q, bmV, evals);
-    Tnew = 0.5 * (Told + T_temp);
-    n++;
-  }
-  return Tnew;
+// one node's share of the sum; r2, z2: squared distances across and along z
+__device__ static inline double easm_node(const EasmProps& m, double ts, double w, double r2, double z2) {
+  const double a = m.a4 * ts, D = fma(m.a4, ts, 2 * (kEasmSigma * kEasmSigma));
+  const double inv = rcp_f64(a * D);
+  return w * exp_neg_f64(-(r2 * a + z2 * D) * inv) * (a * inv);
 }
 
 // TempField::EASM's voxel loop (S/TempField.C:90-115): 0 K above the laser plane, 0.99 T0
 // ahead of the laser in the top layer, EASM_Temp_LG from 0 K elsewhere; BuildjID as the
 // analytic model sets it; the "T >= tL" flag for SetLiquid3; O.any_melt collects whether
 // some voxel stayed below tL (the all_of test of S/TempField.C:121-124 is its negation).
+constexpr int EASM_LIM = 100, EASM_FIRST = 12;
+constexpr double EASM_TOL = 10;
 __global__ __launch_bounds__(GB) void k_easm(Inst* I, const int* bstart, int ninst, const amcd_step* S, amcd_out* O,
                                              double Q, double layerT, unsigned long long* n_evals) {
+  __shared__ EasmNodes nd;
+  __shared__ double lx[GB], ly[GB], lz[GB], lT[GB];  // voxels left after the first integrals
+  __shared__ int lown[GB], nleft;
   int ii = find_inst(bstart, ninst, blockIdx.x);
   const Inst d = I[ii];  // a copy: stores in the loops cannot alias it
-  const amcd_step& st = S[ii];
+  const amcd_step st = S[ii];
   if (st.skip) return;
-  const int v = (blockIdx.x - bstart[ii]) * GB + threadIdx.x;
-  bool cold = false;
+  const int tid = threadIdx.x, v = (blockIdx.x - bstart[ii]) * GB + tid;
+  const amcd_params& p = d.p;
+  if (tid < AMC_GL25_N) {
+    const double slp = kEasmT / 2.0, x = slp + slp * kGLx[tid];
+    nd.x[tid] = (st.lx - p.bmV * kEasmT) + p.bmV * x;
+    nd.ts[tid] = kEasmT - x;
+    nd.w[tid] = kGLw[tid] * slp / sqrt(kEasmT - x);
+  }
+  if (tid == 0) nleft = 0;
+  __syncthreads();
   int evals = 0;
+  double T = 0.0, zp = 0.0, xp = 0.0, y2 = 0.0, z2 = 0.0;
+  bool solve = false;
   if (v < d.N) {
     int i, j, k;
     decode(d, v, i, j, k);
-    const amcd_params& p = d.p;
-    const double x0 = ((double)i + .5) * p.dx;
-    const double y0 = ((double)j + .5) * p.dy;
-    const double zp = ((double)k + .5) * p.dz;
-    double T = 0.0;
+    const double x0 = ((double)i + .5) * p.dx, y0 = ((double)j + .5) * p.dy;
+    zp = ((double)k + .5) * p.dz;
     if (!(zp > st.lz)) {
-      const double xp = st.cg * (x0 - p.hx) + st.sg * (y0 - p.hy) + p.hx;
+      xp = st.cg * (x0 - p.hx) + st.sg * (y0 - p.hy) + p.hx;
       const double yp = (-st.sg) * (x0 - p.hx) + st.cg * (y0 - p.hy) + p.hy;
-      const double R[3] = {xp, yp, zp}, L[3] = {st.lx, st.ly, st.lz};
-      if ((x0 > st.lx) && (zp > (st.lz - layerT)))
-        T = .99 * p.T0;
-      else
-        T = easm_temp(L, R, 0.0, Q, p.bmV, &evals);
+      const double dy = yp - st.ly, dz = zp - st.lz;
+      y2 = dy * dy;
+      z2 = dz * dz;
+      solve = !((x0 > st.lx) && (zp > (st.lz - layerT)));
+      if (!solve) T = .99 * p.T0;
+    }
+  }
+  bool go = solve;
+  for (int n = 0; n < EASM_FIRST && __any(go); ++n) {
+    const EasmProps m = easm_props(T, Q);
+    double sum = 0.0;
+#pragma unroll 5
+    for (int q = 0; q < AMC_GL25_N; ++q) {
+      const double dx = xp - nd.x[q];
+      sum += easm_node(m, nd.ts[q], nd.w[q], fma(dx, dx, y2), z2);
+    }
+    const double F = 300 + m.C2 * sum, Tn = n == 0 ? F : 0.5 * (T + F);
+    if (go) {
+      ++evals;
+      go = fabs(T - Tn) > EASM_TOL;
+      T = Tn;
+    }
+  }
+  // the voxels that go on, to groups of 16 lanes
+  if (go) {
+    const int at = atomicAdd(&nleft, 1);
+    lx[at] = xp;
+    ly[at] = y2;
+    lz[at] = z2;
+    lT[at] = T;
+    lown[at] = tid;
+  }
+  __syncthreads();
+  const int left = nleft, sub = tid & 15;
+  for (int at = tid >> 4; at < left; at += GB / 16) {  // (whole groups: a voxel's lanes stay together)
+    const double y2g = ly[at], z2g = lz[at], dxa = lx[at] - nd.x[sub];
+    const bool two = sub + 16 < AMC_GL25_N;
+    const int q2 = two ? sub + 16 : sub;
+    const double dxb = lx[at] - nd.x[q2], ra = fma(dxa, dxa, y2g), rb = fma(dxb, dxb, y2g);
+    const double tsa = nd.ts[sub], tsb = nd.ts[q2], wa = nd.w[sub], wb = two ? nd.w[q2] : 0.0;
+    double Tg = lT[at], anchor = Tg;
+    int n = EASM_FIRST - 1, lim = EASM_LIM, seen = n, next = 2 * n;
+    while (n < lim) {
+      const EasmProps m = easm_props(Tg, Q);
+      double s = easm_node(m, tsa, wa, ra, z2g) + easm_node(m, tsb, wb, rb, z2g);
+      s += dpp<0xb1>(s);   // quad_perm [1, 0, 3, 2]
+      s += dpp<0x4e>(s);   // quad_perm [2, 3, 0, 1]
+      s += dpp<0x141>(s);  // row_half_mirror
+      s += dpp<0x140>(s);  // row_mirror
+      const double Tn = 0.5 * (Tg + (300 + m.C2 * s));
+      ++n;
+      const bool stop = !(fabs(Tg - Tn) > EASM_TOL);
+      Tg = Tn;
+      if (stop) break;
+      if (lim == EASM_LIM && Tg == anchor) {
+        // period n - seen: the values go round until the limit, and only the rest of the last round is
+        // evaluated (all of them count)
+        lim = n + (EASM_LIM - n) % (n - seen);
+      } else if (lim == EASM_LIM && n == next) {
+        anchor = Tg;
+        seen = n;
+        next = 2 * n;
+      }
+    }
+    if (sub == 0) {
+      lT[at] = Tg;
+      lx[at] = (double)(n == lim ? EASM_LIM + 1 : n + 1);  // integrals of this voxel
+    }
+  }
+  __syncthreads();
+  if (tid < left) {  // results back to the voxels' threads
+    ly[lown[tid]] = lT[tid];
+    lz[lown[tid]] = lx[tid];
+  }
+  __syncthreads();
+  if (go) {
+    T = ly[tid];
+    evals = (int)lz[tid];
+  }
+  bool cold = false;
+  if (v < d.N) {
+    if (!(zp > st.lz)) {
       if (T > p.tL) d.bj[v] = 1;
       else if (T < p.T0) d.bj[v] = 0;
     }
@@ -526,9 +656,9 @@ __global__ __launch_bounds__(GB) void k_easm(Inst* I, const int* bstart, int nin
     cold = !hot;
     d.vs[v] = (d.vs[v] & 3) | (hot ? 0x80 : 0);
   }
-  if (__any(cold) && (threadIdx.x & 63) == 0) atomicOr(&O[ii].any_melt, 1);
+  if (__any(cold) && (tid & 63) == 0) atomicOr(&O[ii].any_melt, 1);
   for (int m = 32; m >= 1; m >>= 1) evals += __shfl_xor(evals, m);
-  if ((threadIdx.x & 63) == 0 && evals) atomicAdd(n_evals, (unsigned long long)evals);
+  if ((tid & 63) == 0 && evals) atomicAdd(n_evals, (unsigned long long)evals);
 }
 
 // SetLiquid3 (S/VoxelsCA.C:1098-1116) when the temperature kernel ran without it.
@@ -1451,20 +1581,6 @@ __device__ static inline bool better(const Best& a, const Best& b) {
 // mirrors leave a row's result in all 16 of its lanes, row_bcast:15 and row_bcast:31
 // carry rows 0 and 2 into rows 1 and 3 and then row 1 into rows 2 and 3, so that lane
 // 63 ends with the result for the whole wave.  Every lane must be active.
-template <int CTRL, int ROWS = 0xf>
-__device__ static inline int dpp(int v) {
-  return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
-}
-template <int CTRL, int ROWS = 0xf>
-__device__ static inline float dpp(float v) {
-  return __int_as_float(dpp<CTRL, ROWS>(__float_as_int(v)));
-}
-template <int CTRL, int ROWS = 0xf>
-__device__ static inline double dpp(double v) {
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)dpp<CTRL, ROWS>((int)b), hi = (unsigned)dpp<CTRL, ROWS>((int)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
 constexpr int kQuadX1 = 0xb1, kQuadX2 = 0x4e, kHalfMirror = 0x141, kMirror = 0x140, kBcast15 = 0x142,
               kBcast31 = 0x143;
 __device__ static inline float wave_min(float v) {
@@ -3090,6 +3206,7 @@ struct amcd_batch {
   uint8_t* d_mark = nullptr;  // SetBuild's grain marks (mark_cap bytes)
   size_t mark_cap = 0;
   std::vector<size_t> pool_off;
+  unsigned long long* d_evals = nullptr;  // source integrals of an EASM evaluation
   hipEvent_t pool_ev = nullptr;  // the last staging copy (the staging area is rewritten after it)
   // The driver's step as HIP graphs (AMCAFE_GRAPH=0 launches the stages one by one): the stages up
   // to the capture loop, per capture tier, and the finishing pass; each is captured again when the
@@ -3274,7 +3391,7 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
       dalloc(b, &b->d_lstart, (size_t)n + 1) || dalloc(b, &b->d_cstart, (size_t)n + 1) ||
       dalloc(b, &b->d_bstartZ, (size_t)n + 1) || dalloc(b, &b->d_astart, (size_t)n + 1) ||
       dalloc(b, &b->d_bstartF, (size_t)n + 1) ||
-      dalloc(b, &b->d_steps, (size_t)n) || dalloc(b, &b->d_outs, (size_t)n)) {
+      dalloc(b, &b->d_steps, (size_t)n) || dalloc(b, &b->d_evals, 1) || dalloc(b, &b->d_outs, (size_t)n)) {
     snprintf(err, errlen, "%s", g_dev_err.c_str());
     amcd_destroy(b);
     return -1;
@@ -3536,8 +3653,7 @@ static int read_outs(amcd_batch* b, amcd_out* outs);
 int amcd_easm(amcd_batch* b, const amcd_step* steps, double Q, double layerT, amcd_out* outs,
               unsigned long long* n_evals) {
   if (put_steps(b, steps) || launch_step_in(b, true)) return -1;
-  unsigned long long* dn = nullptr;
-  HIPT(hipMalloc(&dn, sizeof(unsigned long long)));
+  unsigned long long* dn = b->d_evals;
   HIPT(hipMemsetAsync(dn, 0, sizeof(unsigned long long), b->stream));
   tmark(b, 0);
   hipLaunchKernelGGL(k_easm, dim3(b->bstartG[b->n]), dim3(GB), 0, b->stream, b->d_inst, b->d_bstartG, b->n,
@@ -3547,7 +3663,6 @@ int amcd_easm(amcd_batch* b, const amcd_step* steps, double Q, double layerT, am
   unsigned long long hn = 0;
   HIPT(hipMemcpyAsync(&hn, dn, sizeof(hn), hipMemcpyDeviceToHost, b->stream));
   if (read_outs(b, outs)) return -1;
-  HIPT(hipFree(dn));
   if (b->timing) {
     float ms = 0;
     (void)hipEventElapsedTime(&ms, b->ev[0], b->ev[1]);
