@@ -3206,6 +3206,7 @@ struct amcd_batch {
   uint8_t* d_mark = nullptr;  // SetBuild's grain marks (mark_cap bytes)
   size_t mark_cap = 0;
   std::vector<size_t> pool_off;
+  std::vector<std::pair<void**, size_t>> wanted;  // device arrays of the next allocation
   unsigned long long* d_evals = nullptr;  // source integrals of an EASM evaluation
   hipEvent_t pool_ev = nullptr;  // the last staging copy (the staging area is rewritten after it)
   // The driver's step as HIP graphs (AMCAFE_GRAPH=0 launches the stages one by one): the stages up
@@ -3238,31 +3239,55 @@ static thread_local std::string g_dev_err;
     }                                                                                  \
   } while (0)
 
-// Every device array has 256 bytes beyond its length: the list-block reads of the
+// Device arrays are asked for one by one and come out of one allocation: freeing an allocation
+// waits for the device, 95 us each; twelve domains' 505 took 48 ms to close, as one 2 ms.
+// Every array has 256 bytes beyond its length: the list-block reads of the
 // capture loop run up to four entries past the last slot's list.
 template <class T>
-static int dalloc(amcd_batch* b, T** p, size_t n) {
-  void* q = nullptr;
-  HIPT(hipMalloc(&q, n * sizeof(T) + 256));
+static void want(amcd_batch* b, T** p, size_t n) {
+  b->wanted.emplace_back((void**)p, (n * sizeof(T) + 256 + 255) & ~(size_t)255);
+}
+static int alloc_wanted(amcd_batch* b) {
+  std::vector<std::pair<void**, size_t>> wanted;
+  wanted.swap(b->wanted);
+  size_t total = 0;
+  for (const auto& w : wanted) total += w.second;
+  char* q = nullptr;
+  HIPT(hipMalloc((void**)&q, total));
   b->allocs.push_back(q);
-  *p = (T*)q;
+  for (const auto& w : wanted) {
+    *w.first = q;
+    q += w.second;
+  }
   return 0;
 }
 
-static int alloc_active(amcd_batch* b, Inst& d, int acap) {
+static void want_active(amcd_batch* b, Inst& d, int acap) {
   d.acap = acap;
   size_t c = (size_t)acap;
   // about 80 entries per growing cell, of which there are far fewer than active cells
   d.precap = (int)std::min<size_t>(8 * c, (size_t)1 << 26);
   if (c * AMCD_NB + (size_t)d.precap > 0x7fffff00ull) d.precap = 0;  // entries are counted in 32 bits
-  if (dalloc(b, &d.aVox, c) || dalloc(b, &d.aVS, c) || dalloc(b, &d.aG, c) || dalloc(b, &d.aT, c) ||
-      dalloc(b, &d.aExt, c) || dalloc(b, &d.aCx, c) || dalloc(b, &d.aCy, c) || dalloc(b, &d.aCz, c) ||
-      dalloc(b, &d.ruq, c) || dalloc(b, &d.aRow, c) || dalloc(b, &d.events, c) || dalloc(b, &d.aScan, c) ||
-      dalloc(b, &d.slots, c) || dalloc(b, &d.gExt, c) || dalloc(b, &d.gVhat, c) || dalloc(b, &d.gLH, c) ||
-      dalloc(b, &d.gHd, c) || dalloc(b, &d.cand, c * AMCD_NB + d.precap) ||
-      dalloc(b, &d.cF, c * AMCD_NB + d.precap) || dalloc(b, &d.cap, c * AMCD_NB + d.precap))
-    return -1;
-  return 0;
+  want(b, &d.aVox, c);
+  want(b, &d.aVS, c);
+  want(b, &d.aG, c);
+  want(b, &d.aT, c);
+  want(b, &d.aExt, c);
+  want(b, &d.aCx, c);
+  want(b, &d.aCy, c);
+  want(b, &d.aCz, c);
+  want(b, &d.ruq, c);
+  want(b, &d.aRow, c);
+  want(b, &d.events, c);
+  want(b, &d.aScan, c);
+  want(b, &d.slots, c);
+  want(b, &d.gExt, c);
+  want(b, &d.gVhat, c);
+  want(b, &d.gLH, c);
+  want(b, &d.gHd, c);
+  want(b, &d.cand, c * AMCD_NB + d.precap);
+  want(b, &d.cF, c * AMCD_NB + d.precap);
+  want(b, &d.cap, c * AMCD_NB + d.precap);
 }
 
 static int push_inst(amcd_batch* b) {
@@ -3335,15 +3360,52 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
     d.nblkS = (d.N + SB - 1) / SB;
     d.nblkT = (d.N + GB * TV - 1) / (GB * TV);
     size_t Nn = (size_t)d.N;
-    if (dalloc(b, &d.vs, Nn) || dalloc(b, &d.gid, Nn) || dalloc(b, &d.ext, Nn) || dalloc(b, &d.cx, Nn) ||
-        dalloc(b, &d.cy, Nn) || dalloc(b, &d.cz, Nn) || dalloc(b, &d.T, Nn) || dalloc(b, &d.bj, Nn) || dalloc(b, &d.build, Nn) ||
-        dalloc(b, &d.amap, Nn) || dalloc(b, &d.bcA, (size_t)d.nblkZ) || dalloc(b, &d.bcM, (size_t)d.nblkZ) ||
-        dalloc(b, &d.chA, (size_t)d.nblkZ / 1024 + 1) || dalloc(b, &d.chM, (size_t)d.nblkZ / 1024 + 1) ||
-        dalloc(b, &d.zliq, 2 * (size_t)p[i].nz) || dalloc(b, &d.ls, 1)) {
-      snprintf(err, errlen, "%s", g_dev_err.c_str());
-      amcd_destroy(b);
-      return -1;
-    }
+    want(b, &d.vs, Nn);
+    want(b, &d.gid, Nn);
+    want(b, &d.ext, Nn);
+    want(b, &d.cx, Nn);
+    want(b, &d.cy, Nn);
+    want(b, &d.cz, Nn);
+    want(b, &d.T, Nn);
+    want(b, &d.bj, Nn);
+    want(b, &d.build, Nn);
+    want(b, &d.amap, Nn);
+    want(b, &d.bcA, (size_t)d.nblkZ);
+    want(b, &d.bcM, (size_t)d.nblkZ);
+    want(b, &d.chA, (size_t)d.nblkZ / 1024 + 1);
+    want(b, &d.chM, (size_t)d.nblkZ / 1024 + 1);
+    want(b, &d.zliq, 2 * (size_t)p[i].nz);
+    want(b, &d.ls, 1);
+    // (it grows on overflow; 2^23 interface cells are far more than a domain this size needs)
+    int acap = (int)std::min<long long>(N, std::max<long long>(1 << 16, std::min<long long>(N / 8, 1 << 23)));
+    if (const char* ac = getenv("AMCAFE_ACTIVE_CAP_INIT"))  // tests: start small to exercise the growth path
+      acap = (int)std::min<long long>(N, std::max(64, atoi(ac)));
+    want_active(b, d, acap);
+    d.gcap = 0;
+    d.rot = nullptr;
+    d.poolcap = 0;
+    d.pool = nullptr;
+    b->bstartG[i + 1] = b->bstartG[i] + d.nblkG;
+    b->bstartS[i + 1] = b->bstartS[i] + d.nblkS;
+    b->bstartT[i + 1] = b->bstartT[i] + d.nblkT;
+    b->cstart[i + 1] = b->cstart[i] + (d.nblkZ + 1023) / 1024;
+    b->bstartZ[i + 1] = b->bstartZ[i] + d.nblkZ;
+    b->bstartF[i + 1] = b->bstartF[i] + (d.nblkZ + 3) / 4;
+  }
+  want(b, &b->d_inst, (size_t)n);
+  for (int** starts : {&b->d_bstartG, &b->d_bstartS, &b->d_bstartT, &b->d_lstart, &b->d_cstart, &b->d_bstartZ, &b->d_astart,
+                       &b->d_bstartF})
+    want(b, starts, (size_t)n + 1);
+  want(b, &b->d_steps, (size_t)n);
+  want(b, &b->d_outs, (size_t)n);
+  want(b, &b->d_evals, 1);
+  if (alloc_wanted(b)) {
+    snprintf(err, errlen, "%s", g_dev_err.c_str());
+    amcd_destroy(b);
+    return -1;
+  }
+  for (Inst& d : b->h) {
+    size_t Nn = (size_t)d.N;
     hipError_t me = hipSuccess;
     auto zero = [&](void* q, int val, size_t bytes) {
       const hipError_t e = hipMemsetAsync(q, val, bytes, b->stream);
@@ -3358,7 +3420,7 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
     zero(d.T, 0, Nn * 8);
     zero(d.bj, 0, Nn);
     zero(d.build, 0, Nn);
-    zero(d.zliq, 0xff, (size_t)p[i].nz * 8);  // unknown: every plane may hold liquid
+    zero(d.zliq, 0xff, (size_t)d.p.nz * 8);  // unknown: every plane may hold liquid
     zero(d.amap, 0xff, Nn * 4);
     zero(d.ls, 0, sizeof(LoopState));
     if (me != hipSuccess) {
@@ -3366,35 +3428,6 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
       amcd_destroy(b);
       return -1;
     }
-    // (it grows on overflow; 2^23 interface cells are far more than a domain this size needs)
-    int acap = (int)std::min<long long>(N, std::max<long long>(1 << 16, std::min<long long>(N / 8, 1 << 23)));
-    if (const char* ac = getenv("AMCAFE_ACTIVE_CAP_INIT"))  // tests: start small to exercise the growth path
-      acap = (int)std::min<long long>(N, std::max(64, atoi(ac)));
-    if (alloc_active(b, d, acap)) {
-      snprintf(err, errlen, "%s", g_dev_err.c_str());
-      amcd_destroy(b);
-      return -1;
-    }
-    d.gcap = 0;
-    d.rot = nullptr;
-    d.poolcap = 0;
-    d.pool = nullptr;
-    b->bstartG[i + 1] = b->bstartG[i] + d.nblkG;
-    b->bstartS[i + 1] = b->bstartS[i] + d.nblkS;
-    b->bstartT[i + 1] = b->bstartT[i] + d.nblkT;
-    b->cstart[i + 1] = b->cstart[i] + (d.nblkZ + 1023) / 1024;
-    b->bstartZ[i + 1] = b->bstartZ[i] + d.nblkZ;
-    b->bstartF[i + 1] = b->bstartF[i] + (d.nblkZ + 3) / 4;
-  }
-  if (dalloc(b, &b->d_inst, (size_t)n) || dalloc(b, &b->d_bstartG, (size_t)n + 1) ||
-      dalloc(b, &b->d_bstartS, (size_t)n + 1) || dalloc(b, &b->d_bstartT, (size_t)n + 1) ||
-      dalloc(b, &b->d_lstart, (size_t)n + 1) || dalloc(b, &b->d_cstart, (size_t)n + 1) ||
-      dalloc(b, &b->d_bstartZ, (size_t)n + 1) || dalloc(b, &b->d_astart, (size_t)n + 1) ||
-      dalloc(b, &b->d_bstartF, (size_t)n + 1) ||
-      dalloc(b, &b->d_steps, (size_t)n) || dalloc(b, &b->d_evals, 1) || dalloc(b, &b->d_outs, (size_t)n)) {
-    snprintf(err, errlen, "%s", g_dev_err.c_str());
-    amcd_destroy(b);
-    return -1;
   }
   if (hipHostMalloc((void**)&b->h_steps, sizeof(amcd_step) * n, 0) != hipSuccess ||
       hipHostMalloc((void**)&b->h_outs, sizeof(amcd_out) * n, 0) != hipSuccess) {
@@ -3811,10 +3844,10 @@ static int grow_active(amcd_batch* b, const amcd_out* outs) {
     int need = outs[i].n_active;
     int ncap = (int)std::min<long long>(d.N, std::max<long long>((long long)need * 3 / 2, (long long)d.acap * 2));
     // old arrays stay allocated until destroy; they are simply no longer referenced
-    if (alloc_active(b, d, ncap)) return -1;
+    want_active(b, d, ncap);
     any = true;
   }
-  if (any && push_inst(b)) return -1;
+  if (any && (alloc_wanted(b) || push_inst(b))) return -1;
   return 0;
 }
 
