@@ -126,10 +126,12 @@ struct LoopState {
 struct alignas(16) CandRec {
   double D, r;  // capture distance, ruqs
   int tgt;      // target (active index)
-  int nb;       // neighbour rank
   float tn;     // lower bound on the time from a capture through this entry to the first capture
                 // by the cell it creates (-inf: unknown)
-  int n;        // entries from this one to the list's end
+  float back;   // lower bound on how far the clock may step back after it before that cell's
+                // half-diagonal is zero (-inf: unknown)
+  short nb;     // neighbour rank
+  short n;      // entries from this one to the list's end
 };
 // What the capture loop reads of an active cell whose voxel is captured, in one cache line.
 struct alignas(128) CellRow {
@@ -1351,15 +1353,23 @@ __device__ static inline float time_bound(double lead, double V) {
   const float f = (float)x;
   return (double)f > x ? nextafterf(f, 0.0f) : f;
 }
+// Lower bound on the time that takes a half-diagonal E back to zero at velocity V (-inf: none).
+__device__ static inline float back_bound(double E, double V) {
+  if (!(E >= 0.0) || !(V >= 0.0)) return -__builtin_inff();
+  return V > 0.0 ? (float)(E / V * (1.0 - 1e-6)) : __builtin_inff();
+}
 // Lower bound on the time from the capture of active cell t (voxel v; new centroid c, rotation R,
 // half-diagonal E0) to the first capture by the cell it becomes, over the neighbours that are
-// liquid before the loop.  -inf: no useful bound; +inf: the cell does not grow.
+// liquid before the loop, and (*back) on the step back that takes E0 to zero.  -inf: no useful
+// bound; +inf: the cell does not grow.
 __device__ static inline float first_capture_after(const Inst& d, int t, int v, const double* c, double E0,
-                                                   const float* Rf) {
+                                                   const float* Rf, float* back) {
+  *back = __builtin_inff();
   if (!d.aRow[t].cold) return __builtin_inff();
   const amcd_params& p = d.p;
   const double T = d.aRow[t].T;
   const double V = T == p.tS ? p.vhat_tS : (T == p.T0 ? p.vhat_T0 : p.Avel * pow(p.tL - T, p.nvel) * (1 + 1e-9));
+  *back = back_bound(E0, V);
   if (!(V > 0.0) || !(E0 == E0)) return -__builtin_inff();
   int i, j, k;
   decode(d, v, i, j, k);
@@ -1441,7 +1451,7 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     const int t2 = q < AMCD_NB && (two || !half) ? d.aRow[tj].nbr[q] : -1;
     const bool on = t2 >= 0 && d.aVS[t2] == 1;
     double D2 = __builtin_inf(), f2 = 0.0, r2 = __builtin_inf();
-    float tn2 = -__builtin_inff();
+    float tn2 = -__builtin_inff(), back2 = -__builtin_inff();
     CapRec cr = {0.0, 0.0, 0.0, 0.0, -1, sr.G, 0.0};
     if (on) {
       r2 = .5 * (d.ruq[tj] + d.ruq[t2]);
@@ -1454,7 +1464,7 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
       const int v2 = vj + ddz * d.nxy + ddy * p.nx + ddx;
       double nc[3], ne;
       recentre(d, vj, v2, c, R, f2, nc, &ne);
-      tn2 = first_capture_after(d, t2, v2, nc, ne, Rf);
+      tn2 = first_capture_after(d, t2, v2, nc, ne, Rf, &back2);
       cr.x = nc[0];
       cr.y = nc[1];
       cr.z = nc[2];
@@ -1469,7 +1479,7 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     const bool fits = base >= 0 && base <= d.precap - na - nb;
     const size_t at = (size_t)d.acap * AMCD_NB + (half ? base + na : base);
     if (on && fits) {
-      d.cand[at + rank2] = {D2, r2, t2, q, tn2, (half ? nb : na) - rank2};
+      d.cand[at + rank2] = {D2, r2, t2, tn2, back2, (short)q, (short)((half ? nb : na) - rank2)};
       d.cF[at + rank2] = f2;
       d.cap[at + rank2] = cr;
     }
@@ -1489,7 +1499,7 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     }
   }
   if (liq) {
-    d.cand[cb + rank] = {D, r, t, lane, tnew, n - rank};
+    d.cand[cb + rank] = {D, r, t, tnew, cold ? back_bound(rc.w, V) : __builtin_inff(), (short)lane, (short)(n - rank)};
     d.cF[cb + rank] = f;
     d.cap[cb + rank] = {rc.x, rc.y, rc.z, rc.w, pre, sr.G, V};
   }
@@ -1532,8 +1542,10 @@ __global__ void k_clear_npre(Inst* I) {
 //            scan order), the event's uniform draw, T += Dt, E += V*Dt of its lanes, and the
 //            captured voxel's entries drop out.  No candidate outside the window can come first:
 //            their lower bounds exceed W, and the earliest capture by a cell that an event creates
-//            is bounded from below by the set-up (CandRec::tn), which ends the window where the
-//            bound falls below W and the cell's candidates are not entries themselves;
+//            is bounded from below by the set-up (CandRec::tn) or, for a list made in the loop, by
+//            BUILD, which the engine waits for then; the window ends where the bound falls below W
+//            and the cell's candidates are not entries themselves.  A step back of the clock goes
+//            on like any other unless it could take some half-diagonal below zero (CandRec::back);
 //   BUILD    meanwhile the other waves create the cells of the events as they are published:
 //            grain, centre, half-diagonal, list (S/VoxelsCA.C:396-440, 486-506, 528-605);
 //   APPLY    heads that died move to the next live candidate (the cells are listed in LDS first, so
@@ -1546,13 +1558,13 @@ __global__ void k_clear_npre(Inst* I) {
 //
 // What bounds it: a chain of dependent instructions.  An event is about 100 instructions of one
 // wave (11 to 13 cycles each), and every window pays five barriers and two rounds of list reads;
-// hence as many events per window as its 64 entries give (25 where the interface is wide, 8 where
-// a cell captures within a step of its own capture), records that are one cache line, and lists
-// and capture constants made by the set-up's parallel pass.  One wave per event with the window
-// built around each event took 6.9K cycles an event in these decks and 13.7K with the state in
-// memory; now (cycles per event, 2.4 GHz): 5.6K with few growing cells (at most 300), 3.0K with
-// 3 thousand, 2.9K with 3 thousand of a raster over a wide plate, 10.1K with 15 thousand (state in
-// memory).
+// hence as many events per window as its 64 entries give (31 where the interface is wide, 8 where
+// there are few cells), records that are one cache line, and lists and capture constants made by the
+// set-up's parallel pass.  One decision per barrier with the lists built around each event took
+// 6.9K cycles an event in these decks and 13.7K with the state in memory; now (cycles per event, 2.4
+// GHz): 5.5K with few growing cells (at most 300), 2.8K with 3 thousand of a single track or of a
+// raster over a wide plate, 6.7K with 15 thousand (state in memory; 10.1K while a cell without a
+// bound from the set-up, or any step back, ended the window).
 typedef const __attribute__((address_space(4))) Inst CInst;
 struct Best {
   double t, r;
@@ -1682,7 +1694,7 @@ __device__ static inline CandRec load_rec(const CandRec* p) {
   const v2d x = q[0], y = q[1];
   const unsigned long long a = (unsigned long long)__double_as_longlong(y.x);
   const unsigned long long b = (unsigned long long)__double_as_longlong(y.y);
-  return {x.x, x.y, (int)a, (int)(a >> 32), __int_as_float((int)b), (int)(b >> 32)};
+  return {x.x, x.y, (int)a, __int_as_float((int)(a >> 32)), __int_as_float((int)b), (short)(b >> 32), (short)(b >> 48)};
 }
 // First live entry of a sorted list from entry `from` on, four records at a time with no branches
 // between the loads.  Positions past the list's end read what follows it, at the array's end the
@@ -1784,12 +1796,14 @@ struct Window {
   double y[WCAP];   // reciprocal of V
   int parent[WCAP]; // the entry whose capture creates this one's cell (-1: the cell is there)
   int rank[WCAP];   // position by hi
+  float back[WCAP]; // CandRec::back
   // events, in order: entry (-1: nucleation, -2: not performed yet) and voxel, published one by
   // one; growth time; the slot of the cell it created (-1: none)
   int2 ev[WCAP];
   double dt[WCAP];
   int slot[WCAP], base[WCAP];  // (base: its list's first entry)
   double E0[WCAP], V0[WCAP];
+  int first[WCAP];  // after an event: CandRec::tn of the cell as BUILD has made it, as bits (kPending: not yet)
   int n;        // entries asked for (more than WCAP: the window is too full)
   int m;        // events
   int decided;  // events decided in this window (one more than m when the last waits for the pool)
@@ -1806,6 +1820,7 @@ struct LoopShared {
   double tE[TCAP], tV[TCAP];
   int tS[TCAP], tn;
   float red[16];
+  int back;      // CandRec::back's minimum over the cells, as float bits (they order like the values)
   int hist[32];  // heads by lower bound, in thirty-seconds of twice the window's span
   int nslots;
   int fin;  // 1: goes on, 0: finished, -1: pool refill, -2: larger tier, -4: no progress
@@ -1862,7 +1877,8 @@ __device__ static inline int order_key(float f) {
   const int i = __float_as_int(f);
   return i ^ ((i >> 31) & 0x7fffffff);
 }
-constexpr int kKeyInf = 0x7f800000, kKeyNone = 0x7fffffff;  // +inf; after every bound
+// +inf; after every bound; as an entry's limit: BUILD is asked when it is captured
+constexpr int kKeyInf = 0x7f800000, kKeyNone = 0x7fffffff, kKeyAsk = 0x7ffffffe;
 template <int CTRL, int ROWS = 0xf>
 __device__ static inline int dpp_min(int v) {
   return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
@@ -1909,6 +1925,7 @@ struct EngineState {
   int nd;  // draws consumed
   int visits;
 };
+constexpr int kPending = 0x7fc00bad;  // (no float result has these bits)
 struct EngineRun {
   double T, rdt;
   int m, used, visits, fin, ri1, rent;
@@ -1918,16 +1935,26 @@ template <bool PLAIN>
 __device__ static inline void engine_run(EngineRun& o, Window& win, double D, double E, double V, double y, double r,
                                          int tgt, int key, int src, int parent, int lo, int hi, int lim_,
                                          unsigned long long live, unsigned long long close, unsigned long long draws, int W, int mmax,
-                                         double DelT, int scan0) {
+                                         double DelT, int scan0, float back) {
   const int lane = threadIdx.x & 63;
-  double T = o.T, rdt = 0.0;
+  double T = o.T, rdt = 0.0, rT = 0.0;
+  const double T0 = T;
   int m = 0, ri1 = -1, rent = -2, used = 0, visits = 0, fin = 1, lim = W;
+  bool ask = false;  // the last event's cell has no bound yet
   bool nuc = false;
   unsigned long long killed = 0;
   double Vg = parent < 0 ? V : 0.0;  // a cell grows from the event that creates it on
   while (live != 0) {
     int wl = 63 - __builtin_clzll(live);
     const int u = __builtin_amdgcn_readlane(hi, wl);
+    if (ask) {  // BUILD's (it is at work on the event, whatever this wave does)
+      int b;
+      while ((b = uni(*(volatile int*)&win.first[m - 1])) == kPending) __builtin_amdgcn_s_sleep(1);
+      const float f = __int_as_float(b), Tf = (float)T;
+      const float x = Tf + f - 0x1p-20f * (fabsf(Tf) + fabsf(f));
+      lim = min(lim, f == -__builtin_inff() ? (int)0x80000000 : f == __builtin_inff() ? kKeyNone : uni(order_key(x)) - 2);
+      ask = false;
+    }
     if (u > lim) break;
     if (!(T < DelT)) {  // loop condition (S/VoxelsCA.C:381)
       fin = 0;
@@ -1983,11 +2010,17 @@ __device__ static inline void engine_run(EngineRun& o, Window& win, double D, do
     nuc = (draws >> m) & 1ull;
     if (nuc) break;
     // capture: growth of every cell (S/VoxelsCA.C:511-516); the lanes' cells all have a live
-    // candidate.  A step back in time (negative Dt) ends the window, since it may clamp a
+    // candidate.  A step back in time (negative Dt) ends the window if it may clamp a
     // half-diagonal at zero and so move a capture time.
     rent = me ? ent : rent;
+    bool clamp = false;
+    if (th < 0) {
+      const double f = lane < m ? rT - (double)win.back[rent < 0 ? 0 : rent] : -__builtin_inf();
+      clamp = !(T + tw > fmax(-wave_min_f64(-f), T0 - (double)back));
+    }
     *(volatile unsigned long long*)&win.ev[lane] = ((unsigned long long)(unsigned)ri1 << 32) | (unsigned)rent;
     T = T + tw;
+    rT = me ? T : rT;
     E = E + Vg * tw;
     rdt = me ? tw : rdt;
     killed |= __ballot(tgt == i1);
@@ -1999,8 +2032,10 @@ __device__ static inline void engine_run(EngineRun& o, Window& win, double D, do
       key = mine ? (scan0 + m) * 32 + key : key;
     }
     live &= ~killed;
-    lim = min(lim, __builtin_amdgcn_readlane(lim_, wl));
-    lim = th < 0 ? (int)0x80000000 : lim;
+    const int bound = __builtin_amdgcn_readlane(lim_, wl);
+    ask = bound == kKeyAsk;
+    lim = min(lim, bound);
+    lim = clamp ? (int)0x80000000 : lim;
     ++m;
     if (m >= mmax) break;
   }
@@ -2042,13 +2077,14 @@ __device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& wi
   EngineRun o;
   o.T = uni(es.T);
   const int Wk = uni(order_key(W));
+  const float back = __int_as_float(uni(sh.back));
   mmax = uni(mmax);
   if (plain)
     engine_run<true>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
-                      uni(es.vSind2));
+                      uni(es.vSind2), back);
   else
     engine_run<false>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
-                      uni(es.vSind2));
+                      uni(es.vSind2), back);
   int fin = n == 0 ? 0 : o.fin, m = o.m;  // n == 0: no candidate left
   es.captures += m;
   if (fin == 1 && o.nuc) {  // S/VoxelsCA.C:483-506
@@ -2116,7 +2152,7 @@ __device__ __attribute__((noinline)) static double velocity_out(const Inst* I, d
 // The sorted list of a cell that no set-up list was built ahead for (a nucleus, or a capture by a
 // cell of this launch), out of line as the other rare parts.
 __device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb, int i1, int G, int v1, int tn, int liq,
-                                                          double c0, double c1, double c2) {
+                                                          double c0, double c1, double c2, double E0, double V0, int k) {
   CInst& d = *(CInst*)I;
   auto& p = d.p;
   const int lane = threadIdx.x & 63;
@@ -2136,12 +2172,19 @@ __device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb,
     candidate_at(ct, cen, R, &D, &f);
     r = .5 * (gmem(d.ruq)[i1] + gmem(d.ruq)[tn]);
   }
+  const bool bad = __any(liq && !(D == D));
+  const double Dm = wave_min_f64(liq ? D : __builtin_inf());
+  if (lane == 0) {  // (first of all: the engine may wait for it)
+    asm volatile("" ::: "memory");
+    *(volatile int*)&s_loop.win.first[k] = __float_as_int(bad ? -__builtin_inff() : time_bound(Dm - E0, V0));
+  }
   const int rank = list_rank(D, r, liq != 0, -1), n = (int)__popcll(__ballot(liq != 0));
   if (liq) {
     typedef double v2d __attribute__((ext_vector_type(2)));
     const auto q = gmem((v2d*)(d.cand + cb + rank));
     q[0] = v2d{D, r};
-    q[1] = v2d{pack2(tn, lane), pack2(__float_as_int(-__builtin_inff()), n - rank)};
+    const int none = __float_as_int(-__builtin_inff());
+    q[1] = v2d{pack2(tn, none), pack2(none, lane | (n - rank) << 16)};
     gmem(d.cF)[cb + rank] = f;
   }
 }
@@ -2201,18 +2244,26 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
     if (lane == 0) slot = atomicAdd(&sh.nslots, 1);
     slot = uni(slot);
     cb = pre >= 0 ? pre : slot * AMCD_NB;
+    const double V0 = (T1 == p.tS) & (T1 < p.tL) ? p.vhat_tS : velocity_out(I, T1);
+    if (lane == 0 && ent >= 0 && win.lim[ent] == kKeyAsk) win.back[ent] = back_bound(E0, V0);
     if (pre < 0) {
       if (ent < 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the nucleus's rotation, read back
-      list_out(I, cb, i1, G, v1, tn, liq, cen[0], cen[1], cen[2]);
+      list_out(I, cb, i1, G, v1, tn, liq, cen[0], cen[1], cen[2], E0, V0, k);
     }
-    const double V0 = (T1 == p.tS) & (T1 < p.tL) ? p.vhat_tS : velocity_out(I, T1);
     if (lane == 0) {
       win.base[k] = cb;
       win.E0[k] = E0;
       win.V0[k] = V0;
     }
   }
-  if (lane == 0) win.slot[k] = slot;
+  if (lane == 0) {
+    win.slot[k] = slot;
+    if (!grows && ent >= 0 && win.lim[ent] == kKeyAsk) win.back[ent] = __builtin_inff();
+    if (!grows || pre >= 0) {  // (the set-up's list for the cell gave the engine no bound)
+      asm volatile("" ::: "memory");
+      *(volatile int*)&win.first[k] = __float_as_int(grows ? -__builtin_inff() : __builtin_inff());
+    }
+  }
   // the slot's record by lanes 0..2 and the event's by lanes 3..5, 16 bytes each
   const int q = lane < 3 ? lane : lane - 3;
   const double c02 = q == 0 ? cen[0] : cen[2];
@@ -2320,6 +2371,7 @@ __device__ static inline int put_entry(Window& win, const CandRec& e, double E, 
   win.parent[i] = parent;
   win.lo[i] = lo;
   win.hi[i] = hi;
+  win.back[i] = e.back;
   return i;
 }
 template <bool GD>
@@ -2347,8 +2399,8 @@ __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Wind
       // window, its candidates join it
       const float tn = e[q].tn;
       const float x = lo + tn - 0x1p-20f * (fabsf(lo) + fabsf(tn));
-      int lim = tn == -__builtin_inff() ? (int)0x80000000 : tn == __builtin_inff() ? kKeyNone : order_key(x) - 2;
-      if (lim < order_key(W) && (p + q < ns_pre * AMCD_NB)) {
+      int lim = tn == -__builtin_inff() ? kKeyAsk : tn == __builtin_inff() ? kKeyNone : order_key(x) - 2;
+      if ((lim < order_key(W) || lim == kKeyAsk) && (p + q < ns_pre * AMCD_NB)) {
         const CapRec cr = d.cap[p + q];
         if (cr.pre >= 0) {
           lim = kKeyNone;
@@ -2358,16 +2410,15 @@ __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Wind
             tau_bounds(ec.D, cr.E, cr.V, 0.0, l, h);
             const int lk = order_key(lo + l) - 1, hk = order_key(hi + h) + 1;
             if (l == __builtin_inff() || lk > order_key(W)) break;
-            if (l == -__builtin_inff()) {  // (no bound: the window ends with the capture)
-              lim = (int)0x80000000;
+            if (l == -__builtin_inff()) {  // (no bound)
+              lim = kKeyAsk;
               break;
             }
             if (!live.dead(ec.tgt)) {
               const int ic = put_entry(win, ec, cr.E, cr.V, ec.nb, pc, -1, i, lk, hk);
               if (ic < 0) return;
               const float xc = lo + l + ec.tn - 0x1p-20f * (fabsf(lo) + fabsf(l) + fabsf(ec.tn));
-              win.lim[ic] = ec.tn == -__builtin_inff() ? (int)0x80000000
-                                                       : ec.tn == __builtin_inff() ? kKeyNone : order_key(xc) - 2;
+              win.lim[ic] = ec.tn == -__builtin_inff() ? kKeyAsk : ec.tn == __builtin_inff() ? kKeyNone : order_key(xc) - 2;
             }
             if (ec.n <= 1) break;
           }
@@ -2469,6 +2520,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
     sh.T = ls->tinc;
     sh.fin = go > 0 ? 1 : (go == 0 ? 0 : -2);
     sh.units = 0;
+    sh.back = 0;
     sh.cur = ls->rng;
   }
   if (tid < 32) sh.hist[tid] = 0;
@@ -2579,6 +2631,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       if (lane == 0) sh.red[w] = u;
       if (tid < WCAP) {
         win.ev[tid] = make_int2(-2, -1);
+        win.first[tid] = kPending;
         win.rank[tid] = 0;
       }
       if (w == 1) {  // the window's uniforms, one per lane (S/VoxelsCA.C:483)
@@ -2735,6 +2788,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         if (lane == 0) {
           sh.all = nev >= (1 << 20);
           sh.neg = 0;
+          sh.back = kKeyInf;
         }
         nev = nev >= (1 << 20) ? 0 : nev;
       }
@@ -2791,6 +2845,10 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       // growth, event by event in the reference's order (S/VoxelsCA.C:511-516), of the cells of
       // before the window; a nucleation's time is 0: E + V*0 = E
       bool neg = false;
+      float back = fInf;  // CandRec::back over the cells, after the window
+      auto step_back = [](double e, double v) {
+        return v > 0.0 ? e > 0.0 ? (float)e * __builtin_amdgcn_rcpf((float)v) : 0.0f : __builtin_inff();
+      };
       for (int s0 = w * 64; s0 < ns; s0 += KR * NT) {
         if constexpr (MEM) {
 #pragma unroll
@@ -2808,6 +2866,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
           neg |= c.E[k] < 0.0;
+          if (s0 + lane + k * NT < ns) back = fminf(back, step_back(c.E[k], c.V[k]));
           if constexpr (MEM) {
             const int s = s0 + lane + k * NT;
             if (s < ns) gmem(d.gExt)[s] = c.E[k];
@@ -2843,6 +2902,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
           } else {
             gmem(d.gExt)[s] = o.grown;
             gmem(d.gVhat)[s] = v;
+            back = fminf(back, step_back(o.grown, v));
           }
           if (HM || s < CAP) {
             set_hd<HM>(d, s, o.tgt >= 0 ? o.c1 : i, o.tgt);
@@ -2855,6 +2915,8 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         }
       }
       if (neg) sh.neg = 1;
+      back = wave_min(back);
+      if (lane == 0) atomicMin(&sh.back, __float_as_int(back * (1.0f - 0x1p-16f)));
       __syncthreads();
       PHASE(pt, 5);
       // what the list's threads found: cells out of candidates, and the new cells
