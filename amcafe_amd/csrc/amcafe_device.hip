@@ -67,6 +67,33 @@ __device__ __forceinline__ void gstore8(V* p, V v) {
   *gmem((unsigned long long*)p) = __builtin_bit_cast(unsigned long long, v);
 }
 
+// LDS words that the waves of a workgroup exchange while they run, each one access in program order (a
+// wave's LDS operations are performed in order: what was stored before a word is there when the word
+// is seen).  As accesses through a generic pointer to volatile they were flat and system-wide, each
+// with a wait for its acknowledgement.
+template <class T>
+__device__ __forceinline__ void lds_put(T* p, T v) {
+  typedef __attribute__((address_space(3))) unsigned u32;
+  typedef __attribute__((address_space(3))) unsigned long long u64;
+  asm volatile("" ::: "memory");
+  if constexpr (sizeof(T) == 8)
+    __hip_atomic_store((u64*)p, __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else
+    __hip_atomic_store((u32*)p, __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class T>
+__device__ __forceinline__ T lds_get(T* p) {
+  typedef __attribute__((address_space(3))) unsigned u32;
+  typedef __attribute__((address_space(3))) unsigned long long u64;
+  T v;
+  if constexpr (sizeof(T) == 8)
+    v = __builtin_bit_cast(T, __hip_atomic_load((u64*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  else
+    v = __builtin_bit_cast(T, __hip_atomic_load((u32*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  asm volatile("" ::: "memory");
+  return v;
+}
+
 // lane l's value of v (l must be the same in every lane)
 __device__ static inline double lane_f64(double v, int l) {
   const long long b = __double_as_longlong(v);
@@ -78,7 +105,10 @@ __device__ static inline double lane_f64(double v, int l) {
 // another lane's value by a DPP row operation
 template <int CTRL, int ROWS = 0xf>
 __device__ static inline int dpp(int v) {
-  return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
+  if constexpr (ROWS == 0xf && (CTRL < 0x100 || CTRL == 0x140 || CTRL == 0x141))  // every lane reads an active one
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, false);
+  else
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
 }
 template <int CTRL, int ROWS = 0xf>
 __device__ static inline float dpp(float v) {
@@ -1907,8 +1937,7 @@ __device__ static inline int dpp_min_shift(int v) {  // with the lane's lower ne
 // An event for BUILD to start on: one 8-byte store (a wave's LDS stores are performed in order, so
 // what was stored before it is there when it is seen).
 __device__ static inline void publish(Window& win, int m, int ent, int i1) {
-  asm volatile("" ::: "memory");
-  *(volatile unsigned long long*)&win.ev[m] = ((unsigned long long)(unsigned)i1 << 32) | (unsigned)ent;
+  lds_put(&win.ev[m], make_int2(ent, i1));
 }
 
 // ENGINE: the events of window `win`, by one wave.  The entries are sorted by their upper
@@ -1931,35 +1960,33 @@ struct EngineRun {
   int m, used, visits, fin, ri1, rent;
   bool nuc;
 };
+// The body is straight: one branch leaves the loop, whatever the reason, and only near-ties, asking
+// BUILD and steps back branch inside (a taken branch costs as much as three instructions).
 template <bool PLAIN>
 __device__ static inline void engine_run(EngineRun& o, Window& win, double D, double E, double V, double y, double r,
                                          int tgt, int key, int src, int parent, int lo, int hi, int lim_,
-                                         unsigned long long live, unsigned long long close, unsigned long long draws, int W, int mmax,
+                                         unsigned long long live, unsigned long long close, unsigned long long draws, int W,
                                          double DelT, int scan0, float back) {
   const int lane = threadIdx.x & 63;
-  double T = o.T, rdt = 0.0, rT = 0.0;
+  double T = o.T, rdt = 0.0;
   const double T0 = T;
-  int m = 0, ri1 = -1, rent = -2, used = 0, visits = 0, fin = 1, lim = W;
-  bool ask = false;  // the last event's cell has no bound yet
+  int m = 0, ri1 = -1, rent = -2, visits = 0, lim = W, fin = 1, used = 0;
   bool nuc = false;
+  bool ask = false;  // the last event's cell has no bound yet
   unsigned long long killed = 0;
   double Vg = parent < 0 ? V : 0.0;  // a cell grows from the event that creates it on
   while (live != 0) {
     int wl = 63 - __builtin_clzll(live);
     const int u = __builtin_amdgcn_readlane(hi, wl);
-    if (ask) {  // BUILD's (it is at work on the event, whatever this wave does)
+    if (__builtin_expect(ask, 0)) {  // BUILD's (it is at work on the event, whatever this wave does)
       int b;
-      while ((b = uni(*(volatile int*)&win.first[m - 1])) == kPending) __builtin_amdgcn_s_sleep(1);
+      while ((b = uni(lds_get(&win.first[m - 1]))) == kPending) __builtin_amdgcn_s_sleep(1);
       const float f = __int_as_float(b), Tf = (float)T;
       const float x = Tf + f - 0x1p-20f * (fabsf(Tf) + fabsf(f));
       lim = min(lim, f == -__builtin_inff() ? (int)0x80000000 : f == __builtin_inff() ? kKeyNone : uni(order_key(x)) - 2);
       ask = false;
     }
-    if (u > lim) break;
-    if (!(T < DelT)) {  // loop condition (S/VoxelsCA.C:381)
-      fin = 0;
-      break;
-    }
+    const bool late = u > lim;
     const double a = D - E;
     double t;
     if constexpr (PLAIN) {
@@ -1969,58 +1996,72 @@ __device__ static inline void engine_run(EngineRun& o, Window& win, double D, do
     } else {
       t = a / V;
     }
-    ++visits;
+    int seen = 1;
+    bool none = false;
     if ((close >> wl) & 1ull) {
       // several within rounding: the smallest time, then (ruqs, key) among the equal ones
       const unsigned long long c = __ballot(lo <= u) & live;
-      visits += __popcll(c) - 1;
+      seen = __popcll(c);
       const bool ok = ((c >> lane) & 1ull) && t <= 1e6;
       const double tmin = wave_min_f64(ok ? t : __builtin_inf());
       unsigned long long at = __ballot(ok && t == tmin);
-      if (at == 0) {
-        if (m == 0) fin = 0;
-        break;
-      }
-      wl = __builtin_ctzll(at);
-      at &= at - 1;
-      if (at != 0) {
-        double rb = lane_f64(r, wl);
-        int kb = __builtin_amdgcn_readlane(key, wl);
-        for (; at != 0; at &= at - 1) {
-          const int l = __builtin_ctzll(at);
-          const double rl = lane_f64(r, l);
-          const int kl = __builtin_amdgcn_readlane(key, l);
-          const bool first = rl < rb || (!(rl > rb) && kl < kb);
-          wl = first ? l : wl;
-          rb = first ? rl : rb;
-          kb = first ? kl : kb;
+      none = at == 0;
+      if (!none) {
+        wl = __builtin_ctzll(at);
+        at &= at - 1;
+        if (at != 0) {
+          double rb = lane_f64(r, wl);
+          int kb = __builtin_amdgcn_readlane(key, wl);
+          for (; at != 0; at &= at - 1) {
+            const int l = __builtin_ctzll(at);
+            const double rl = lane_f64(r, l);
+            const int kl = __builtin_amdgcn_readlane(key, l);
+            const bool first = rl < rb || (!(rl > rb) && kl < kb);
+            wl = first ? l : wl;
+            rb = first ? rl : rb;
+            kb = first ? kl : kb;
+          }
         }
       }
     }
     const double tw = lane_f64(t, wl);
     const int th = (int)(__double_as_longlong(tw) >> 32);
-    if (th >= 0x412e8480) {  // 1e6 or more, or not a number (S/VoxelsCA.C:480)
-      fin = 0;
-      break;
-    }
     const int i1 = __builtin_amdgcn_readlane(tgt, wl), ent = __builtin_amdgcn_readlane(src, wl);
     const bool me = lane == m;
-    ri1 = me ? i1 : ri1;
-    used = m + 1;
-    nuc = (draws >> m) & 1ull;
-    if (nuc) break;
+    const int over = __ballot(T < DelT) == 0;         // loop condition (S/VoxelsCA.C:381)
+    const int far = th >= 0x412e8480;                 // 1e6 or more, or not a number (S/VoxelsCA.C:480)
+    const int draw = (int)((draws >> m) & 1ull);      // nucleation (S/VoxelsCA.C:483)
+    if ((int)late | over | (int)none | far | draw) {
+      if (!late) {
+        fin = over ? 0 : none ? (m == 0 ? 0 : 1) : far ? 0 : 1;
+        visits += over ? 0 : seen;
+        nuc = !over && !none && !far;
+        if (nuc) {
+          ri1 = me ? i1 : ri1;
+          used = m + 1;
+        }
+      }
+      break;
+    }
+    visits += seen;
     // capture: growth of every cell (S/VoxelsCA.C:511-516); the lanes' cells all have a live
     // candidate.  A step back in time (negative Dt) ends the window if it may clamp a
     // half-diagonal at zero and so move a capture time.
-    rent = me ? ent : rent;
     bool clamp = false;
-    if (th < 0) {
-      const double f = lane < m ? rT - (double)win.back[rent < 0 ? 0 : rent] : -__builtin_inf();
-      clamp = !(T + tw > fmax(-wave_min_f64(-f), T0 - (double)back));
+    if (__builtin_expect(th < 0, 0)) {
+      double Tk = rdt;  // the clock after each event so far (to rounding, which `back` has room for)
+      for (int s = 1; s < 64; s <<= 1) {
+        const double p = __shfl_up(Tk, s);
+        Tk += lane >= s ? p : 0.0;
+      }
+      Tk += T0 + 0x1p-40 * (fabs(T0) + fabs(Tk));
+      const double f = lane < m ? Tk - (double)win.back[rent < 0 ? 0 : rent] : -__builtin_inf();
+      clamp = !(T + tw > fmax(-wave_min_f64(-f), T0 + 0x1p-40 * fabs(T0) - (double)back));
     }
-    *(volatile unsigned long long*)&win.ev[lane] = ((unsigned long long)(unsigned)ri1 << 32) | (unsigned)rent;
+    ri1 = me ? i1 : ri1;
+    rent = me ? ent : rent;
+    lds_put(&win.ev[lane], make_int2(rent, ri1));
     T = T + tw;
-    rT = me ? T : rT;
     E = E + Vg * tw;
     rdt = me ? tw : rdt;
     killed |= __ballot(tgt == i1);
@@ -2037,19 +2078,18 @@ __device__ static inline void engine_run(EngineRun& o, Window& win, double D, do
     lim = min(lim, bound);
     lim = clamp ? (int)0x80000000 : lim;
     ++m;
-    if (m >= mmax) break;
   }
   o.T = T;
   o.rdt = rdt;
   o.m = m;
-  o.used = used;
+  o.used = nuc ? used : m;
   o.visits = visits;
   o.fin = fin;
   o.ri1 = ri1;
   o.rent = rent;
   o.nuc = nuc;
 }
-__device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& win, EngineState& es, float W, int mmax,
+__device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& win, EngineState& es, float W,
                                             double DelT_, int n_pool, LoopState* ls) {
   const int lane = threadIdx.x & 63;
   const int n = uni(win.n);
@@ -2078,12 +2118,11 @@ __device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& wi
   o.T = uni(es.T);
   const int Wk = uni(order_key(W));
   const float back = __int_as_float(uni(sh.back));
-  mmax = uni(mmax);
   if (plain)
-    engine_run<true>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
+    engine_run<true>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, DelT,
                       uni(es.vSind2), back);
   else
-    engine_run<false>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, mmax, DelT,
+    engine_run<false>(o, win, D, E, V, y, r, tgt, key, src, parent, lo, hi, lim, live, close, draws, Wk, DelT,
                       uni(es.vSind2), back);
   int fin = n == 0 ? 0 : o.fin, m = o.m;  // n == 0: no candidate left
   es.captures += m;
@@ -2108,7 +2147,7 @@ __device__ static inline void engine_window(CInst& d, LoopShared& sh, Window& wi
       ++m;
     }
   }
-  if (lane == 0) *(volatile int*)&win.done = 1;
+  if (lane == 0) lds_put(&win.done, 1);
   if (lane < m) {
     win.dt[lane] = o.rdt;
     gmem(d.aScan)[o.ri1] = es.vSind2 + lane;
@@ -2174,10 +2213,8 @@ __device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb,
   }
   const bool bad = __any(liq && !(D == D));
   const double Dm = wave_min_f64(liq ? D : __builtin_inf());
-  if (lane == 0) {  // (first of all: the engine may wait for it)
-    asm volatile("" ::: "memory");
-    *(volatile int*)&s_loop.win.first[k] = __float_as_int(bad ? -__builtin_inff() : time_bound(Dm - E0, V0));
-  }
+  // (first of all: the engine may wait for it)
+  if (lane == 0) lds_put(&s_loop.win.first[k], __float_as_int(bad ? -__builtin_inff() : time_bound(Dm - E0, V0)));
   const int rank = list_rank(D, r, liq != 0, -1), n = (int)__popcll(__ballot(liq != 0));
   if (liq) {
     typedef double v2d __attribute__((ext_vector_type(2)));
@@ -2198,7 +2235,7 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
   typedef double v2d __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
   auto& p = d.p;
-  const int evi = lane <= k ? ((volatile int2*)win.ev)[lane].y : -1;  // lane j: voxel of event j
+  const int evi = lane <= k ? lds_get(&win.ev[lane]).y : -1;  // lane j: voxel of event j
   const int i1 = __builtin_amdgcn_readlane(evi, k), scan = uni(win.scan0) + k;
   const int cand = ent >= 0 ? uni(win.cand[ent]) : -1, sw = ent >= 0 ? uni(win.own[ent]) : -1;
   // an entry of a list the set-up built (the cells' own, and those ahead)
@@ -2259,10 +2296,8 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
   if (lane == 0) {
     win.slot[k] = slot;
     if (!grows && ent >= 0 && win.lim[ent] == kKeyAsk) win.back[ent] = __builtin_inff();
-    if (!grows || pre >= 0) {  // (the set-up's list for the cell gave the engine no bound)
-      asm volatile("" ::: "memory");
-      *(volatile int*)&win.first[k] = __float_as_int(grows ? -__builtin_inff() : __builtin_inff());
-    }
+    // (the set-up's list for the cell gave the engine no bound)
+    if (!grows || pre >= 0) lds_put(&win.first[k], __float_as_int(grows ? -__builtin_inff() : __builtin_inff()));
   }
   // the slot's record by lanes 0..2 and the event's by lanes 3..5, 16 bytes each
   const int q = lane < 3 ? lane : lane - 3;
@@ -2286,8 +2321,8 @@ __device__ __attribute__((noinline)) static void build_cells(const Inst* I, int 
   for (int k = first; k < WCAP; k += step) {
     int ent;
     for (;;) {
-      const int done = uni(*(volatile int*)&win.done);
-      ent = uni(((volatile int2*)win.ev)[k].x);  // (read after `done`: a set flag means all is published)
+      const int done = uni(lds_get(&win.done));
+      ent = uni(lds_get(&win.ev[k]).x);  // (read after `done`: a set flag means all is published)
       if (ent != -2 || done) break;
       __builtin_amdgcn_s_sleep(1);
     }
@@ -2744,7 +2779,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         // ---- ENGINE
         if (w == 0) {
           __builtin_amdgcn_s_setprio(3);
-          engine_window(d, sh, win, es, W, mode == 3 ? 1 : WCAP, DelT, n_pool, ls);
+          engine_window(d, sh, win, es, W, DelT, n_pool, ls);
           __builtin_amdgcn_s_setprio(0);
         }
       } else if (w == 0) {
@@ -2760,7 +2795,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
           gmem(d.aScan)[i1] = es.vSind2;
           *gmem(&ls->pending) = 0;
           publish(win, 0, -1, i1);
-          *(volatile int*)&win.done = 1;
+          lds_put(&win.done, 1);
         }
         es.vSind2++;
         es.pool_used++;
