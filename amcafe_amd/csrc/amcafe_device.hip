@@ -1343,10 +1343,12 @@ __device__ static inline void recentre(DI& d, int vcap, int vnew, const double* 
 // evaluated here for every entry, over the whole chip, instead of on the capture loop's one compute
 // unit: the re-centring by the entry's lane, the new cell's sorted list two entries at a time (a
 // half wave each), with the re-centring of its own entries and a single-precision bound on the time
-// to the captures after them.  About one list in forty of those built ahead is used.  Bound by the
-// latency of a wave's own chain, not by the chip (a few thousand waves): 64 us for 3.3 thousand
-// growing cells and 37 us for 300 (18 and 15 us with the cells' own lists alone); with the lists
-// ahead the loop's windows end later: 3291 -> 2863 cycles per event in the former deck.
+// to the captures after them.  Only for the captures that the step has time for: a cell grows half a
+// voxel a step, which leaves about a third of the entries.  Bound by the latency of a wave's own
+// chain, not by the chip (a few thousand waves): 33 us for 3.3 thousand growing cells, 44 us for 15
+// thousand and 22 us for 300 (64, 109 and 38 us with lists ahead for every entry, 18 and 15 us in the
+// first and last without any); with the lists ahead the loop's windows end later: 3291 -> 2863
+// cycles per event in the first deck.
 __device__ static inline int list_rank(double D, double r, bool on, int half) {
   // position in (D, ruqs, neighbour) order among the entries of this lane's half wave (all of it
   // for half < 0), NaN distances last
@@ -1464,7 +1466,9 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
   // the lists ahead, for the entries whose target would grow
   const int half = lane >> 5, q = lane & 31;
   const int qq = q < 13 ? q : q + 1, ddx = qq % 3 - 1, ddy = (qq / 3) % 3 - 1, ddz = qq / 9 - 1;
-  for (unsigned todo = (unsigned)__ballot(liq && cold); todo != 0;) {
+  // and whose capture the step has time for (a step's last event may come later: its list is made then)
+  const bool soon = !(D > d.gExt[slot] + d.gVhat[slot] * p.DelT * (1 + 1e-6));
+  for (unsigned todo = (unsigned)__ballot(liq && cold && soon); todo != 0;) {
     const int j0 = __builtin_ctz(todo);
     todo &= todo - 1;
     const bool two = todo != 0;
@@ -1529,6 +1533,7 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     }
   }
   if (liq) {
+    if (cold && !soon) tnew = -__builtin_inff();
     d.cand[cb + rank] = {D, r, t, tnew, cold ? back_bound(rc.w, V) : __builtin_inff(), (short)lane, (short)(n - rank)};
     d.cF[cb + rank] = f;
     d.cap[cb + rank] = {rc.x, rc.y, rc.z, rc.w, pre, sr.G, V};
