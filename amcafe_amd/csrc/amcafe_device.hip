@@ -142,6 +142,7 @@ struct LoopState {
   int Na, nmushy0;
   int npre;          // entries of the lists built ahead
   int zhot0, zhot1;  // z planes the last temperature evaluation could have melted
+  int zold0, zold1;  // the same of the evaluation that tvalid speaks of
   // T holds the analytic field of a laser plane at lz_prev (tvalid = 1): every voxel is xi
   // where its hot flag (vs bit 7) is set, else T0 above lz_prev and tS below it
   int tvalid;
@@ -322,7 +323,14 @@ __device__ static inline void decode(DI& d, int v, int& i, int& j, int& k) {
 //    extent plus two voxels (in the unrotated frame: the rotation about the plate centre
 //    preserves distances up to rounding far below that margin) cannot reach tL, so in the
 //    planes the pool can reach it changes nothing unless one of its voxels was hot.
-#define TV 16  // voxels per thread (their state bytes in 16-byte loads)
+//  * planes that neither this evaluation nor the last could melt keep everything while the laser
+//    stays in its plane: the workgroups go over the others only.
+// A thread takes four voxels (one state word): what bounds it is the chain of a thread whose voxels
+// are near the laser, some FP64 instructions and two or three divisions one after another for
+// each, and the stores.  20 us for 512x512x128, 8.8 for 256x192x64, 7.2 for 40x24x20; with sixteen voxels a
+// thread, a workgroup to every block of the domain and the melt flag of the step set by an atomic
+// per wave 32, 20 and 14.
+#define TV 4  // voxels per thread
 __global__ __launch_bounds__(GB) void k_temperature(Inst* I, const int* bstart, int ninst, const amcd_step* S,
                                                     amcd_out* O, int setliquid) {
   int ii = find_inst(bstart, ninst, blockIdx.x);
@@ -331,44 +339,43 @@ __global__ __launch_bounds__(GB) void k_temperature(Inst* I, const int* bstart, 
   const Inst d = I[ii];
   const amcd_step st = S[ii];
   if (st.skip) return;
-  const int v0 = ((blockIdx.x - bstart[ii]) * GB + threadIdx.x) * TV;
   const amcd_params& p = d.p;
-  if (v0 == 0) {  // planes with (k+.5)dz in (lz - max depth, lz] are the only ones T can reach tL in
-    const double depth = fmax(p.a1[2], p.a1[5]);
-    d.ls->zhot0 = max(0, (int)floor((st.lz - depth) / p.dz - 0.5) - 1);
-    d.ls->zhot1 = min(p.nz - 1, (int)floor(st.lz / p.dz - 0.5) + 1);
+  // planes with (k+.5)dz in (lz - max depth, lz] are the only ones T can reach tL in (with a plane of
+  // margin; the ellipsoid tests need |zp - lz| < depth): elsewhere T is T0 or tS without geometry
+  const double depth = fmax(p.a1[2], p.a1[5]);
+  const int kh0 = (int)floor((st.lz - depth) / p.dz - 0.5) - 1, kh1 = (int)floor(st.lz / p.dz - 0.5) + 1;
+  if (blockIdx.x == bstart[ii] && threadIdx.x == 0) {
+    d.ls->zhot0 = max(0, kh0);
+    d.ls->zhot1 = min(p.nz - 1, kh1);
   }
   bool anyhot = false;
   // the three temperatures as values (selected through their struct fields, the compiler
   // would keep the struct in scratch memory and load through the selected address)
   const double T0 = p.T0, tS = p.tS, tL = p.tL, xi = p.xi;
-  if (v0 < d.N) {
-    const bool valid = d.ls->tvalid != 0 && tS < tL && T0 < tL;
-    const double lzp = d.ls->lz_prev;
-    const double e1 = 1 + 0x1p-40;
-    const double lim1 = p.a1[1] * e1, lim2 = p.a1[2] * e1, lim3 = p.a1[3] * e1, lim4 = p.a1[4] * e1,
-                 lim5 = p.a1[5] * e1;
+  const bool valid = d.ls->tvalid != 0 && tS < tL && T0 < tL;
+  const double lzp = d.ls->lz_prev;
+  const int zold0 = d.ls->zold0, zold1 = d.ls->zold1;
+  const double e1 = 1 + 0x1p-40;
+  const double lim1 = p.a1[1] * e1, lim2 = p.a1[2] * e1, lim3 = p.a1[3] * e1, lim4 = p.a1[4] * e1,
+               lim5 = p.a1[5] * e1;
+  int first = 0, last = d.nblkT - 1;
+  if (valid && st.lz == lzp && !(tS < T0)) {  // (tS < T0: the melt flags of planes below the laser's are cleared)
+    first = max(0, min(p.nz - 1, min(kh0, zold0))) * d.nxy / (GB * TV);
+    last = min(last, ((max(0, min(p.nz - 1, max(kh1, zold1))) + 1) * d.nxy - 1) / (GB * TV));
+  }
+  const int nb = bstart[ii + 1] - bstart[ii];
+  for (int blk = first + (int)blockIdx.x - bstart[ii]; blk <= last; blk += nb) {
+    const int v0 = (blk * GB + (int)threadIdx.x) * TV;
+    if (v0 >= d.N) continue;
     uint8_t sv[TV];
     if (v0 + TV <= d.N) {
-      unsigned ws[TV / 4];
+      const unsigned w = *reinterpret_cast<const unsigned*>(d.vs + v0);
 #pragma unroll
-      for (int c = 0; c < TV / 16; ++c) {  // 16-byte loads of the run's state bytes
-        const uint4 w = *reinterpret_cast<const uint4*>(d.vs + v0 + 16 * c);
-        ws[4 * c] = w.x;
-        ws[4 * c + 1] = w.y;
-        ws[4 * c + 2] = w.z;
-        ws[4 * c + 3] = w.w;
-      }
-#pragma unroll
-      for (int q = 0; q < TV; ++q) sv[q] = (uint8_t)(ws[q >> 2] >> (8 * (q & 3)));
+      for (int q = 0; q < TV; ++q) sv[q] = (uint8_t)(w >> (8 * q));
     } else {
 #pragma unroll
       for (int q = 0; q < TV; ++q) sv[q] = v0 + q < d.N ? d.vs[v0 + q] : 0;
     }
-    // planes outside (lz - max depth, lz] (with a plane of margin) cannot reach tL: the
-    // ellipsoid tests need |zp - lz| < depth, so T is T0 or tS there without geometry
-    const double depth = fmax(p.a1[2], p.a1[5]);
-    const int kh0 = (int)floor((st.lz - depth) / p.dz - 0.5) - 1, kh1 = (int)floor(st.lz / p.dz - 0.5) + 1;
     int i, j, k;
     decode(d, v0, i, j, k);
     // Nothing changes for a run of voxels in one plane outside [kh0, kh1] when none of them
@@ -458,7 +465,7 @@ __global__ __launch_bounds__(GB) void k_temperature(Inst* I, const int* bstart, 
       }
     }
   }
-  if (__any(anyhot) && (threadIdx.x & 63) == 0) atomicOr(&O[ii].any_melt, 1);
+  if (__any(anyhot) && (threadIdx.x & 63) == 0) O[ii].any_melt = 1;  // (every writer stores 1)
 }
 // After a temperature pass: the field now matches this step's laser plane.
 __global__ void k_temp_commit(Inst* I, const amcd_step* S, int valid) {
@@ -466,6 +473,8 @@ __global__ void k_temp_commit(Inst* I, const amcd_step* S, int valid) {
   if (threadIdx.x != 0 || S[blockIdx.x].skip) return;
   d.ls->tvalid = valid;
   d.ls->lz_prev = S[blockIdx.x].lz;
+  d.ls->zold0 = d.ls->zhot0;
+  d.ls->zold1 = d.ls->zhot1;
 }
 
 // -------------------------------------------------------------------------------------
@@ -688,7 +697,7 @@ __global__ __launch_bounds__(GB) void k_easm(Inst* I, const int* bstart, int nin
     cold = !hot;
     d.vs[v] = (d.vs[v] & 3) | (hot ? 0x80 : 0);
   }
-  if (__any(cold) && (tid & 63) == 0) atomicOr(&O[ii].any_melt, 1);
+  if (__any(cold) && (tid & 63) == 0) O[ii].any_melt = 1;
   for (int m = 32; m >= 1; m >>= 1) evals += __shfl_xor(evals, m);
   if ((tid & 63) == 0 && evals) atomicAdd(n_evals, (unsigned long long)evals);
 }
@@ -992,6 +1001,8 @@ __global__ __launch_bounds__(1024) void k_scan(Inst* I, const int* cstart, int n
       if (commit) {
         ls->tvalid = 1;
         ls->lz_prev = st.lz;
+        ls->zold0 = ls->zhot0;
+        ls->zold1 = ls->zhot1;
       }
     }
   }
@@ -3489,7 +3500,7 @@ int amcd_create(const amcd_params* p, int n, amcd_batch** out, char* err, int er
     d.pool = nullptr;
     b->bstartG[i + 1] = b->bstartG[i] + d.nblkG;
     b->bstartS[i + 1] = b->bstartS[i] + d.nblkS;
-    b->bstartT[i + 1] = b->bstartT[i] + d.nblkT;
+    b->bstartT[i + 1] = b->bstartT[i] + std::min(d.nblkT, std::max(64, 2048 / n));  // (what the chip holds at a time)
     b->cstart[i + 1] = b->cstart[i] + (d.nblkZ + 1023) / 1024;
     b->bstartZ[i + 1] = b->bstartZ[i] + d.nblkZ;
     b->bstartF[i + 1] = b->bstartF[i] + (d.nblkZ + 3) / 4;
