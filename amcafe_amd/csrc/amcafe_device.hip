@@ -4234,7 +4234,7 @@ int amcd_step_fused(amcd_batch* b, const amcd_step* steps, amcd_out* outs) {
 }
 
 int amcd_resume(amcd_batch* b, const amcd_step* steps, amcd_out* outs) {
-  if (put_steps(b, steps)) return -1;
+  if (put_steps(b, steps) || launch_step_in(b, false)) return -1;
   if (launch_event_loop(b)) return -1;
   if (read_outs(b, outs)) return -1;
   if (widen(b, outs) || regrow_tier(b, outs)) return -1;

@@ -42,7 +42,8 @@ def _state(extent, every, rotated):
 
 
 CASES = [("equal", 3, False, 0.0, 0), ("equal", 3, True, 0.0, 2), ("mixed", 3, True, 2e-4, 0), ("beyond", 3, False, 1e-4, 2),
-         ("beyond", 2, True, 0.0, 0), ("equal", 16, False, 0.0, 2)]
+         ("beyond", 2, True, 0.0, 0), ("equal", 16, False, 0.0, 2),
+         ("mixed", 3, True, 2e-2, 0)]  # every event nucleates: the pool of orientations is refilled over and over
 
 
 @functools.lru_cache(maxsize=None)
