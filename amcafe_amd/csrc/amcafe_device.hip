@@ -3165,12 +3165,22 @@ __global__ __launch_bounds__(GB) void k_finish(Inst* I, const int* astart, int n
 // ---- per-layer helpers ---------------------------------------------------------------
 // After a host upload of vState: the "T >= tL" flag (bit 7) follows the device's current
 // temperature field, so SetLiquid3 still sees the caller's melt pool.
-// A step's records: in from the pinned staging area with fresh output records (`clear` words), and the
-// outputs back.  As kernels in the step's graph they cost 2 us each; as stream copies beside it, 10.
-__global__ void k_step_in(unsigned* steps, const unsigned* staged, int nwords, unsigned* outs, int clear) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < nwords) steps[q] = staged[q];
-  if (q < clear) outs[q] = 0u;
+// A step's records: in from the pinned staging area with fresh output records (`clear` words) and the
+// instances' nucleation pools (a workgroup each, after the first `nrec`), and the outputs back.  As
+// kernels in the step's graph they cost 3.5 us each; as stream copies beside it, 10.
+__global__ void k_step_in(unsigned* steps, const unsigned* staged, int nwords, unsigned* outs, int clear, const Inst* I,
+                          int nrec, const double* dpool, const double* hpool) {
+  if ((int)blockIdx.x < nrec) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < nwords) steps[q] = staged[q];
+    if (q < clear) outs[q] = 0u;
+    return;
+  }
+  const int i = blockIdx.x - nrec;
+  const int n = 9 * min(((const amcd_step*)staged)[i].n_pool, I[i].poolcap);
+  double* to = I[i].pool;
+  const double* from = hpool + (to - dpool);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) to[q] = from[q];
 }
 __global__ void k_step_out(unsigned* staged, const unsigned* outs, int nwords) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3378,7 +3388,7 @@ struct amcd_batch {
   int min_tier = 0;  // lowest tier a step starts in (AMCAFE_CAPTURE_TIER_MIN; tests use it to
                      // run small decks in the larger tiers; 5 = memory tier, bitmap in memory)
   // nucleation pools of every instance in one device region (instance i's at pool_off[i]
-  // entries of 9 doubles), filled from one pinned staging copy per step
+  // entries of 9 doubles), staged in pinned memory, from which the step takes them
   double* d_pool = nullptr;
   double* h_pool = nullptr;  // pinned
   uint8_t* d_mark = nullptr;  // SetBuild's grain marks (mark_cap bytes)
@@ -3386,7 +3396,6 @@ struct amcd_batch {
   std::vector<size_t> pool_off;
   std::vector<std::pair<void**, size_t>> wanted;  // device arrays of the next allocation
   unsigned long long* d_evals = nullptr;  // source integrals of an EASM evaluation
-  hipEvent_t pool_ev = nullptr;  // the last staging copy (the staging area is rewritten after it)
   // The driver's step as HIP graphs (AMCAFE_GRAPH=0 launches the stages one by one): the stages up
   // to the capture loop, per capture tier, and the finishing pass; each is captured again when the
   // block counts it was captured with change (capacity growth)
@@ -3646,7 +3655,6 @@ void amcd_destroy(amcd_batch* b) {  // best effort: errors while tearing down ar
   if (b->h_pool) (void)hipHostFree(b->h_pool);
   if (b->d_pool) (void)hipFree(b->d_pool);
   if (b->d_mark) (void)hipFree(b->d_mark);
-  if (b->pool_ev) (void)hipEventDestroy(b->pool_ev);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
 }
@@ -3750,15 +3758,18 @@ int amcd_get_rot(amcd_batch* b, int i, double* rot9, int ngrain) {
   return 0;
 }
 
-// Every instance's pool lives in one device region behind one pinned staging area: the
-// pools of a step go to the device in one copy instead of one pageable copy per instance
-// (each of which the host waits for).  A pool larger than its instance's capacity
+// Every instance's pool lives in one device region behind one pinned staging area, from which the
+// step's first kernel takes it.  A pool larger than its instance's capacity
 // re-lays the region out for every instance (capacities at least double).
 int amcd_set_pools(amcd_batch* b, const double* const* rot9, const int* n) {
   bool grow = b->d_pool == nullptr;
   for (int i = 0; i < b->n; ++i) grow = grow || n[i] > b->h[i].poolcap;
+  HIPT(hipStreamSynchronize(b->stream));  // no launch reads the staging area or the old pools any more
   if (grow) {
-    HIPT(hipStreamSynchronize(b->stream));  // no launch reads the old pools any more
+    for (auto& g : b->gstep) {  // (captured with the old region)
+      if (g) (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
     std::vector<size_t> off(b->n + 1, 0);
     for (int i = 0; i < b->n; ++i) {
       Inst& d = b->h[i];
@@ -3780,23 +3791,10 @@ int amcd_set_pools(amcd_batch* b, const double* const* rot9, const int* n) {
     b->h_pool = hp;
     b->pool_off = off;
     for (int i = 0; i < b->n; ++i) b->h[i].pool = dp + 9 * off[i];
-    if (!b->pool_ev) HIPT(hipEventCreateWithFlags(&b->pool_ev, hipEventDisableTiming));
     if (push_inst(b)) return -1;
-  } else {
-    HIPT(hipEventSynchronize(b->pool_ev));  // the previous copy has read the staging area
   }
-  size_t lo = (size_t)-1, hi = 0;
-  for (int i = 0; i < b->n; ++i) {
-    if (n[i] <= 0 || !rot9[i]) continue;
-    const size_t o = b->pool_off[i];
-    memcpy(b->h_pool + 9 * o, rot9[i], sizeof(double) * 9 * (size_t)n[i]);
-    lo = std::min(lo, o);
-    hi = std::max(hi, o + (size_t)n[i]);
-  }
-  if (hi > lo)
-    HIPT(hipMemcpyAsync(b->d_pool + 9 * lo, b->h_pool + 9 * lo, sizeof(double) * 9 * (hi - lo),
-                        hipMemcpyHostToDevice, b->stream));
-  HIPT(hipEventRecord(b->pool_ev, b->stream));
+  for (int i = 0; i < b->n; ++i)
+    if (n[i] > 0 && rot9[i]) memcpy(b->h_pool + 9 * b->pool_off[i], rot9[i], sizeof(double) * 9 * (size_t)n[i]);
   return 0;
 }
 
@@ -3816,12 +3814,13 @@ static int put_steps(amcd_batch* b, const amcd_step* steps) {
   memcpy(b->h_steps, steps, sizeof(amcd_step) * b->n);
   return 0;
 }
-// the staged step records to the device, with fresh output records when `clear`
+// the staged step records and pools to the device, with fresh output records when `clear`
 static int launch_step_in(amcd_batch* b, bool clear) {
   static_assert(sizeof(amcd_step) % 4 == 0 && sizeof(amcd_out) % 4 == 0, "records copied as words");
   const int ns = (int)(sizeof(amcd_step) / 4) * b->n, no = clear ? (int)(sizeof(amcd_out) / 4) * b->n : 0;
-  hipLaunchKernelGGL(k_step_in, dim3((std::max(ns, no) + 255) / 256), dim3(256), 0, b->stream, (unsigned*)b->d_steps,
-                     (const unsigned*)b->h_steps, ns, (unsigned*)b->d_outs, no);
+  const int nrec = (std::max(ns, no) + 255) / 256;
+  hipLaunchKernelGGL(k_step_in, dim3(nrec + (b->d_pool ? b->n : 0)), dim3(256), 0, b->stream, (unsigned*)b->d_steps,
+                     (const unsigned*)b->h_steps, ns, (unsigned*)b->d_outs, no, b->d_inst, nrec, b->d_pool, b->h_pool);
   HIPT(hipGetLastError());
   return 0;
 }
