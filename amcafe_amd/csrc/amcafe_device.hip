@@ -1894,6 +1894,7 @@ struct LoopShared {
   int fin;  // 1: goes on, 0: finished, -1: pool refill, -2: larger tier, -4: no progress
   double T;
   int go, r_i1, all, neg, nexec;
+  int tied;  // cells whose head can be the first, where a window takes the exact best of every wave
   unsigned cur;  // random engine state
   unsigned long long units;
 };
@@ -2680,6 +2681,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
     double step = DelT * fmin(1.0, 80.0 / (double)max(ns_first, 1));
     int nev = 0;  // events since the bounds were last recomputed
     int want = 44;  // heads asked for
+    int start = 0;  // the first way of filling that the next window tries
     bool resume = go == 2;
     PHASE_INIT(pt);
     for (;;) {
@@ -2718,6 +2720,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         win.done = 0;
         win.scan0 = es.vSind2;
         sh.tn = 0;
+        if constexpr (MEM) sh.tied = 0;
       }
       __syncthreads();
       PHASE(pt, 0);
@@ -2735,7 +2738,12 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         float W = fmaxf(Tf + (float)bins / ibin, u);
         step *= bins >= 32 ? 1.6 : fmax(0.4, (bins + 8) / 26.0);
         // ---- the window's entries
-        int mode = 0;  // 0: clock span, 1: less of it, 2: up to u, 3: exact best of every wave, one event
+        // 0: clock span, 1: less of it, 2: up to u, 3: exact best of every wave, one event.  Where one
+        // window needed that, the next ones hold the same ties (a flat front's cells reach their
+        // neighbours at one time), so in the memory tier, where each way costs a pass over every cell's
+        // state, they begin there while more than a window's are left (118x93x74, 12 thousand growing
+        // cells: 10.9K -> 10.3K cycles per event; in the register tiers the first ways cost little).
+        int mode = start;
         for (;; ++mode) {
           if (mode > 0) W = mode == 1 ? fmaxf(Tf + 0.4f * (W - Tf), u) : u;
           if (mode < 3) {
@@ -2769,19 +2777,21 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
             }
           } else {  // exact best of every wave
             Best b = best_none();
-            int bs = 0;
+            int bs = 0, near = 0;
             double be = 0, bv = 0;
             for (int s0 = tid; s0 < ns; s0 += KR * NT) {
 #pragma unroll
               for (int k = 0; k < KR; ++k) {
                 const int s = s0 + k * NT;
                 const float lo = s < ns ? get_lh<HM>(d, s).x : fInf;
+                if constexpr (MEM) near += lo != fInf && lo <= u;
                 if (lo != fInf && lo <= u)
                   exact_cell<GD>(d, live, s, MEM ? gmem(d.gExt)[s] : c.E[k], MEM ? gmem(d.gVhat)[s] : c.V[k],
                                  get_hd<HM>(d, s).x, b, bs, be, bv);
               }
               if (!MEM) break;
             }
+            if (MEM && near != 0) atomicAdd(&sh.tied, near);
             const Best wb = wave_best(b);
             if (wb.cand >= 0 && wb.cand == b.cand) {
               const int i = put_entry(win, load_rec(d.cand + b.cand), be, bv, b.key, b.cand, bs, -1, order_key(-fInf),
@@ -2796,7 +2806,8 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
           __syncthreads();
         }
         // (as many heads as leave room for what comes on top of them)
-        want = mode > 0 ? max(8, want * 5 / 8) : win.n < 44 ? min(56, want + 2) : win.n > 56 ? want - 1 : want;
+        if (start == 0) want = mode > 0 ? max(8, want * 5 / 8) : win.n < 44 ? min(56, want + 2) : win.n > 56 ? want - 1 : want;
+        if constexpr (MEM) start = mode < 3 ? 0 : sh.tied > WCAP ? 3 : 2;
         {
           // every entry's position by its upper bound: each wave counts a share of the others
           const int n = win.n, j0 = w * (WCAP / NW);
