@@ -88,7 +88,8 @@ int amcd_set_pool(amcd_batch* b, int i, const double* rot9, int n);
 int amcd_set_build(amcd_batch* b, int i, int ngrain);
 int amcd_build_init(amcd_batch* b, int i, long long n_built);
 int amcd_get_build(amcd_batch* b, int i, int* out);
-// every instance's pool in one staged copy (rot9[i] NULL or n[i] = 0: instance i unchanged)
+// every instance's pool staged for the next step or resume, whose first kernel takes it (rot9[i] NULL or
+// n[i] = 0: instance i unchanged)
 int amcd_set_pools(amcd_batch* b, const double* const* rot9, const int* n);
 // graph launches of the step so far (all batches of the process)
 long long amcd_graph_launches(void);

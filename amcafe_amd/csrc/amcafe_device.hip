@@ -1630,8 +1630,8 @@ __global__ void k_clear_npre(Inst* I) {
 // there are few cells), records that are one cache line, and lists and capture constants made by the
 // set-up's parallel pass.  One decision per barrier with the lists built around each event took
 // 6.9K cycles an event in these decks and 13.7K with the state in memory; now (cycles per event, 2.4
-// GHz): 5.5K with few growing cells (at most 300), 2.8K with 3 thousand of a single track or of a
-// raster over a wide plate, 6.7K with 15 thousand (state in memory; 10.1K while a cell without a
+// GHz): 5.3K with few growing cells (at most 300), 2.7K with 3 thousand of a single track or of a
+// raster over a wide plate, 6.5K with 15 thousand (state in memory; 10.1K while a cell without a
 // bound from the set-up, or any step back, ended the window).
 typedef const __attribute__((address_space(4))) Inst CInst;
 struct Best {
