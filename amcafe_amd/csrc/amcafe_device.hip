@@ -257,13 +257,8 @@ __host__ __device__ static inline unsigned int lcg_pow(unsigned long long e) {  
   }
   return (unsigned int)r;
 }
-// two steps back: 16807^-2 mod (2^31-1) = 1407677000^2 mod m (16807 * 1407677000 = 1 mod m)
-__host__ __device__ static inline unsigned int rng_back(unsigned int x) {
-  const unsigned long long inv = 1407677000ull;
-  return mod_m(mod_m((unsigned long long)x * inv) * inv);
-}
 // 16807^(2 d 256^q) mod m: digit q (base 256) of a cell's index, so that the engine is at a cell's two
-// outputs after four products (by squaring, up to 18 cells' index bits took as many dependent pairs)
+// outputs after four products (by squaring, as many dependent pairs as its index has bits)
 struct LcgTable {
   unsigned p[4][256];
 };
@@ -1948,19 +1943,6 @@ __device__ static inline int order_key(float f) {
 }
 // +inf; after every bound; as an entry's limit: BUILD is asked when it is captured
 constexpr int kKeyInf = 0x7f800000, kKeyNone = 0x7fffffff, kKeyAsk = 0x7ffffffe;
-template <int CTRL, int ROWS = 0xf>
-__device__ static inline int dpp_min(int v) {
-  return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xf, false));
-}
-__device__ static inline int wave_min(int v) {
-  v = dpp_min<kQuadX1>(v);
-  v = dpp_min<kQuadX2>(v);
-  v = dpp_min<kHalfMirror>(v);
-  v = dpp_min<kMirror>(v);
-  v = dpp_min<kBcast15, 0xa>(v);
-  v = dpp_min<kBcast31, 0xc>(v);
-  return __builtin_amdgcn_readlane(v, 63);
-}
 __device__ static inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ static inline double uni(double v) {
   const long long b = __double_as_longlong(v);
