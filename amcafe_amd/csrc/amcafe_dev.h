@@ -122,6 +122,7 @@ int amcd_add_layer(amcd_batch* b, int i, int iz1, int ilaserLoc, int gbase, cons
 // (theta, target, grad: 4 per instance; loss: one per instance): mode 0 loss (FP32), 1 loss
 // and gradient (FP32), 2 loss (FP64); amcafe_heat_desc is declared in include/amcafe.h
 struct amcafe_heat_desc_s;
+void amcd_heat_shape(const struct amcafe_heat_desc_s* d, int nsteps, int fp64, int steps, int* out5);
 unsigned long long amcd_heat_last_evals(void);
 // the FP32 batch loss and gradient with every device buffer in a static device array
 // (no allocation): 0 ok, -1 device error, -2 the call needs more than that array holds

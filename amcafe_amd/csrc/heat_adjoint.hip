@@ -25,6 +25,7 @@
 // serves finite differences.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "amcafe_dev.h"
@@ -39,7 +40,7 @@ thread_local unsigned long long g_last_evals = 0;
 template <typename F, bool GRAD>
 int run(const amcafe_heat_desc* d, int nb, const double* theta, const double* target, int step0, int nsteps,
         double* loss, double* grad, float* ms, char* err, int errlen) {
-  const Shape sp = shape_of<F>(d);
+  const Shape sp = shape_of<F>(d, nsteps);
   const size_t nblk = (size_t)sp.groups * sp.runs;
   std::vector<Src> hs;
   sources(nb, theta, target, hs);
@@ -80,5 +81,12 @@ extern "C" int amcd_heat(const amcafe_heat_desc* d, int nb, const double* theta,
   if (mode == 0) return run<float, false>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
   if (mode == 1) return run<float, true>(d, nb, theta, target, step0, nsteps, loss, grad, ms, err, errlen);
   return run<double, false>(d, nb, theta, target, step0, nsteps, loss, nullptr, ms, err, errlen);
+}
+// the launch shape of such a call (for tests): groups, shares, steps per launch, shares' tiles in a launch of
+// `steps` steps, columns of a tile
+extern "C" void amcd_heat_shape(const amcafe_heat_desc* d, int nsteps, int fp64, int steps, int* out5) {
+  const Shape s = fp64 ? shape_of<double>(d, nsteps) : shape_of<float>(d, nsteps);
+  const int v[5] = {s.groups, s.runs, s.seg, s.ctiles(steps), s.ct};
+  std::copy(v, v + 5, out5);
 }
 extern "C" unsigned long long amcd_heat_last_evals(void) { return g_last_evals; }

@@ -474,7 +474,8 @@ struct Bufs {
   unsigned long long* evals;
 };
 
-// The launch shape of a segment of at most `seg` steps: groups of ROWS rows and shares of `per` column
+// The launch shape of a call: segments of at most `checkpoint` steps and no longer than the call (nor than
+// 2^30 columns, so that every count of tiles fits an int), groups of ROWS rows, and shares of `per` column
 // tiles (FP32: 16, so few that the hot tenth of a 256x256x64 domain's 6400 blocks fills the chip; a
 // cold block leaves after its bounds.  Loss / loss and gradient / 32 sets of 128x128x48, ms: 4 tiles
 // 3.22 / 4.34 / 10.2, 8: 3.16 / 4.29 / 9.8, 16: 2.91 / 4.01 / 8.8, 32: 3.32 / 4.48 / 8.7; blocks of 128
@@ -482,43 +483,51 @@ struct Bufs {
 // call's account) unless there are more groups than that (nx = 1: at most twice).  Rows in patches of 8 x 4
 // where the patches' padding is at most 1.9 times the rows and nx makes up for it.
 struct Shape {
-  int groups, runs, ctiles, seg, patch;
+  int groups, runs, seg, patch, nx, ct;
+  // column tiles of each share in a launch of `steps` steps: a segment shorter than the others is
+  // spread over all shares too
+  int ctiles(int steps) const {
+    const long long tiles = ((long long)steps * nx + ct - 1) / ct;
+    return (int)((tiles + runs - 1) / runs);
+  }
 };
-static inline Shape shape(const amcafe_heat_desc* d, int ct, int per, bool patches) {
+static inline Shape shape(const amcafe_heat_desc* d, int nsteps, int ct, int per, bool patches) {
   Shape s;
   const int nx = d->nX[0], ny = d->nX[1], nz = d->nX[2];
-  s.seg = d->checkpoint > 0 ? d->checkpoint : 100;
+  s.nx = nx;
+  s.ct = ct;
+  s.seg = std::min({d->checkpoint > 0 ? d->checkpoint : 100, std::max(nsteps, 1), std::max((1 << 30) / nx, 1)});
   s.patch = patches && nx >= 2 && ny >= 16 && nz >= 8;
   const long long rtiles = s.patch ? (long long)((ny + 7) / 8) * ((nz + 3) / 4) : ((long long)ny * nz + RT - 1) / RT;
   s.groups = (int)((rtiles + HB / 64 - 1) / (HB / 64));
   const long long tiles = ((long long)s.seg * nx + ct - 1) / ct;
   const long long blocks = ((long long)nx * ny * nz + 255) / 256;
   const long long runs = std::max<long long>(1, std::min<long long>({(tiles + per - 1) / per, blocks / s.groups, 65535}));
-  s.ctiles = (int)((tiles + runs - 1) / runs);
-  s.runs = (int)((tiles + s.ctiles - 1) / s.ctiles);
+  const long long share = (tiles + runs - 1) / runs;
+  s.runs = (int)((tiles + share - 1) / share);
   return s;
 }
 template <typename F>
-static Shape shape_of(const amcafe_heat_desc* d) {
-  return sizeof(F) == 8 ? shape(d, CT64, 8, false) : shape(d, CT, 16, true);
+static Shape shape_of(const amcafe_heat_desc* d, int nsteps) {
+  return sizeof(F) == 8 ? shape(d, nsteps, CT64, 8, false) : shape(d, nsteps, CT, 16, true);
 }
 
-// Segments of at most `checkpoint` steps, one launch each (all instances of the batch in it),
+// The call's segments, one launch each (all instances of the batch in it),
 // then the fixed-order reduction; everything on `stream`.  No steps: every slot holds zero.
 template <typename F, bool GRAD>
 static void launch_all(const amcafe_heat_desc* d, int nb, const Bufs<F>& B, int step0, int nsteps,
                        hipStream_t stream) {
-  const Shape h = shape_of<F>(d);
+  const Shape h = shape_of<F>(d, nsteps);
   const Geo g = geo(d);
   const dim3 grid(h.groups, h.runs, nb);
-  for (int m = 0; m == 0 || m < nsteps; m += h.seg) {
-    const int c = std::max(0, std::min(nsteps - m, h.seg));
+  for (long long m = 0; m == 0 || m < nsteps; m += h.seg) {
+    const int c = (int)std::max(0ll, std::min<long long>(nsteps - m, h.seg)), ctiles = h.ctiles(c);
     if constexpr (sizeof(F) == 8)
-      hipLaunchKernelGGL(k_heat64, grid, dim3(HB), 0, stream, g, B.src, B.src + nb, step0 + m, c, h.ctiles, B.part,
+      hipLaunchKernelGGL(k_heat64, grid, dim3(HB), 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles, B.part,
                          m == 0 ? 1 : 0);
     else
-      hipLaunchKernelGGL((k_heat<GRAD>), grid, dim3(HB), 0, stream, g, B.src, B.src + nb, step0 + m, c, h.ctiles, h.patch,
-                         B.part, m == 0 ? 1 : 0, B.evals);
+      hipLaunchKernelGGL((k_heat<GRAD>), grid, dim3(HB), 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles,
+                         h.patch, B.part, m == 0 ? 1 : 0, B.evals);
   }
   hipLaunchKernelGGL((k_heat_reduce<F>), dim3(nb), dim3(256), 0, stream, B.part, h.groups * h.runs, B.out);
 }

@@ -60,7 +60,7 @@ int run_noalloc(const amcafe_heat_desc* d, int nb, const double* theta, const do
     }
     base = (unsigned char*)g_scratch_ptr[dev];
   }
-  const Shape sp = shape_of<float>(d);
+  const Shape sp = shape_of<float>(d, nsteps);
   std::vector<Src> hs;
   sources(nb, theta, target, hs);
   Bufs<float> B;
