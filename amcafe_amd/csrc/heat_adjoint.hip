@@ -61,7 +61,10 @@ int run(const amcafe_heat_desc* d, int nb, const double* theta, const double* ta
   HCHECK(hipEventRecord(e1, 0));
   std::vector<F> h(5 * (size_t)nb);
   HCHECK(hipMemcpy(h.data(), B.out, sizeof(F) * 5 * nb, hipMemcpyDeviceToHost));
-  HCHECK(hipMemcpy(&g_last_evals, B.evals, sizeof(unsigned long long), hipMemcpyDeviceToHost));
+  if constexpr (sizeof(F) == 8)  // (the FP64 loss evaluates every voxel at every step)
+    g_last_evals = (unsigned long long)std::max(nsteps, 0) * d->nX[0] * d->nX[1] * d->nX[2] * nb;
+  else
+    HCHECK(hipMemcpy(&g_last_evals, B.evals, sizeof(unsigned long long), hipMemcpyDeviceToHost));
   float el = 0;
   HCHECK(hipEventElapsedTime(&el, e0, e1));
   (void)hipEventDestroy(e0);
