@@ -2567,14 +2567,16 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
     else if (ns_first > CAP)
       go = -2;  // more growing cells than this tier holds
     else if (ls->pending)
-      go = 2;   // resume with the pending nucleation
+      // resume with the pending nucleation, or ask again: another instance's larger tier relaunches the
+      // loop for all of them, before the host has refilled this one's pool
+      go = ls->pool_used >= n_pool || ls->pool_used >= d.poolcap || ls->nGrain >= d.gcap ? -1 : 2;
     else if (ls->events == 0 && Na == ls->nmushy0)
       go = 0;   // loop condition vSind2 != countS fails at once (S/VoxelsCA.C:381)
     sh.go = go;
     sh.r_i1 = ls->pend_tgt;
     sh.nslots = ns_first;
     sh.T = ls->tinc;
-    sh.fin = go > 0 ? 1 : (go == 0 ? 0 : -2);
+    sh.fin = go > 0 ? 1 : go == -3 ? -2 : go;  // (-1: pool refill, -2: larger tier)
     sh.units = 0;
     sh.back = 0;
     sh.cur = ls->rng;
