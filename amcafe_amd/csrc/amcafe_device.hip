@@ -587,6 +587,10 @@ __global__ __launch_bounds__(GB) void k_easm(Inst* I, const int* bstart, int nin
   if (st.skip) return;
   const int tid = threadIdx.x, v = (blockIdx.x - bstart[ii]) * GB + tid;
   const amcd_params& p = d.p;
+  if (v == 0) {  // planes that can melt: up to the laser's (with a plane of margin)
+    d.ls->zhot0 = 0;
+    d.ls->zhot1 = min(p.nz - 1, (int)floor(st.lz / p.dz - 0.5) + 1);
+  }
   if (tid < AMC_GL25_N) {
     const double slp = kEasmT / 2.0, x = slp + slp * kGLx[tid];
     nd.x[tid] = (st.lx - p.bmV * kEasmT) + p.bmV * x;
