@@ -3379,6 +3379,7 @@ struct amcd_batch {
   amcd_out* d_outs = nullptr;
   amcd_step* h_steps = nullptr;  // pinned
   amcd_out* h_outs = nullptr;    // pinned
+  bool staged = false;  // launched work may still have to read h_steps
   std::vector<void*> allocs;
   hipEvent_t ev[16];
   double last_ms[16] = {0};
@@ -3764,6 +3765,7 @@ int amcd_set_pools(amcd_batch* b, const double* const* rot9, const int* n) {
   bool grow = b->d_pool == nullptr;
   for (int i = 0; i < b->n; ++i) grow = grow || n[i] > b->h[i].poolcap;
   HIPT(hipStreamSynchronize(b->stream));  // no launch reads the staging area or the old pools any more
+  b->staged = false;
   if (grow) {
     for (auto& g : b->gstep) {  // (captured with the old region)
       if (g) (void)hipGraphExecDestroy(g);
@@ -3810,6 +3812,10 @@ int amcd_set_pool(amcd_batch* b, int i, const double* rot9, int n) {
 int amcd_reserve_grains(amcd_batch* b, int i, int need) { return ensure_grains(b, b->h[i], need); }
 
 static int put_steps(amcd_batch* b, const amcd_step* steps) {
+  if (b->staged) {  // (a temperature whose output records nobody has read)
+    HIPT(hipStreamSynchronize(b->stream));
+    b->staged = false;
+  }
   memcpy(b->h_steps, steps, sizeof(amcd_step) * b->n);
   return 0;
 }
@@ -3818,6 +3824,7 @@ static int launch_step_in(amcd_batch* b, bool clear) {
   static_assert(sizeof(amcd_step) % 4 == 0 && sizeof(amcd_out) % 4 == 0, "records copied as words");
   const int ns = (int)(sizeof(amcd_step) / 4) * b->n, no = clear ? (int)(sizeof(amcd_out) / 4) * b->n : 0;
   const int nrec = (std::max(ns, no) + 255) / 256;
+  b->staged = true;
   hipLaunchKernelGGL(k_step_in, dim3(nrec + (b->d_pool ? b->n : 0)), dim3(256), 0, b->stream, (unsigned*)b->d_steps,
                      (const unsigned*)b->h_steps, ns, (unsigned*)b->d_outs, no, b->d_inst, nrec, b->d_pool, b->h_pool);
   HIPT(hipGetLastError());
@@ -3930,6 +3937,7 @@ static int launch_event_loop(amcd_batch* b) {
 
 static int wait_outs(amcd_batch* b, amcd_out* outs) {
   HIPT(hipStreamSynchronize(b->stream));
+  b->staged = false;
   memcpy(outs, b->h_outs, sizeof(amcd_out) * b->n);
   return 0;
 }
@@ -4105,6 +4113,7 @@ static int launch_step_graph(amcd_batch* b) {
     if (capture_graph(b, true, &g)) return -1;
     b->gstep_key[t] = key;
   }
+  b->staged = true;
   HIPT(hipGraphLaunch(g, b->stream));
   g_graph_launches++;
   return 0;
