@@ -137,7 +137,7 @@ struct LoopState {
   int nGrain;
   int pool_used;
   unsigned int rng;  // minstd_rand0 state
-  int nslots_pre;    // slots whose lists the step's set-up built (-1 before the loop runs)
+  int nslots_pre;    // slots whose entries have a CapRec (-1 before the loop runs)
   long long draws;
   double tinc;
   int events, captures, nucs, done;
@@ -223,12 +223,15 @@ struct Inst {
   double *gExt, *gVhat;
   float2* gLH;      // per slot: capture-clock bounds (lo, hi) of the memory-resident tier
   int2* gHd;        // per slot: list head (entry, target) of the memory-resident tier
-  // Lists: slot s's at 26 s when the set-up or the loop built it; from 26 acap on, the lists that
-  // the set-up built ahead for the cells that captures would create.
+  // Lists: first those that the set-up built ahead for the cells that captures would create (`precap`
+  // entries at most), then slot s's at precap + 26 s, when the set-up or the loop built it.
+  // The entries ahead and those of the set-up's first `capslots` lists have a CapRec, the others their
+  // shape factor (at the entry's place less precap), from which a capture is re-centred when it
+  // happens: far fewer cells grow than are active, and a CapRec for every active cell took 1.25 of 3.3 KB.
   CandRec* cand;
-  double* cF;       // per entry: shape factor
-  CapRec* cap;      // per entry (of the lists that the set-up built)
-  int precap;       // entries that the lists built ahead may take
+  CapRec* cap;
+  double* cF;
+  int precap, capslots;
   // grains
   int gcap;
   double* rot;
@@ -1271,7 +1274,7 @@ __global__ __launch_bounds__(GB) void k_active_setup(Inst* I, const int* bstart,
     const int G = d.aG[a];
     const bool bad = G < 1 || G > d.gcap;  // a growing cell must carry a valid grain
     if (bad) atomicOr(&O[ii].err_state, 1);
-    d.slots[slot] = {{d.aCx[a], d.aCy[a], d.aCz[a]}, d.aVox[a], G, a, d.aScan[a], slot * AMCD_NB, bad ? -1 : 0};
+    d.slots[slot] = {{d.aCx[a], d.aCy[a], d.aCz[a]}, d.aVox[a], G, a, d.aScan[a], d.precap + slot * AMCD_NB, bad ? -1 : 0};
   }
 }
 
@@ -1492,14 +1495,15 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
   }
   const unsigned long long bal = __ballot(liq);
   const int n = (int)__popcll(bal);
-  const size_t cb = (size_t)slot * AMCD_NB;
+  const size_t cb = d.precap + (size_t)slot * AMCD_NB;
   const int rank = list_rank(D, r, liq, -1);
   int pre = -1;
   // the lists ahead, for the entries whose target would grow
   const int half = lane >> 5, q = lane & 31;
   const int qq = q < 13 ? q : q + 1, ddx = qq % 3 - 1, ddy = (qq / 3) % 3 - 1, ddz = qq / 9 - 1;
   // and whose capture the step has time for (a step's last event may come later: its list is made then)
-  const bool soon = !(D > d.gExt[slot] + d.gVhat[slot] * p.DelT * (1 + 1e-6));
+  const bool recs = slot < d.capslots;  // the entries have a CapRec
+  const bool soon = recs && !(D > d.gExt[slot] + d.gVhat[slot] * p.DelT * (1 + 1e-6));
   for (unsigned todo = (unsigned)__ballot(liq && cold && soon); todo != 0;) {
     const int j0 = __builtin_ctz(todo);
     todo &= todo - 1;
@@ -1543,10 +1547,9 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     if (lane == 0) base = atomicAdd(&d.ls->npre, na + nb);
     base = __builtin_amdgcn_readfirstlane(base);
     const bool fits = base >= 0 && base <= d.precap - na - nb;
-    const size_t at = (size_t)d.acap * AMCD_NB + (half ? base + na : base);
+    const int at = half ? base + na : base;
     if (on && fits) {
       d.cand[at + rank2] = {D2, r2, t2, tn2, back2, (short)q, (short)((half ? nb : na) - rank2)};
-      d.cF[at + rank2] = f2;
       d.cap[at + rank2] = cr;
     }
     // the time to the new cell's first capture
@@ -1556,19 +1559,19 @@ __device__ static inline void grow_list(const Inst& d, int slot, int lane) {
     if (fa != 0) {
       const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tn), __builtin_ctz(fa)));
       tnew = lane == j0 ? x : tnew;
-      pre = lane == j0 && fits ? d.acap * AMCD_NB + base : pre;
+      pre = lane == j0 && fits ? base : pre;
     }
     if (fb != 0) {
       const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tn), 32 + __builtin_ctz(fb)));
       tnew = lane == j1 ? x : tnew;
-      pre = lane == j1 && fits ? d.acap * AMCD_NB + base + na : pre;
+      pre = lane == j1 && fits ? base + na : pre;
     }
   }
   if (liq) {
     if (cold && !soon) tnew = -__builtin_inff();
     d.cand[cb + rank] = {D, r, t, tnew, cold ? back_bound(rc.w, V) : __builtin_inff(), (short)lane, (short)(n - rank)};
-    d.cF[cb + rank] = f;
-    d.cap[cb + rank] = {rc.x, rc.y, rc.z, rc.w, pre, sr.G, V};
+    if (!recs) d.cF[(size_t)slot * AMCD_NB + rank] = f;
+    else d.cap[cb + rank] = {rc.x, rc.y, rc.z, rc.w, pre, sr.G, V};
   }
   if (lane == 0) d.slots[slot].n = n;
 }
@@ -2205,7 +2208,7 @@ __device__ __attribute__((noinline)) static Octahedron recentre_out(const Inst* 
   double R[9], o[3], e;
 #pragma unroll
   for (int q = 0; q < 9; ++q) R[q] = gmem(d.rot)[9 * (size_t)(G - 1) + q];
-  recentre(d, q->vox, v1, c, R, gmem(d.cF)[cand], o, &e);
+  recentre(d, q->vox, v1, c, R, gmem(d.cF)[cand - d.precap], o, &e);
   return {o[0], o[1], o[2], e};
 }
 __device__ __attribute__((noinline)) static double velocity_out(const Inst* I, double T) {
@@ -2247,7 +2250,7 @@ __device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb,
     q[0] = v2d{D, r};
     const int none = __float_as_int(-__builtin_inff());
     q[1] = v2d{pack2(tn, none), pack2(none, lane | (n - rank) << 16)};
-    gmem(d.cF)[cb + rank] = f;
+    gmem(d.cF)[cb - d.precap + rank] = f;
   }
 }
 
@@ -2256,15 +2259,14 @@ __device__ __attribute__((noinline)) static void list_out(const Inst* I, int cb,
 // of loads: the captured cell's row by lanes 0..31, the entry's capture by lanes 32..43.
 template <bool GD>
 __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh, Window& win, const Liveness<GD>& live,
-                                         int ent, int k, int ns_pre, int nm0) {
+                                         int ent, int k, int nrec, int nm0) {
   typedef double v2d __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
   auto& p = d.p;
   const int evi = lane <= k ? lds_get(&win.ev[lane]).y : -1;  // lane j: voxel of event j
   const int i1 = __builtin_amdgcn_readlane(evi, k), scan = uni(win.scan0) + k;
   const int cand = ent >= 0 ? uni(win.cand[ent]) : -1, sw = ent >= 0 ? uni(win.own[ent]) : -1;
-  // an entry of a list the set-up built (the cells' own, and those ahead)
-  const bool first = cand >= 0 && (cand < ns_pre * AMCD_NB || cand >= d.acap * AMCD_NB);
+  const bool first = cand >= 0 && cand < nrec;  // it has a CapRec
   const int* at = (const int*)(d.aRow + i1) + (lane & 31);
   if (lane >= 32) at = first ? (const int*)(d.cap + cand) + min(lane - 32, 11) : at;
   const int x = gmem(at)[0];
@@ -2287,7 +2289,7 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
     E0 = word2(38);
     pre = __builtin_amdgcn_readlane(x, 40);
     G = __builtin_amdgcn_readlane(x, 41);
-  } else if (ent >= 0) {  // by a cell made in this launch
+  } else if (ent >= 0) {  // by a cell made in this launch, or beyond the slots with a CapRec
     G = uni(gmem(d.slots)[sw].G);
     const Octahedron o = recentre_out(I, sw, cand, v1);
     cen[0] = uni(o.x);
@@ -2305,7 +2307,7 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
   if (grows) {
     if (lane == 0) slot = atomicAdd(&sh.nslots, 1);
     slot = uni(slot);
-    cb = pre >= 0 ? pre : slot * AMCD_NB;
+    cb = pre >= 0 ? pre : d.precap + slot * AMCD_NB;
     const double V0 = (T1 == p.tS) & (T1 < p.tL) ? p.vhat_tS : velocity_out(I, T1);
     if (lane == 0 && ent >= 0 && win.lim[ent] == kKeyAsk) win.back[ent] = back_bound(E0, V0);
     if (pre < 0) {
@@ -2339,7 +2341,7 @@ __device__ static inline void build_cell(CInst& d, const Inst* I, LoopShared& sh
 // when it is done); out of line: its registers do not add to those that hold the cells.  The
 // engine ends after at most WCAP events whatever these waves do, so the wait ends.
 template <bool GD>
-__device__ __attribute__((noinline)) static void build_cells(const Inst* I, int first, int step, int ns_pre, int nm0) {
+__device__ __attribute__((noinline)) static void build_cells(const Inst* I, int first, int step, int nrec, int nm0) {
   CInst& d = *(CInst*)I;
   Window& win = s_loop.win;
   const Liveness<GD> live = {s_dead_bits, d.aVS};
@@ -2352,7 +2354,7 @@ __device__ __attribute__((noinline)) static void build_cells(const Inst* I, int 
       __builtin_amdgcn_s_sleep(1);
     }
     if (ent == -2) break;
-    build_cell<GD>(d, I, s_loop, win, live, ent, k, ns_pre, nm0);
+    build_cell<GD>(d, I, s_loop, win, live, ent, k, nrec, nm0);
   }
 }
 
@@ -2436,7 +2438,7 @@ __device__ static inline int put_entry(Window& win, const CandRec& e, double E, 
 }
 template <bool GD>
 __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Window& win, int s, double E, double V,
-                                        int c1, float lo, float hi, double T, float W, int ns_pre) {
+                                        int c1, float lo, float hi, double T, float W, int nrec) {
   const int scan = gmem(d.slots)[s].scan;
   bool first = true;
   for (int p = c1;; p += 2) {
@@ -2460,7 +2462,7 @@ __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Wind
       const float tn = e[q].tn;
       const float x = lo + tn - 0x1p-20f * (fabsf(lo) + fabsf(tn));
       int lim = tn == -__builtin_inff() ? kKeyAsk : tn == __builtin_inff() ? kKeyNone : order_key(x) - 2;
-      if ((lim < order_key(W) || lim == kKeyAsk) && (p + q < ns_pre * AMCD_NB)) {
+      if ((lim < order_key(W) || lim == kKeyAsk) && p + q >= d.precap && p + q < nrec) {
         const CapRec cr = d.cap[p + q];
         if (cr.pre >= 0) {
           lim = kKeyNone;
@@ -2546,7 +2548,8 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
   const int n_pool = S[blockIdx.x].n_pool;
   const int Na = ls->Na;
   const int ns_first = ls->nslots;
-  const int ns_pre = ls->nslots_pre < 0 ? ns_first : ls->nslots_pre;  // slots the set-up made
+  const int ns_pre = min(ls->nslots_pre < 0 ? ns_first : ls->nslots_pre, d.capslots);  // slots whose entries have a CapRec
+  const int nrec = d.precap + ns_pre * AMCD_NB;  // entries that have one
   const Liveness<GD> live = {s_dead_bits, d.aVS};
   if (!GD && Na <= AMCD_DEAD_BITS) {  // liveness bitmap from the current states
     for (int wd = tid; wd < (Na + 31) / 32; wd += NT) {
@@ -2759,7 +2762,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
                   }
                 }
                 const float2 b = get_lh<HM>(d, s);
-                push_cell<GD>(d, live, win, s, E, V, get_hd<HM>(d, s).x, b.x, b.y, T, W, ns_pre);
+                push_cell<GD>(d, live, win, s, E, V, get_hd<HM>(d, s).x, b.x, b.y, T, W, nrec);
               }
               if (!MEM) break;
             }
@@ -2841,7 +2844,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       resume = false;
       PHASE(pt, 2);
       // ---- BUILD, while the engine goes on
-      if (w > 0) build_cells<GD>(I + blockIdx.x, w - 1, NW - 1, ns_pre, nm0);
+      if (w > 0) build_cells<GD>(I + blockIdx.x, w - 1, NW - 1, nrec, nm0);
       __syncthreads();
       PHASE(pt, 3);
       T = sh.T;
@@ -3452,8 +3455,11 @@ static int alloc_wanted(amcd_batch* b) {
 static void want_active(amcd_batch* b, Inst& d, int acap) {
   d.acap = acap;
   size_t c = (size_t)acap;
-  // about 80 entries per growing cell, of which there are far fewer than active cells
-  d.precap = (int)std::min<size_t>(8 * c, (size_t)1 << 26);
+  // Growing cells are a tenth of the active ones in a raster, and what they need beyond a list of their
+  // own is sized for a quarter: records of captures, and about 27 entries of lists ahead each.  2.15 KB per
+  // active cell in all; cells beyond that go without (see Inst::cand).
+  d.capslots = (int)(c / 4);
+  d.precap = (int)std::min<size_t>(6 * c, (size_t)1 << 26);
   if (c * AMCD_NB + (size_t)d.precap > 0x7fffff00ull) d.precap = 0;  // entries are counted in 32 bits
   want(b, &d.aVox, c);
   want(b, &d.aVS, c);
@@ -3473,8 +3479,8 @@ static void want_active(amcd_batch* b, Inst& d, int acap) {
   want(b, &d.gLH, c);
   want(b, &d.gHd, c);
   want(b, &d.cand, c * AMCD_NB + d.precap);
-  want(b, &d.cF, c * AMCD_NB + d.precap);
-  want(b, &d.cap, c * AMCD_NB + d.precap);
+  want(b, &d.cap, (size_t)d.capslots * AMCD_NB + d.precap);
+  want(b, &d.cF, c * AMCD_NB);
 }
 
 static int push_inst(amcd_batch* b) {
@@ -4389,6 +4395,16 @@ double amcd_host_pow(double x, double y) { return amc_pow_cr(x, y); }
 int amcd_host_pow_n(const double* x, const double* y, int n, double* out) {
   for (int i = 0; i < n; ++i) out[i] = amc_pow_cr(x[i], y[i]);
   return 0;
+}
+
+// device memory that an active-list capacity takes (for tests)
+size_t amcd_active_bytes(int acap) {
+  amcd_batch b;
+  Inst d = {};
+  want_active(&b, d, acap);
+  size_t total = 0;
+  for (const auto& w : b.wanted) total += w.second;
+  return total;
 }
 
 // the capture shape factor evaluated by the host build of the device math
