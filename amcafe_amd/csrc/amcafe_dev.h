@@ -157,6 +157,7 @@ int amcd_uniform_jump(unsigned long long seed, int n, double* out);
 // host build of the device's shape factor pow(cos th sin ph, .5), n vectors xyz
 int amcd_host_shape_factor(const double* dnx, int n, double* out);
 size_t amcd_active_bytes(int acap);
+double amcd_window_span(double span, int bins, int mode, double DelT, int cells);
 double amcd_host_pow(double x, double y);
 int amcd_host_pow_n(const double* x, const double* y, int n, double* out);
 

@@ -1855,6 +1855,18 @@ __device__ unsigned long long g_phase[32];
 #endif
 
 // ---- windows
+// Clock span of a window (the histogram's scale), adapted to the heads it gets: about half of the growing
+// cells have a candidate within a step.  A window that had to fall back to its smallest clock value (mode
+// 2 or more: a flat front's ties) says nothing of the span.  Bounded on both sides: hundreds of
+// windows in a row that take a few heads, or too many, would bring it to infinity or zero, and every
+// later window to one event.
+__host__ __device__ static inline double first_span(double DelT, int cells) {
+  return DelT * fmin(1.0, 80.0 / (double)(cells > 1 ? cells : 1));
+}
+__host__ __device__ static inline double next_span(double span, int bins, int mode, double DelT, int cells) {
+  if (mode < 2) span *= bins >= 32 ? 1.6 : fmax(0.4, (bins + 8) / 26.0);
+  return fmin(fmax(span, 0x1p-10 * first_span(DelT, cells)), 64 * DelT);
+}
 constexpr int WCAP = 64;   // entries of a window: one per lane of the engine wave
 constexpr int TCAP = 256;  // touched cells (heads that died) listed per window
 struct Window {
@@ -2549,7 +2561,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
   const int Na = ls->Na;
   const int ns_first = ls->nslots;
   const int ns_pre = min(ls->nslots_pre < 0 ? ns_first : ls->nslots_pre, d.capslots);  // slots whose entries have a CapRec
-  const int nrec = d.precap + ns_pre * AMCD_NB;  // entries that have one
+  const int nrec = uni(d.precap + ns_pre * AMCD_NB);  // entries that have one
   const Liveness<GD> live = {s_dead_bits, d.aVS};
   if (!GD && Na <= AMCD_DEAD_BITS) {  // liveness bitmap from the current states
     for (int wd = tid; wd < (Na + 31) / 32; wd += NT) {
@@ -2667,9 +2679,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       }
     }
     refresh_own(true, 0, 0, 0.0, T);
-    // clock span of a window, adapted to the entries it gets (about half of the growing cells
-    // have a candidate within a step)
-    double step = DelT * fmin(1.0, 80.0 / (double)max(ns_first, 1));
+    double step = first_span(DelT, ns_first);  // clock span of a window
     int nev = 0;  // events since the bounds were last recomputed
     int want = 44;  // heads asked for
     int start = 0;  // the first way of filling that the next window tries
@@ -2727,7 +2737,6 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         cum += __builtin_amdgcn_update_dpp(0, cum, kBcast15, 0xa, 0xf, false);
         const int bins = __popcll(__ballot(lane < 32 && cum <= want));
         float W = fmaxf(Tf + (float)bins / ibin, u);
-        step *= bins >= 32 ? 1.6 : fmax(0.4, (bins + 8) / 26.0);
         // ---- the window's entries
         // 0: clock span, 1: less of it, 2: up to u, 3: exact best of every wave, one event.  Where one
         // window needed that, the next ones hold the same ties (a flat front's cells reach their
@@ -2796,6 +2805,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
           if (tid == 0) win.n = 0;
           __syncthreads();
         }
+        step = next_span(step, bins, mode, DelT, ns_first);
         // (as many heads as leave room for what comes on top of them)
         if (start == 0) want = mode > 0 ? max(8, want * 5 / 8) : win.n < 44 ? min(56, want + 2) : win.n > 56 ? want - 1 : want;
         if constexpr (MEM) start = mode < 3 ? 0 : sh.tied > WCAP ? 3 : 2;
@@ -4397,6 +4407,10 @@ int amcd_host_pow_n(const double* x, const double* y, int n, double* out) {
   return 0;
 }
 
+// the clock span of the window after one that took `bins` of the histogram in `mode` (for tests)
+double amcd_window_span(double span, int bins, int mode, double DelT, int cells) {
+  return span < 0.0 ? first_span(DelT, cells) : next_span(span, bins, mode, DelT, cells);
+}
 // device memory that an active-list capacity takes (for tests)
 size_t amcd_active_bytes(int acap) {
   amcd_batch b;
