@@ -156,6 +156,7 @@ int amcd_uniform_stream(unsigned long long seed, int n, double* out);
 int amcd_uniform_jump(unsigned long long seed, int n, double* out);
 // host build of the device's shape factor pow(cos th sin ph, .5), n vectors xyz
 int amcd_host_shape_factor(const double* dnx, int n, double* out);
+float amcd_step_back(double e, double v);
 size_t amcd_active_bytes(int acap);
 double amcd_window_span(double span, int bins, int mode, double DelT, int cells);
 double amcd_host_pow(double x, double y);

@@ -1867,6 +1867,18 @@ __host__ __device__ static inline double next_span(double span, int bins, int mo
   if (mode < 2) span *= bins >= 32 ? 1.6 : fmax(0.4, (bins + 8) / 26.0);
   return fmin(fmax(span, 0x1p-10 * first_span(DelT, cells)), 64 * DelT);
 }
+// How far the clock may step back before a half-diagonal e of velocity v is zero, in single precision (the
+// loop takes 2^-16 off for the rounding): e/v; nothing for a velocity whose reciprocal would leave that
+// range (0 times infinity, not a number, would be dropped from the minimum over the cells).
+__host__ __device__ static inline float step_back(double e, double v) {
+  const float f = (float)v;
+#ifdef __HIP_DEVICE_COMPILE__
+  const float y = __builtin_amdgcn_rcpf(f);
+#else
+  const float y = 1.0f / f;
+#endif
+  return f > 1e-30f ? fmaxf((float)e * y, 0.0f) : v > 0.0 ? 0.0f : __builtin_inff();
+}
 constexpr int WCAP = 64;   // entries of a window: one per lane of the engine wave
 constexpr int TCAP = 256;  // touched cells (heads that died) listed per window
 struct Window {
@@ -2931,9 +2943,6 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       // before the window; a nucleation's time is 0: E + V*0 = E
       bool neg = false;
       float back = fInf;  // CandRec::back over the cells, after the window
-      auto step_back = [](double e, double v) {
-        return v > 0.0 ? e > 0.0 ? (float)e * __builtin_amdgcn_rcpf((float)v) : 0.0f : __builtin_inff();
-      };
       for (int s0 = w * 64; s0 < ns; s0 += KR * NT) {
         if constexpr (MEM) {
 #pragma unroll
@@ -4411,6 +4420,8 @@ int amcd_host_pow_n(const double* x, const double* y, int n, double* out) {
 double amcd_window_span(double span, int bins, int mode, double DelT, int cells) {
   return span < 0.0 ? first_span(DelT, cells) : next_span(span, bins, mode, DelT, cells);
 }
+// the step back that a cell allows (for tests)
+float amcd_step_back(double e, double v) { return step_back(e, v); }
 // device memory that an active-list capacity takes (for tests)
 size_t amcd_active_bytes(int acap) {
   amcd_batch b;
