@@ -62,8 +62,8 @@ typedef struct {
   double tinc;
   int overflow;        // active list exceeded capacity
   int err_state;        // a growing cell carried no valid grain id (the domain state is corrupt)
-  long long slot_visits;  // growing cells with live candidates, summed over the loop's scans
-  long long cand_evals;   // capture times evaluated, summed over the loop's scans
+  long long slot_visits;  // growing cells whose candidates were looked at, summed over the loop's scans
+  long long cand_evals;   // candidates whose time was evaluated or bounded for a scan's window, and times compared
   long long interface_events;  // growing-list length summed over the loop's events
   long long loop_cycles;       // shader-clock cycles of the capture loop, summed over its launches
 } amcd_out;

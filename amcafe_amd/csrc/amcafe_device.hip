@@ -1923,6 +1923,7 @@ struct LoopShared {
   int tied;  // cells whose head can be the first, where a window takes the exact best of every wave
   unsigned cur;  // random engine state
   unsigned long long units;
+  unsigned seen[8], exact[8];  // per wave: cells that the windows looked at, and exact times of theirs
 };
 
 // The workgroup's exchange: the window, the liveness bitmap and, for the register tiers, every
@@ -2004,7 +2005,7 @@ struct EngineState {
   double T;
   int vSind2, nGrain, pool_used, events, captures, nucs;
   int nd;  // draws consumed
-  int visits;
+  long long visits;  // candidates bounded as entries, and times compared
 };
 constexpr int kPending = 0x7fc00bad;  // (no float result has these bits)
 struct EngineRun {
@@ -2494,7 +2495,7 @@ __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Wind
             const CandRec ec = load_rec(d.cand + pc);
             float l, h;
             tau_bounds(ec.D, cr.E, cr.V, 0.0, l, h);
-            const int lk = order_key(lo + l) - 1, hk = order_key(hi + h) + 1;
+                const int lk = order_key(lo + l) - 1, hk = order_key(hi + h) + 1;
             if (l == __builtin_inff() || lk > order_key(W)) break;
             if (l == -__builtin_inff()) {  // (no bound)
               lim = kKeyAsk;
@@ -2517,15 +2518,17 @@ __device__ static inline void push_cell(CInst& d, const Liveness<GD>& live, Wind
 }
 
 // The exact best candidate of one cell (its head and the entries tied with it in time) against
-// b (S/VoxelsCA.C:420-440).
+// b (S/VoxelsCA.C:420-440).  Returns the times evaluated.
 template <bool GD>
-__device__ static inline void exact_cell(CInst& d, const Liveness<GD>& live, int s, double E, double V, int c1, Best& b,
+__device__ static inline int exact_cell(CInst& d, const Liveness<GD>& live, int s, double E, double V, int c1, Best& b,
                                          int& bs, double& be, double& bv) {
   const int scan = gmem(d.slots)[s].scan;
   double t1 = 0.0;
+  int evals = 0;
   for (int p = c1;; ++p) {
     const CandRec e = load_rec(d.cand + p);
     const double t = (e.D - E) / V;
+    ++evals;
     if (p == c1) {
       t1 = t;
       if (!(t1 <= 1e6)) break;
@@ -2545,6 +2548,7 @@ __device__ static inline void exact_cell(CInst& d, const Liveness<GD>& live, int
     }
     if (e.n <= 1) break;
   }
+  return evals;
 }
 
 // GD: an interface of more than AMCD_DEAD_BITS cells, whose liveness is read from the states
@@ -2628,6 +2632,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
   es.nd = 0;
   es.visits = 0;
   unsigned long long units = 0;
+  unsigned seen = 0, exact = 0;  // cells whose candidates this thread has looked at, and exact times of theirs
   Cells<KR> c;
   if (go > 0) {
     const unsigned int aj = lcg_pow(2ull * lane + 1);
@@ -2783,6 +2788,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
                   }
                 }
                 const float2 b = get_lh<HM>(d, s);
+                ++seen;
                 push_cell<GD>(d, live, win, s, E, V, get_hd<HM>(d, s).x, b.x, b.y, T, W, nrec);
               }
               if (!MEM) break;
@@ -2797,9 +2803,11 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
                 const int s = s0 + k * NT;
                 const float lo = s < ns ? get_lh<HM>(d, s).x : fInf;
                 if constexpr (MEM) near += lo != fInf && lo <= u;
-                if (lo != fInf && lo <= u)
-                  exact_cell<GD>(d, live, s, MEM ? gmem(d.gExt)[s] : c.E[k], MEM ? gmem(d.gVhat)[s] : c.V[k],
-                                 get_hd<HM>(d, s).x, b, bs, be, bv);
+                if (lo != fInf && lo <= u) {
+                  ++seen;
+                  exact += exact_cell<GD>(d, live, s, MEM ? gmem(d.gExt)[s] : c.E[k], MEM ? gmem(d.gVhat)[s] : c.V[k],
+                                          get_hd<HM>(d, s).x, b, bs, be, bv);
+                }
               }
               if (!MEM) break;
             }
@@ -2813,6 +2821,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
           }
           __syncthreads();
           if (win.n <= WCAP) break;
+          es.visits += win.n;
           __syncthreads();
           if (tid == 0) win.n = 0;
           __syncthreads();
@@ -2824,6 +2833,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         {
           // every entry's position by its upper bound: each wave counts a share of the others
           const int n = win.n, j0 = w * (WCAP / NW);
+          es.visits += mode < 3 ? n : 0;
           if (lane < n && j0 < n) {
             const int h = win.hi[lane];
             int before = 0;
@@ -3077,6 +3087,14 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       }
     }
   }
+  for (int o = 32; o >= 1; o >>= 1) {
+    seen += __shfl_xor(seen, o);
+    exact += __shfl_xor(exact, o);
+  }
+  if (lane == 0) {
+    sh.seen[w] = seen;
+    sh.exact[w] = exact;
+  }
   if (tid == 0) sh.nexec = es.vSind2 - nm0;
   __syncthreads();
   // ---- loop state and counters
@@ -3120,8 +3138,11 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
     o.tinc = es.T;
     o.draws = ls->draws;
     o.interface_events += (long long)(units + sh.units);
-    o.slot_visits += es.visits;
     o.cand_evals += es.visits;
+    for (int q = 0; q < NW; ++q) {
+      o.slot_visits += sh.seen[q];
+      o.cand_evals += sh.exact[q];
+    }
     o.loop_cycles += (long long)(clock64() - c_start);
   }
 }

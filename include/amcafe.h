@@ -77,8 +77,10 @@ typedef struct {
   int nGrain;          /* grains after the step */
   long long draws;     /* minstd_rand0 outputs consumed */
   double tinc;         /* time advanced by the capture loop */
-  long long slot_visits; /* growing cells with live candidates, summed over the loop's scans */
-  long long cand_evals;  /* capture times evaluated, summed over the loop's scans */
+  long long slot_visits; /* growing cells whose candidates were looked at, summed over the loop's scans
+                            (one or more for a window of events) */
+  long long cand_evals;  /* candidates whose capture time was evaluated or bounded for a scan's window,
+                            and times compared in deciding the events */
   long long interface_events; /* growing cells summed over the capture loop's events (the
                                  cells the reference scans per event, S/VoxelsCA.C:386-400) */
   long long loop_cycles;      /* the capture loop's duration in shader-clock cycles (read by
