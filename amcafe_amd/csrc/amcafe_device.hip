@@ -3253,7 +3253,7 @@ __global__ void k_remap(int* gid, int N, const int* remap, int ngrain) {
 //   powder layer (S/VoxelsCA.C:920-933): voxel corners (i dx, j dy, (z0 + k) dz), planes
 //     z0..z0+nz-1 (planes above the domain included, as the reference labels them);
 //     best distance starts at 1e6, strict <.
-// A block takes a brick of 8x8x4 voxels.  No site whose distance from the brick's box exceeds the
+// A block takes a brick of 8x8x4 voxels at a time.  No site whose distance from the brick's box exceeds the
 // least of the sites' largest distances to it can be a voxel's nearest (with a margin far
 // above rounding), so the block first finds that least distance, one site a thread, and then every voxel
 // looks at the remaining sites, in draw order, from LDS: some tens of them instead of all.  Plate mode
@@ -3268,10 +3268,7 @@ __global__ __launch_bounds__(VOR_B) void k_voronoi(Inst* I, int ii, int z0, int 
   __shared__ int si[VOR_B], sn[VOR_B / 64];
   const Inst& d = I[ii];
   const int nx = d.p.nx, ny = d.p.ny, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int bx = (nx + 7) / 8, by = (ny + 7) / 8;
-  const int b = blockIdx.x, kb = b / (bx * by), jb = (b - kb * bx * by) / bx, ib = b - (kb * by + jb) * bx;
-  const int i = 8 * ib + (tid & 7), j = 8 * jb + ((tid >> 3) & 7), k = 4 * kb + (tid >> 6);
-  const bool in = i < nx && j < ny && k < nz;
+  const int bx = (nx + 7) / 8, by = (ny + 7) / 8, nb = bx * by * ((nz + 3) / 4);
   const double dx = d.p.dx, dy = d.p.dy, dz = d.p.dz;
   auto at = [&](int i, int j, int k, double& x, double& y, double& z) {
     if (LAYER) {
@@ -3284,73 +3281,77 @@ __global__ __launch_bounds__(VOR_B) void k_voronoi(Inst* I, int ii, int z0, int 
       z = ((double)(z0 + k) + .5) * dz;
     }
   };
-  double x, y, z, lo[3], hi[3];
-  at(i, j, k, x, y, z);
-  at(8 * ib, 8 * jb, 4 * kb, lo[0], lo[1], lo[2]);
-  at(min(nx, 8 * ib + 8) - 1, min(ny, 8 * jb + 8) - 1, min(nz, 4 * kb + 4) - 1, hi[0], hi[1], hi[2]);
-  double far = __builtin_huge_val();
-  for (int q = tid; q < ng; q += VOR_B) {
-    double s2 = 0.0;
-    for (int c = 0; c < 3; ++c) {
-      const double s = xs[3 * q + c], m = fmax(fabs(s - lo[c]), fabs(s - hi[c]));
-      s2 += m * m;
-    }
-    far = fmin(far, s2);
-  }
-  for (int o = 32; o >= 1; o >>= 1) far = fmin(far, __shfl_xor(far, o));
-  if (lane == 0) su[w] = far;
-  __syncthreads();
-  for (int q = 0; q < VOR_B / 64; ++q) far = fmin(far, su[q]);
-  far *= 1 + 1e-9;
-  double bd = LAYER ? 1e6 : __builtin_huge_val();
-  int best = 0;
-  for (int c0 = 0; c0 < ng; c0 += VOR_B) {
-    double s[3] = {0.0, 0.0, 0.0}, near = 0.0;
-    bool keep = false;
-    if (c0 + tid < ng) {
+  for (int b = blockIdx.x; b < nb; b += gridDim.x) {
+    const int kb = b / (bx * by), jb = (b - kb * bx * by) / bx, ib = b - (kb * by + jb) * bx;
+    const int i = 8 * ib + (tid & 7), j = 8 * jb + ((tid >> 3) & 7), k = 4 * kb + (tid >> 6);
+    const bool in = i < nx && j < ny && k < nz;
+    double x, y, z, lo[3], hi[3];
+    at(i, j, k, x, y, z);
+    at(8 * ib, 8 * jb, 4 * kb, lo[0], lo[1], lo[2]);
+    at(min(nx, 8 * ib + 8) - 1, min(ny, 8 * jb + 8) - 1, min(nz, 4 * kb + 4) - 1, hi[0], hi[1], hi[2]);
+    double far = __builtin_huge_val();
+    for (int q = tid; q < ng; q += VOR_B) {
+      double s2 = 0.0;
       for (int c = 0; c < 3; ++c) {
-        s[c] = xs[3 * (c0 + tid) + c];
-        const double m = fmax(0.0, fmax(lo[c] - s[c], s[c] - hi[c]));
-        near += m * m;
+        const double s = xs[3 * q + c], m = fmax(fabs(s - lo[c]), fabs(s - hi[c]));
+        s2 += m * m;
       }
-      keep = !(near > far);
+      far = fmin(far, s2);
     }
-    const unsigned long long bal = __ballot(keep);
-    if (lane == 0) sn[w] = __popcll(bal);
-    __syncthreads();  // (the last sites have been looked at)
-    int base = 0, m = 0;
-    for (int q = 0; q < VOR_B / 64; ++q) {
-      base += q < w ? sn[q] : 0;
-      m += sn[q];
-    }
-    if (keep) {
-      const int p = base + __popcll(bal & ((1ull << lane) - 1));
-      sx[p] = s[0];
-      sy[p] = s[1];
-      sz[p] = s[2];
-      si[p] = c0 + tid;
-    }
+    for (int o = 32; o >= 1; o >>= 1) far = fmin(far, __shfl_xor(far, o));
+    if (lane == 0) su[w] = far;
     __syncthreads();
-    for (int q = 0; q < m; ++q) {
-      const double ax = x - sx[q], ay = y - sy[q], az = z - sz[q];
-      const double dd = ax * ax + ay * ay + az * az;
-      const bool lt = dd < bd;
-      bd = lt ? dd : bd;
-      best = lt ? si[q] : best;
+    for (int q = 0; q < VOR_B / 64; ++q) far = fmin(far, su[q]);
+    far *= 1 + 1e-9;
+    double bd = LAYER ? 1e6 : __builtin_huge_val();
+    int best = 0;
+    for (int c0 = 0; c0 < ng; c0 += VOR_B) {
+      double s[3] = {0.0, 0.0, 0.0}, near = 0.0;
+      bool keep = false;
+      if (c0 + tid < ng) {
+        for (int c = 0; c < 3; ++c) {
+          s[c] = xs[3 * (c0 + tid) + c];
+          const double m = fmax(0.0, fmax(lo[c] - s[c], s[c] - hi[c]));
+          near += m * m;
+        }
+        keep = !(near > far);
+      }
+      const unsigned long long bal = __ballot(keep);
+      if (lane == 0) sn[w] = __popcll(bal);
+      __syncthreads();  // (the last sites have been looked at)
+      int base = 0, m = 0;
+      for (int q = 0; q < VOR_B / 64; ++q) {
+        base += q < w ? sn[q] : 0;
+        m += sn[q];
+      }
+      if (keep) {
+        const int p = base + __popcll(bal & ((1ull << lane) - 1));
+        sx[p] = s[0];
+        sy[p] = s[1];
+        sz[p] = s[2];
+        si[p] = c0 + tid;
+      }
+      __syncthreads();
+      for (int q = 0; q < m; ++q) {
+        const double ax = x - sx[q], ay = y - sy[q], az = z - sz[q];
+        const double dd = ax * ax + ay * ay + az * az;
+        const bool lt = dd < bd;
+        bd = lt ? dd : bd;
+        best = lt ? si[q] : best;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-  }
-  if (!in) return;
-  const long long v = (long long)d.nxy * k + (long long)nx * j + i;
-  if (LAYER) {
-    label[v] = best;
-    used[best] = 1;
-  } else {
-    d.gid[v] = best + 1;
-    d.vs[v] = (v < (long long)d.nxy * (nz - 1)) ? 3 : 2;
-    d.cx[v] = x;
-    d.cy[v] = y;
-    d.cz[v] = z;
+    const long long v = (long long)d.nxy * k + (long long)nx * j + i;
+    if (in && LAYER) {
+      label[v] = best;
+      used[best] = 1;
+    } else if (in) {
+      d.gid[v] = best + 1;
+      d.vs[v] = (v < (long long)d.nxy * (nz - 1)) ? 3 : 2;
+      d.cx[v] = x;
+      d.cy[v] = y;
+      d.cz[v] = z;
+    }
   }
 }
 
@@ -4379,8 +4380,11 @@ int amcd_remap_grains(amcd_batch* b, int i, const int* remap, int ngrain) {
   return 0;
 }
 
-static unsigned voronoi_bricks(const Inst& d, int nz) {
-  return (unsigned)((d.p.nx + 7) / 8) * (unsigned)((d.p.ny + 7) / 8) * (unsigned)((nz + 3) / 4);
+// workgroups of k_voronoi: one to a brick, up to a number whose threads a launch can count (a domain one voxel
+// wide has as many bricks as an eighth or a quarter of its voxels)
+static unsigned voronoi_blocks(int nx, int ny, int nz) {
+  const long long bricks = (long long)((nx + 7) / 8) * ((ny + 7) / 8) * ((nz + 3) / 4);
+  return (unsigned)std::min<long long>(bricks, 1 << 20);
 }
 int amcd_init_plate(amcd_batch* b, int i, int nzh, const double* xs, int ng) {
   if (i < 0 || i >= b->n || ng <= 0 || nzh <= 0) return -1;
@@ -4389,7 +4393,7 @@ int amcd_init_plate(amcd_batch* b, int i, int nzh, const double* xs, int ng) {
   double* dx = nullptr;
   HIPT(hipMalloc(&dx, sizeof(double) * 3 * (size_t)ng));
   HIPT(hipMemcpyAsync(dx, xs, sizeof(double) * 3 * (size_t)ng, hipMemcpyHostToDevice, b->stream));
-  hipLaunchKernelGGL(k_voronoi<false>, dim3(voronoi_bricks(d, nzh)), dim3(VOR_B), 0, b->stream, b->d_inst, i, 0, nzh, dx,
+  hipLaunchKernelGGL(k_voronoi<false>, dim3(voronoi_blocks(d.p.nx, d.p.ny, nzh)), dim3(VOR_B), 0, b->stream, b->d_inst, i, 0, nzh, dx,
                      ng, nullptr, nullptr);
   HIPT(hipGetLastError());
   HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 8, b->stream));
@@ -4414,7 +4418,7 @@ int amcd_add_layer(amcd_batch* b, int i, int iz1, int ilaserLoc, int gbase, cons
   HIPT(hipMemcpyAsync(dx, xs, sizeof(double) * 3 * (size_t)ng, hipMemcpyHostToDevice, b->stream));
   HIPT(hipMemsetAsync(used, 0, sizeof(int) * (2 * (size_t)ng + 1), b->stream));
   if (cnt)
-    hipLaunchKernelGGL(k_voronoi<true>, dim3(voronoi_bricks(d, nl)), dim3(VOR_B), 0, b->stream, b->d_inst, i, iz1, nl, dx,
+    hipLaunchKernelGGL(k_voronoi<true>, dim3(voronoi_blocks(d.p.nx, d.p.ny, nl)), dim3(VOR_B), 0, b->stream, b->d_inst, i, iz1, nl, dx,
                        ng, lab, used);
   hipLaunchKernelGGL(k_site_rank, dim3(1), dim3(1024), 0, b->stream, used, ng, rank, tot);
   hipLaunchKernelGGL(k_write_layer, dim3((d.N + 255) / 256), dim3(256), 0, b->stream, b->d_inst, i, iz1, ilaserLoc,
