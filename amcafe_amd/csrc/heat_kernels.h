@@ -82,11 +82,12 @@ __device__ inline float indicator(float d, float ic) {
   return fmaf(fmaf(-x, y, 1.0f), y, y);
 }
 
-// Fixed-order block sum in FP64 (butterfly within each wave, then the waves in order).
+// Fixed-order block sum in FP64 (butterfly within each wave, then the waves in order; a wave is a row of
+// the block).
 __device__ inline double block_sum(double v, double* sh) {
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  if (threadIdx.x == 0) sh[threadIdx.y] = v;
   __syncthreads();
   double t = 0;
   for (int q = 0; q < HB / 64; ++q) t += sh[q];
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(HB, GRAD ? 3 : 4) void k_heat(Geo g, const Src* S, 
   __shared__ double sh[HB / 64];
   __shared__ int sodd;
   const Src s = S[blockIdx.z], tgt = Tg[blockIdx.z];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lane = threadIdx.x, w = threadIdx.y, tid = 64 * w + lane;
   const long long ncol = (long long)nsteps * g.nx;
   const int ntile = (int)((ncol + CT - 1) / CT);
   // Consecutive workgroups go to the chip's eight dies in turn, and the hot groups of a domain lie a
@@ -350,7 +351,7 @@ static __global__ __launch_bounds__(HB, 2) void k_heat64(Geo g, const Src* S, co
   __shared__ double sG[2][2][KP64 * CT64];
   __shared__ double nk[2][4][KP64];  // per set: vtau, 1/D1, 1/(4 alpha tau), amp
   __shared__ double sh[HB / 64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lane = threadIdx.x, w = threadIdx.y, tid = 64 * w + lane;
   const Src s[2] = {S[blockIdx.z], Tg[blockIdx.z]};
   const int nyz = g.ny * g.nz;
   const long long ncol = (long long)nsteps * g.nx;
@@ -519,14 +520,15 @@ static void launch_all(const amcafe_heat_desc* d, int nb, const Bufs<F>& B, int 
                        hipStream_t stream) {
   const Shape h = shape_of<F>(d, nsteps);
   const Geo g = geo(d);
-  const dim3 grid(h.groups, h.runs, nb);
+  // (64 threads along x: a launch counts its threads in 32 bits per dimension, and there may be 2^24 groups)
+  const dim3 grid(h.groups, h.runs, nb), block(64, HB / 64);
   for (long long m = 0; m == 0 || m < nsteps; m += h.seg) {
     const int c = (int)std::max(0ll, std::min<long long>(nsteps - m, h.seg)), ctiles = h.ctiles(c);
     if constexpr (sizeof(F) == 8)
-      hipLaunchKernelGGL(k_heat64, grid, dim3(HB), 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles, B.part,
+      hipLaunchKernelGGL(k_heat64, grid, block, 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles, B.part,
                          m == 0 ? 1 : 0);
     else
-      hipLaunchKernelGGL((k_heat<GRAD>), grid, dim3(HB), 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles,
+      hipLaunchKernelGGL((k_heat<GRAD>), grid, block, 0, stream, g, B.src, B.src + nb, (int)(step0 + m), c, ctiles,
                          h.patch, B.part, m == 0 ? 1 : 0, B.evals);
   }
   hipLaunchKernelGGL((k_heat_reduce<F>), dim3(nb), dim3(256), 0, stream, B.part, h.groups * h.runs, B.out);
