@@ -3718,8 +3718,10 @@ int amcd_upload(amcd_batch* b, int i, const int* gid, const int* vstate, const d
   if (vstate) {
     for (size_t v = 0; v < N; ++v) tmp[v] = (uint8_t)(vstate[v] & 3);
     HIPT(hipMemcpy(d.vs, tmp.data(), N, hipMemcpyHostToDevice));
-    HIPT(hipMemset(d.zliq, 0xff, (size_t)d.p.nz * 8));
-    HIPT(hipMemset(&d.ls->tvalid, 0, sizeof(int)));
+    // (on the batch's stream: a fill on the null stream need not be done when it returns, and the batch's
+    // stream does not wait for it)
+    HIPT(hipMemsetAsync(d.zliq, 0xff, (size_t)d.p.nz * 8, b->stream));
+    HIPT(hipMemsetAsync(&d.ls->tvalid, 0, sizeof(int), b->stream));
     hipLaunchKernelGGL(k_rehot, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, b->stream, d.vs, d.T, d.N, d.p.tL);
     HIPT(hipGetLastError());
     HIPT(hipStreamSynchronize(b->stream));
