@@ -188,8 +188,8 @@ int amcafe_sim_timings(amcafe_sim* s, double* ms, int n);
  *    the last t_hist seconds with the 25-point Gauss-Legendre rule of Utilities::Integral, and
  *    the loss sum over voxels and steps of (s(T) - s(T*))^2, s(T) = 1/(1+exp(-(T-tL)/width)),
  *    T* the field of the target parameters.  theta = {P [W], v [m/s], eta, sigma [m]}.
- *    Steps step0+1 .. step0+nsteps at t = n dt; each launch covers `checkpoint` steps (the field
- *    of a step is recomputed from theta and t, nothing is stored between steps).  *ms: device
+ *    Steps step0+1 .. step0+nsteps at t = n dt; each launch covers at most `checkpoint` steps
+ *    (the field of a step is recomputed from theta and t, nothing is stored between steps).  *ms: device
  *    time (may be NULL).
  * ------------------------------------------------------------------------- */
 typedef struct amcafe_heat_desc_s {
@@ -201,7 +201,8 @@ typedef struct amcafe_heat_desc_s {
   double k, alpha;                  /* conductivity [W/m/K], diffusivity [m^2/s] */
   int checkpoint;                   /* steps per launch (0: 100) */
 } amcafe_heat_desc;
-/* FP32 forward with FP32 accumulation */
+/* FP32 forward: rises as FP32 sums over the quadrature nodes, the loss summed in FP64 within a
+ * block and FP32 across segments */
 int amcafe_heat_loss_f32(const amcafe_heat_desc* d, const double* theta, const double* target, int step0,
                          int nsteps, double* loss, float* ms);
 /* FP32 loss and its gradient with respect to theta (hand-written adjoint) */
@@ -213,22 +214,25 @@ int amcafe_heat_loss_f64(const amcafe_heat_desc* d, const double* theta, const d
 /* n instances on the same grid and track in one launch per checkpoint segment (the calibration
  * form): theta, target and grad hold 4 values per instance, loss one (1 <= n <= 65535).  Each
  * instance's result is bit-identical to amcafe_heat_loss_grad_f32 on its own parameters.
- * All FP32 entry points sum in a fixed order (per thread over steps, per 256-voxel block in a
- * fixed tree, blocks across segments in launch order, block slots in a fixed tree), so a call
- * repeated with the same arguments returns the same bits.  They skip voxels whose temperature
- * bound stays below tL - 40 width at every step for both parameter sets (indicator below e^-40,
- * loss term below 2e-35); the FP64 forward evaluates every voxel. */
+ * All FP32 entry points sum in a fixed order (each lane over the 32 x 32 tiles of rows (y, z) and
+ * columns (x, t) that its wave evaluates, in tile order, and the block's lanes in a fixed tree, both
+ * in FP64; a block's sums across segments in launch order; the blocks' sums in a fixed tree), so a
+ * call repeated with the same arguments returns the same bits.  They skip the tiles in which every
+ * temperature stays below tL - 40 width for both parameter sets (indicator below e^-40, loss term
+ * below 2e-35); the FP64 forward evaluates every voxel at every step. */
 int amcafe_heat_loss_grad_batch_f32(const amcafe_heat_desc* d, int n, const double* theta, const double* target,
                                     int step0, int nsteps, double* loss, double* grad, float* ms);
-/* voxel-steps (per instance) the last heat call of this thread evaluated, after pruning */
+/* voxel-steps the last heat call of this thread evaluated, all instances together: the tiles that
+ * were not skipped (every voxel-step after amcafe_heat_loss_f64) */
 long long amcafe_heat_last_evaluations(void);
 /* amcafe_heat_loss_grad_batch_f32 without any device allocation, for callers that cannot
  * allocate: code under HIP graph capture, serving loops, harnesses that forbid hipMalloc.  No
  * counterpart in the reference.  Same kernels and the same bits as the batch entry point; no
- * timing.  Its device buffers (parameters, block sums) live in one static device array of
- * amcafe_heat_noalloc_max_bytes() (8 MiB) per GPU, held until the process ends: a call needing
- * more (amcafe_heat_noalloc_bytes: about 20 bytes per 256 voxels and instance, so 4.2 M voxels
- * for up to 25 instances) fails with AMCAFE_ERR_ARG before touching the device.  Every call on
+ * timing.  Its device buffers (parameters, block sums) live in one static device array of 16 MiB
+ * per GPU, held until the process ends.  A call is accounted amcafe_heat_noalloc_bytes (about 20
+ * bytes per 256 voxels and instance; domains one or two voxels long use up to twice that) and fails with
+ * AMCAFE_ERR_ARG before touching the device beyond amcafe_heat_noalloc_max_bytes() (8 MiB: 4.2 M
+ * voxels for up to 25 instances).  Every call on
  * a GPU shares that GPU's array: calls that overlap on one GPU (two host threads, or two
  * streams) race and return garbage. */
 int amcafe_heat_loss_grad_batch_f32_noalloc(const amcafe_heat_desc* d, int n, const double* theta,
