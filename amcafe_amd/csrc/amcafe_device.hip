@@ -21,8 +21,8 @@
 //   k_finish           active arrays back to the grid (S/VoxelsCA.C:633-643) and
 //                      ConvertSolid1(0) over the active cells (S/VoxelsCA.C:739-758)
 //   k_step_out         the output records to the pinned staging area
-// Per-voxel passes take runs of 16 voxels per thread (one 16-byte state load).  Layer
-// kernels: k_voronoi, k_site_rank, k_write_layer (base plate and powder layers,
+// Per-voxel passes take runs of 16 voxels per thread (one 16-byte state load; the temperature
+// four).  Layer kernels: k_voronoi, k_site_rank, k_write_layer (base plate and powder layers,
 // S/BasePlate.C, S/VoxelsCA.C AddLayer1/CleanLayer); k_grain_presence, k_remap (grain
 // renumbering).
 // Grid-wide kernels take a flattened block list over all instances, so a batch of
@@ -1380,10 +1380,11 @@ __device__ static inline void recentre(DI& d, int vcap, int vnew, const double* 
 // half wave each), with the re-centring of its own entries and a single-precision bound on the time
 // to the captures after them.  Only for the captures that the step has time for: a cell grows half a
 // voxel a step, which leaves about a third of the entries.  Bound by the latency of a wave's own
-// chain, not by the chip (a few thousand waves): 33 us for 3.3 thousand growing cells, 44 us for 15
-// thousand and 22 us for 300 (64, 109 and 38 us with lists ahead for every entry, 18 and 15 us in the
-// first and last without any); with the lists ahead the loop's windows end later: 3291 -> 2863
-// cycles per event in the first deck.
+// chain, not by the chip (a few thousand waves): averaged over a run's steps 36 us for the 512x512x128
+// raster (49 us at its 3.2 thousand growing cells), 38 us for 256x192x64 (106 us at 6 thousand) and 21 us
+// for 40x24x20 (33 us at 200).  With lists ahead for every entry the runs' averages were 64, 109 and
+// 38 us, in the first and last without any 18 and 15 us; with the lists ahead the loop's windows end
+// later: 3291 -> 2863 cycles per event in the first deck.
 __device__ static inline int list_rank(double D, double r, bool on, int half) {
   // position in (D, ruqs, neighbour) order among the entries of this lane's half wave (all of it
   // for half < 0), NaN distances last
@@ -1628,18 +1629,18 @@ __global__ void k_clear_npre(Inst* I) {
 //
 // What bounds it: a chain of dependent instructions.  An event is about 100 instructions of one
 // wave (11 to 13 cycles each), and every window pays five barriers and two rounds of list reads;
-// hence as many events per window as its 64 entries give (31 where the interface is wide, 8 where
-// there are few cells), records that are one cache line, and lists and capture constants made by the
+// hence as many events per window as its 64 entries give (31 where the interface is wide, 18 in the
+// memory tier, 8 where there are few cells), records that are one cache line, and lists and capture constants made by the
 // set-up's parallel pass.  One decision per barrier with the lists built around each event took
 // 6.9K cycles an event in these decks and 13.7K with the state in memory; now (cycles per event, 2.4
 // GHz): 5.3K with few growing cells (at most 300), 2.7K with 3 thousand of a single track or of a
-// raster over a wide plate, 6.5K with 15 thousand (state in memory; 10.1K while a cell without a
-// bound from the set-up, or any step back, ended the window).
+// raster over a wide plate, 6.0K with 15 thousand (state in memory; 10.1K while a cell without a
+// bound from the set-up, or any step back, ended the window, 6.5K while ties shrank the span).
 typedef const __attribute__((address_space(4))) Inst CInst;
 struct Best {
   double t, r;
   int key;   // scan position * 32 + neighbour rank: the reference's scan order
-  int cand;  // candidate entry (slot * AMCD_NB + position), or the lane that holds it
+  int cand;  // candidate entry, or the lane that holds it
   int tgt;   // active index of the captured voxel
 };
 __device__ static inline Best best_none() {
@@ -2433,7 +2434,7 @@ __device__ static inline Refreshed refresh_cell(CInst& d, const Liveness<GD>& li
       const double g = o.grown + v * lane_f64(dtl, j);
       o.grown = (j > k0) & (j <= last) ? g : o.grown;
     }
-    if (o.grown < 0.0) o.grown = 0.0;  // (only a window's last event can step back)
+    if (o.grown < 0.0) o.grown = 0.0;  // (only a window's last event can take it below zero)
   }
   // tau is the same before and after the growth; a new cell's is taken after it
   if (o.tgt >= 0) tau_bounds(D1, k0 >= 0 ? o.grown : e, v, k0 >= 0 ? T : T0, o.lo, o.hi);
@@ -2759,7 +2760,8 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
         // window needed that, the next ones hold the same ties (a flat front's cells reach their
         // neighbours at one time), so in the memory tier, where each way costs a pass over every cell's
         // state, they begin there while more than a window's are left (118x93x74, 12 thousand growing
-        // cells: 10.9K -> 10.3K cycles per event; in the register tiers the first ways cost little).
+        // cells: 10.9K -> 10.3K cycles per event, 9.1K since ties leave the span alone; in the register
+        // tiers the first ways cost little).
         int mode = start;
         for (;; ++mode) {
           if (mode > 0) W = mode == 1 ? fmaxf(Tf + 0.4f * (W - Tf), u) : u;
@@ -3048,7 +3050,7 @@ __global__ __launch_bounds__(NT) void k_event_loop(Inst* I, const amcd_step* S, 
       }
       if (sh.neg) {
         // the reference's clamp at zero, which moves the cell's capture times: only a window's
-        // last event can step back in time (or grow by a negative velocity) and so need it
+        // last event can take a half-diagonal there and so need it
         if constexpr (MEM) __syncthreads();
         for (int s0 = tid; s0 < ns; s0 += KR * NT) {
 #pragma unroll
@@ -3205,8 +3207,6 @@ __global__ __launch_bounds__(GB) void k_finish(Inst* I, const int* astart, int n
 }
 
 // ---- per-layer helpers ---------------------------------------------------------------
-// After a host upload of vState: the "T >= tL" flag (bit 7) follows the device's current
-// temperature field, so SetLiquid3 still sees the caller's melt pool.
 // A step's records: in from the pinned staging area with fresh output records (`clear` words) and the
 // instances' nucleation pools (a workgroup each, after the first `nrec`), and the outputs back.  As
 // kernels in the step's graph they cost 3.5 us each; as stream copies beside it, 10.
@@ -3228,6 +3228,8 @@ __global__ void k_step_out(unsigned* staged, const unsigned* outs, int nwords) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q < nwords) staged[q] = outs[q];
 }
+// After a host upload of vState: the "T >= tL" flag (bit 7) follows the device's current
+// temperature field, so SetLiquid3 still sees the caller's melt pool.
 __global__ void k_rehot(uint8_t* vs, const double* T, int N, double tL) {
   size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= (size_t)N) return;

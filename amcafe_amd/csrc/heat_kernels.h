@@ -37,7 +37,7 @@ struct Geo {
 // 256x256x64 voxels and 2000 steps are not), so a block first bounds its tiles, one per lane, and
 // goes through those that can count; the rows of a wave are a compact patch of 8 x 4 (y, z), which
 // leaves fewer of them than 32 in a line.  Evaluating the nodes' exponentials for every voxel-step
-// took 50 exponentials each: that domain's loss 45.0 -> 2.9 ms, loss and gradient 60.0 -> 4.0 ms.  The
+// took 50 exponentials each: that domain's loss 45.0 -> 2.7 ms, loss and gradient 60.0 -> 4.1 ms.  The
 // matrix products (26 of 64 cycles per 1024 results) and the indicators (about as much) bound it.
 constexpr int NQ = AMC_GL25_N, KP = 26;  // nodes, padded to pairs (the padding's A is 0)
 constexpr int RT = 32, CT = 32;          // rows and columns of a wave's tile
